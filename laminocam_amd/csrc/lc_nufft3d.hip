@@ -14,7 +14,7 @@
 // shift; the (-1)^m phase and 1/psi_hat sit in per-axis correction factors.
 //   type 1: deterministic sorted-bin spreading -> fine grid, then one pruned
 //           FFT pass per axis (x, y, z), deconvolution in each pass;
-//   type 2: the reverse passes, then 8x8x8 interpolation per point.
+//   type 2: the reverse passes, then 8x8x8 interpolation of the sorted points.
 // Detector transforms are line FFTs along x then y with the reference's shift
 // index maps; widths that are not 2^p 3^q use Bluestein's algorithm with an
 // FP64-built chirp and chirp spectrum.
@@ -48,17 +48,6 @@ __device__ __forceinline__ float es3(float z, float beta) {
     return s > 0.0f ? __expf(beta * (__builtin_amdgcn_sqrtf(s) - 1.0f)) : 0.0f;
 }
 
-// value of v in lane `lane` (the same for every lane: a scalar broadcast, no LDS)
-__device__ __forceinline__ float rl_f32(float v, int lane) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-__device__ __forceinline__ double rl_f64(double v, int lane) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), lane);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
 __device__ __forceinline__ int wrapi(int a, int n) {
     a %= n;
     return a < 0 ? a + n : a;
@@ -87,74 +76,134 @@ __device__ __forceinline__ bool inside_pi(double x, double y, double z) {
 }
 
 // ---------------------------------------------------------------------------
-// type-2 interpolation: a wave per point.  Each lane first finds the footprint
-// of one of the wave's 64 consecutive points; the wave then takes the points
-// in turn with its lanes over the 8 x 8 (y, x) footprint, walking the 8 z
-// planes (each step reads 8 rows of 8 contiguous fine-grid values), and sums
-// the 64 lanes in a fixed order.  Lane i writes point i, so the stores are
-// contiguous.
+// Points by bins of footprint corners.  A point's corner is its first
+// footprint cell, ceil(g - W3/2) per axis, taken modulo nf.  Every axis is cut
+// into nb bins of corners, bin i starting at floor(i nf / nb): an even number
+// of bins of 7 to BE cells (three bins where no even number gives such widths:
+// nf = 24 and 27), so that the footprints of one bin lie in a region of 16
+// cells along z and x (ROWS along y), and the regions of two bins an even
+// distance apart are disjoint, around the periodic wrap too.  k_bin_keys
+// gives every point its bin and, below it, its corner's row in the bin; a
+// stable radix sort (rocPRIM) orders the points, keeping point order where
+// the keys agree; k_bin_ranges marks each bin's run.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256)
-k_interp3d(const float2 *__restrict__ F, float2 *__restrict__ C, const double *__restrict__ rot,
-           Grid3 g) {
-    static_assert(W3 == 8, "the lane layout assumes a footprint of 8 per axis");
-    const int64_t npts = (int64_t)g.nproj * g.nrows * g.ncols;
-    const int lane = threadIdx.x & 63;
-    const int64_t base = ((int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 64;
-    if (base >= npts) return;   // whole wave
-    const int64_t q = base + lane;
+constexpr int RGN = 16;                     // region cells along z and x: the edge of an MFMA tile
+constexpr int BE = RGN - W3 + 1;            // most corner cells of a bin along z and x
+
+// A compiled region shape: ROWS region rows along y (bins of ROWS - W3 + 1
+// corner rows).  More rows mean fewer bins, whose regions overlap less.
+template <int ROWS_> struct Shape3 {
+    static constexpr int ROWS = ROWS_;
+    static constexpr int EY = ROWS - W3 + 1;
+    static constexpr int YB = EY <= 16 ? 4 : EY <= 32 ? 5 : 6;   // key bits of the corner row
+    static constexpr int TEAMS = ROWS <= 16 ? 4 : 3;             // teams of a heavy bin (their tables fill the LDS)
+    static_assert(ROWS % 8 == 0 && EY <= 64, "rows go to four waves in turn; a row index has six bits");
+};
+// the shapes the autotuner (nufft3d_autotune) chooses from for the spread, per
+// fine-grid shape; shape 0 is the default.  Interpolation uses shape 0.
+constexpr int N_SHAPES3 = 3;
+template <typename F> void with_shape3(int i, F &&f) {
+    switch (i) {
+    case 1: f(Shape3<32>{}); break;
+    case 2: f(Shape3<48>{}); break;
+    default: f(Shape3<16>{}); break;
+    }
+}
+
+// bins along an axis of nf >= 16 cells, for bins of at most `edge` corners
+__host__ __device__ constexpr int bins_along(int nf, int edge) {
+    int nb = 2 * ((nf + 2 * edge - 1) / (2 * edge));
+    return nf / nb >= W3 - 1 ? nb : 3;
+}
+
+struct Bins3 {
+    int nb[3];          // bins per axis
+};
+__device__ __forceinline__ int bin_first(int i, int nf, int nb) { return (int)((int64_t)i * nf / nb); }
+// the bin of corner l: the largest i with bin_first(i) <= l
+__device__ __forceinline__ int bin_of(int l, int nf, int nb) { return (int)(((int64_t)(l + 1) * nb - 1) / nf); }
+
+// fine-grid position g, footprint corner l (unwrapped) of point (p, j, k)
+struct Corner3 {
+    double gz, gy, gx;
+    int lz, ly, lx;
+    bool ok;    // false: dropped by the mask
+};
+__device__ __forceinline__ Corner3 corner3(const double *rot, int p, int j, int k, const Grid3 &g) {
+    Corner3 c;
+    double x, y, z;
+    point3(rot, p, j, k, g, x, y, z);
+    c.ok = !g.mask || inside_pi(x, y, z);
     const double hw = 0.5 * W3;
-    const float ihw = 1.0f / (float)hw;
-    double gz = 0.0, gy = 0.0, gx = 0.0;
-    int z0 = 0, y0 = 0, x0 = 0, ok = 0;
-    if (q < npts) {
-        const int k = (int)(q % g.ncols);
-        const int64_t t = q / g.ncols;
-        const int j = (int)(t % g.nrows), p = (int)(t / g.nrows);
-        double x, y, z;
-        point3(rot, p, j, k, g, x, y, z);
-        ok = (!g.mask || inside_pi(x, y, z)) ? 1 : 0;
-        gz = 0.5 * g.nf[0] + z * (g.nf[0] / (2.0 * M_PI));
-        gy = 0.5 * g.nf[1] + y * (g.nf[1] / (2.0 * M_PI));
-        gx = 0.5 * g.nf[2] + x * (g.nf[2] / (2.0 * M_PI));
-        z0 = (int)ceil(gz - hw);
-        y0 = (int)ceil(gy - hw);
-        x0 = (int)ceil(gx - hw);
+    c.gz = 0.5 * g.nf[0] + z * (g.nf[0] / (2.0 * M_PI));
+    c.gy = 0.5 * g.nf[1] + y * (g.nf[1] / (2.0 * M_PI));
+    c.gx = 0.5 * g.nf[2] + x * (g.nf[2] / (2.0 * M_PI));
+    c.lz = (int)ceil(c.gz - hw);
+    c.ly = (int)ceil(c.gy - hw);
+    c.lx = (int)ceil(c.gx - hw);
+    return c;
+}
+__device__ __forceinline__ Corner3 corner3(const double *rot, unsigned pt, const Grid3 &g) {
+    const unsigned pj = pt / (unsigned)g.ncols;
+    const int k = (int)(pt - pj * (unsigned)g.ncols);
+    const int p = (int)(pj / (unsigned)g.nrows), j = (int)(pj - (unsigned)p * (unsigned)g.nrows);
+    return corner3(rot, p, j, k, g);
+}
+
+// key[i]: bin << YB | corner row in the bin of point i, or nbins << YB (sorted
+// last) for a point the mask drops, whose value in `drop` (if given) becomes
+// 0; val[i] = i
+template <typename S>
+__global__ void k_bin_keys(const double *__restrict__ rot, Grid3 g, Bins3 bn, unsigned *__restrict__ key,
+                           unsigned *__restrict__ val, int64_t npts, unsigned nbins, float2 *__restrict__ drop) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= npts) return;
+    const Corner3 c = corner3(rot, (unsigned)i, g);
+    unsigned b = nbins << S::YB;
+    if (c.ok) {
+        const int lz = wrapi(c.lz, g.nf[0]), ly = wrapi(c.ly, g.nf[1]), lx = wrapi(c.lx, g.nf[2]);
+        const int bz = bin_of(lz, g.nf[0], bn.nb[0]), by = bin_of(ly, g.nf[1], bn.nb[1]),
+                  bx = bin_of(lx, g.nf[2], bn.nb[2]);
+        b = (unsigned)(((int64_t)bz * bn.nb[1] + by) * bn.nb[2] + bx) << S::YB |
+            (unsigned)(ly - bin_first(by, g.nf[1], bn.nb[1]));
+    } else if (drop) {
+        drop[i] = make_float2(0.f, 0.f);
     }
-    const int iy = lane >> 3, ix = lane & 7;
-    const int nlast = (int)(npts - 1 - base < 63 ? npts - 1 - base : 63);
-    float2 res = make_float2(0.f, 0.f);
-    for (int j = 0; j <= nlast; ++j) {
-        if (!__builtin_amdgcn_readlane(ok, j)) continue;   // masked point: 0
-        const double gzj = rl_f64(gz, j), gyj = rl_f64(gy, j), gxj = rl_f64(gx, j);
-        const int z0j = __builtin_amdgcn_readlane(z0, j);
-        const int y0j = __builtin_amdgcn_readlane(y0, j);
-        const int x0j = __builtin_amdgcn_readlane(x0, j);
-        // lane (iy, ix) holds the y weight of row iy, the x weight of column
-        // ix, and the z weight of plane ix (read by every lane in the z walk)
-        const float wzl = es3((float)((double)(z0j + ix) - gzj) * ihw, g.beta);
-        const float wyl = es3((float)((double)(y0j + iy) - gyj) * ihw, g.beta);
-        const float wxl = es3((float)((double)(x0j + ix) - gxj) * ihw, g.beta);
-        const int yy = wrapi(y0j + iy, g.nf[1]), xx = wrapi(x0j + ix, g.nf[2]);
-        float rr = 0.f, ri = 0.f;
-#pragma unroll
-        for (int a = 0; a < W3; ++a) {
-            const float wza = rl_f32(wzl, a);
-            const int zz = wrapi(z0j + a, g.nf[0]);
-            const float2 v = F[((int64_t)zz * g.nf[1] + yy) * g.nf[2] + xx];
-            rr += wza * v.x;
-            ri += wza * v.y;
-        }
-        const float w = wyl * wxl;
-        float sr = w * rr, si = w * ri;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            sr += __shfl_xor(sr, off, 64);
-            si += __shfl_xor(si, off, 64);
-        }
-        if (lane == j) res = make_float2(sr, si);
-    }
-    if (q < npts) C[q] = res;
+    key[i] = b;
+    val[i] = (unsigned)i;
+}
+
+// [start[b], end[b]) is bin b's run in the sorted keys (start = end = 0 when
+// empty: both arrays cleared first)
+__global__ void k_bin_ranges(const unsigned *__restrict__ skey, int64_t n, unsigned *__restrict__ start,
+                             unsigned *__restrict__ end, unsigned nbins, int yb) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const unsigned b = skey[i] >> yb;
+    if (b >= nbins) return;
+    if (i == 0 || (skey[i - 1] >> yb) != b) start[b] = (unsigned)i;
+    if (i == n - 1 || (skey[i + 1] >> yb) != b) end[b] = (unsigned)(i + 1);
+}
+
+// launch phases along an axis: two (even and odd bins), or one per bin of three
+__host__ __device__ constexpr int phases_along(int nb) { return nb == 3 ? 3 : 2; }
+
+// the bins in launch order: grouped by phase (bins that may add to the grid
+// side by side), fullest first inside a phase, so a phase's long-running
+// dense bins start first and its tail is short.  key = phase << 26 |
+// (2^26 - 1 - count), val = bin
+constexpr int ORDER_BITS = 31;
+__global__ void k_bin_order_keys(const unsigned *__restrict__ bstart, const unsigned *__restrict__ bend,
+                                 Bins3 bn, unsigned *__restrict__ key, unsigned *__restrict__ val,
+                                 unsigned nbins) {
+    const unsigned b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= nbins) return;
+    const unsigned bx = b % bn.nb[2], by = (b / bn.nb[2]) % bn.nb[1], bz = b / (bn.nb[2] * bn.nb[1]);
+    const unsigned py = phases_along(bn.nb[1]), px = phases_along(bn.nb[2]);
+    const unsigned ph = ((bz % phases_along(bn.nb[0])) * py + by % py) * px + bx % px;
+    const unsigned cnt = min(bend[b] - bstart[b], (1u << 26) - 1);
+    key[b] = (ph << 26) | ((1u << 26) - 1 - cnt);
+    val[b] = b;
 }
 
 // include/fft.h:53-74 (phase_shift2d): detector spectrum C[p][j][k] *=
@@ -177,254 +226,364 @@ __global__ void k_phase_shift3d(float2 *__restrict__ C, const double *__restrict
 }
 
 // ---------------------------------------------------------------------------
-// type-1 spreading by footprint-corner bins.  The fine grid is cut into
-// BZ x BY x BX bins of footprint corners (a point's corner is its first
-// footprint cell, ceil(g - W3/2) per axis, taken modulo nf).  k_bin_keys
-// gives every point its bin; a stable radix sort (rocPRIM) orders the points
-// by bin, keeping point order inside a bin; k_bin_ranges marks each bin's
-// run.  A wave then owns one bin (a bin of more than B3_HEAVY points gets
-// NW3_HEAVY waves, each taking a consecutive part of the bin's points): it
-// takes the points in order and spreads each one's whole 8 x 8 x 8 footprint
-// (lanes over 8 x 8 in x, y; 8 steps in z) into the wave's private LDS copy
-// of the bin's padded region (bin + W3 - 1 cells per axis: 11 x 11 x
-// 15 cells, 15.5 KiB, so a CU holds ten bins).  Every point is spread once,
-// with all 64 lanes inside its footprint, and no point is tested against a
-// bin it does not belong to.  The copies are summed in a fixed order and
-// added into Fp, the fine grid extended by W3 - 1 cells per axis (not
-// periodic).  Bins P apart along an axis have disjoint padded regions when
-// P b >= b + W3 - 1 (P = 3 for b = 4, 2 for b = 8), so the bins run in
-// PZ PY PX = 18 phases (the bin's index modulo P along each axis), each adding
-// without conflicts, fullest bins first; k_fold3d then wraps the overhang
-// back onto the periodic grid.  Every sum runs in a fixed order: the result
-// is deterministic.  On the 32 x 511^2 back-projection from 720 x 128 x 511
-// points the spread takes about 14 ms (8^3 bins in 8 phases: 16 ms), against
-// 53 ms for a tile-gather spread that searched every tile's candidate points.
+// Both directions run on the matrix cores.  With wz, wy, wx a point's 8 weights
+// per axis, placed at its corner in 16 (ROWS) slots that are zero elsewhere,
+//   spread:  R[z][y][x]  = sum_p (wz_p[z] wy_p[y]) (c_p wx_p[x])   K = points
+//   interp:  G[p][x]     = sum_{y,z} (wz_p[z] wy_p[y]) F[z][y][x]  K = (z, y)
+//            c_p         = sum_x wx_p[x] G[p][x]
+// so each region row y is one 16 x 16 FP32 MFMA tile (v_mfma_f32_16x16x4_f32:
+// lane l holds A[l & 15][l >> 4], B[l >> 4][l & 15] and, in register q,
+// D[4 (l >> 4) + q][l & 15]), once for the real and once for the imaginary
+// part.  A block's four waves take the rows y = w, w + 4, ...; the points of a
+// bin come in corner-row order, so a group of consecutive points touches 8 or
+// 9 rows, and a wave skips the others.  A group's other weights are zeros:
+// half the products along z and along x are wasted, which the matrix rate
+// (twice the vector FMA rate, with no LDS access per cell) more than pays for.
+// Weights are computed once per point into LDS tables of BATCH points.
+// Measured: interpolating 23.1 M points (360 x 89 x 721 on 29 x 721^2) takes
+// 3.9 ms against 22.0 ms with a wave per point reading its 512 cells through
+// L1; spreading 47 M points (720 x 128 x 511 on 32 x 511^2) 7.5 ms against 13.5
+// ms with a wave per bin adding each point's cells to an LDS copy of a 4 x 4 x
+// 8 bin's region, and 2.9 M points (8 x 256^2) 1.28 against 2.61 ms.
 // ---------------------------------------------------------------------------
-constexpr int PXS = 16;                     // padded row stride (cells)
-// bins P apart along an axis have disjoint padded regions when P b >= b + W3 - 1
-constexpr int phase_period(int b) { return (b + W3 - 1 + b - 1) / b; }
+using f32x4 = __attribute__((ext_vector_type(4))) float;
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+constexpr int BATCH = 128;                  // points per table; two threads fill a point's slots
 
-// A bin shape (edges in corner cells along z, y, x) the spread is compiled
-// for: its padded region, phase periods and launch phases.  Region cell
-// (z, y, x) -> LDS index with x XOR-ed with 8 on every other row pair, so the
-// 8 rows x 8 columns of one z step fall on distinct bank pairs.
-template <int BZ_, int BY_, int BX_> struct Shape3 {
-    static constexpr int BZ = BZ_, BY = BY_, BX = BX_;
-    static constexpr int RZ = BZ + W3 - 1, RY = BY + W3 - 1, RX = BX + W3 - 1;
-    static constexpr int PZ = phase_period(BZ), PY = phase_period(BY), PX = phase_period(BX);
-    static constexpr int NPH = PZ * PY * PX;   // launch phases
-    // bits of the launch-order key: the phase above a 26-bit descending count
-    static constexpr int ORDER_BITS = 26 + (NPH > 16 ? 5 : NPH > 8 ? 4 : NPH > 4 ? 3 : NPH > 2 ? 2 : 1);
-    static constexpr int PC = RZ * RY * PXS;    // cells of one region copy
-    // waves of a heavy bin: as many region copies as fit 64 KiB
-    static constexpr int NWH = 65536 / (8 * PC) < 1 ? 1 : 65536 / (8 * PC);
-    static_assert(RX <= PXS, "a region row must fit the padded row stride");
-    static_assert(ORDER_BITS <= 32, "launch-order key too wide");
-    __device__ __forceinline__ static int tidx(int z, int y, int x) {
-        return (z * RY + y) * PXS + (x ^ (((y >> 1) & 1) << 3));
-    }
+// footprint corner of a point relative to its bin, and the offset of its first
+// cell from the point (the weights' argument), per axis
+struct Foot {
+    int t[3];
+    float f[3];
 };
-// The shapes the autotuner (spread3d_autotune) chooses from, per fine-grid
-// shape; shape 0 is the default.  On the 32 x 511^2 back-projection
-// (720 x 128 x 511 points) the whole call measured 30.9 ms with 4 x 4 x 8
-// bins, 31.2 with 8 x 4 x 4, 31.8 with 4 x 4 x 4, 32.8 with 2 x 4 x 8 and 33.0
-// with 8 x 8 x 8.
-constexpr int N_SHAPES3 = 3;
-template <typename F> void with_shape3(int i, F &&f) {
-    switch (i) {
-    case 1: f(Shape3<8, 4, 4>{}); break;
-    case 2: f(Shape3<8, 8, 8>{}); break;
-    default: f(Shape3<4, 4, 8>{}); break;
-    }
-}
-constexpr int MAX_ORDER_BITS = 31;
-
-struct Bins3 {
-    int nb[3];          // bins per axis, ceil(nf / bin edge)
-    int pf[3];          // padded grid dims nf + W3 - 1
-};
-
-// fine-grid position g, footprint corner l (unwrapped) of point (p, j, k)
-struct Corner3 {
-    double gz, gy, gx;
-    int lz, ly, lx;
-    bool ok;    // false: dropped by the mask
-};
-__device__ __forceinline__ Corner3 corner3(const double *rot, int p, int j, int k, const Grid3 &g) {
-    Corner3 c;
-    double x, y, z;
-    point3(rot, p, j, k, g, x, y, z);
-    c.ok = !g.mask || inside_pi(x, y, z);
-    const double hw = 0.5 * W3;
-    c.gz = 0.5 * g.nf[0] + z * (g.nf[0] / (2.0 * M_PI));
-    c.gy = 0.5 * g.nf[1] + y * (g.nf[1] / (2.0 * M_PI));
-    c.gx = 0.5 * g.nf[2] + x * (g.nf[2] / (2.0 * M_PI));
-    c.lz = (int)ceil(c.gz - hw);
-    c.ly = (int)ceil(c.gy - hw);
-    c.lx = (int)ceil(c.gx - hw);
-    return c;
+__device__ __forceinline__ Foot foot3(const double *rot, unsigned pt, const Grid3 &g, const int s[3]) {
+    const Corner3 c = corner3(rot, pt, g);
+    Foot q;
+    q.t[0] = wrapi(c.lz, g.nf[0]) - s[0];
+    q.t[1] = wrapi(c.ly, g.nf[1]) - s[1];
+    q.t[2] = wrapi(c.lx, g.nf[2]) - s[2];
+    q.f[0] = (float)((double)c.lz - c.gz);
+    q.f[1] = (float)((double)c.ly - c.gy);
+    q.f[2] = (float)((double)c.lx - c.gx);
+    return q;
 }
 
-// key[i]: the bin of point i's wrapped corner, or nbins (sorted last) for a
-// point the mask drops; val[i] = i
-template <typename S>
-__global__ void k_bin_keys(const double *__restrict__ rot, Grid3 g, Bins3 bn, unsigned *__restrict__ key,
-                           unsigned *__restrict__ val, int64_t npts, unsigned nbins) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= npts) return;
-    const int64_t pj = i / g.ncols;
-    const int k = (int)(i - pj * g.ncols);
-    const int p = (int)(pj / g.nrows), j = (int)(pj - (int64_t)p * g.nrows);
-    const Corner3 c = corner3(rot, p, j, k, g);
-    unsigned b = nbins;
-    if (c.ok) {
-        const int bz = wrapi(c.lz, g.nf[0]) / S::BZ, by = wrapi(c.ly, g.nf[1]) / S::BY,
-                  bx = wrapi(c.lx, g.nf[2]) / S::BX;
-        b = (unsigned)(((int64_t)bz * bn.nb[1] + by) * bn.nb[2] + bx);
-    }
-    key[i] = b;
-    val[i] = (unsigned)i;
-}
-
-// [start[b], end[b]) is bin b's run in the sorted keys (start = end = 0 when
-// empty: both arrays cleared first)
-__global__ void k_bin_ranges(const unsigned *__restrict__ skey, int64_t n, unsigned *__restrict__ start,
-                             unsigned *__restrict__ end, unsigned nbins) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const unsigned b = skey[i];
-    if (b >= nbins) return;
-    if (i == 0 || skey[i - 1] != b) start[b] = (unsigned)i;
-    if (i == n - 1 || skey[i + 1] != b) end[b] = (unsigned)(i + 1);
-}
-
-// the bins in launch order: grouped by phase (the bin's indices modulo the
-// phase periods), fullest first inside a phase, so a phase's long-running
-// dense bins start first and its tail is short.  key = phase << 26 |
-// (2^26 - 1 - count), val = bin
-template <typename S>
-__global__ void k_bin_order_keys(const unsigned *__restrict__ bstart, const unsigned *__restrict__ bend,
-                                 Bins3 bn, unsigned *__restrict__ key, unsigned *__restrict__ val,
-                                 unsigned nbins) {
-    const unsigned b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nbins) return;
-    const unsigned bx = b % bn.nb[2], by = (b / bn.nb[2]) % bn.nb[1], bz = b / (bn.nb[2] * bn.nb[1]);
-    const unsigned ph = ((bz % S::PZ) * S::PY + by % S::PY) * S::PX + bx % S::PX;
-    const unsigned cnt = min(bend[b] - bstart[b], (1u << 26) - 1);
-    key[b] = (ph << 26) | ((1u << 26) - 1 - cnt);
-    val[b] = b;
-}
-
-// Bins of more than B3_HEAVY points are spread by S::NWH waves, each taking a
-// consecutive part of the bin's points into its own copy of the region; the
-// copies are summed in wave order.  Whether a bin is heavy depends only on
-// its own count.
-constexpr unsigned B3_HEAVY = 2048;
-
-// spread bin bid's points with the block's NW waves into their region copies
-// (reg: NW x RZ x RY x PXS) and add the copies' fixed-order sum into Fp
-template <typename S, int NW>
-__device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2 *__restrict__ Fp,
-                                            const double *__restrict__ rot, const unsigned *__restrict__ sval,
-                                            int bid, unsigned s0, unsigned s1, const Grid3 &g, const Bins3 &bn,
-                                            float2 *acc) {
-    constexpr int PC = S::PC, RY = S::RY, RZ = S::RZ, RX = S::RX;
-    const int b[3] = {bid / (bn.nb[1] * bn.nb[2]), (bid / bn.nb[2]) % bn.nb[1], bid % bn.nb[2]};
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    float2 *my = acc + wave * PC;
-    for (int i = lane; i < PC; i += 64) my[i] = make_float2(0.f, 0.f);
-    const int c0[3] = {S::BZ * b[0], S::BY * b[1], S::BX * b[2]};
+// the slots congruent to 4 h .. 4 h + 3 modulo 8 of one axis's `slots` slots:
+// put(slot, weight), where one slot of each residue lies in the footprint
+template <int SLOTS, typename F>
+__device__ __forceinline__ void axis_weights(int t, float f, int h, float beta, F &&put) {
     const float ihw = 1.0f / (0.5f * W3);
-    const int dxl = lane & 7, dyl = lane >> 3;
-    // wave w takes the w-th part of the bin's points, in order
-    const unsigned per = (s1 - s0 + NW - 1) / NW;
-    const unsigned ws = s0 + wave * per, we = min(s1, ws + per);
-    for (unsigned base = ws; base < we; base += 64) {
-        const unsigned i = base + lane;
-        const bool ok = i < we;
-        float2 cv = make_float2(0.f, 0.f);
-        int tz = 0, ty = 0, tx = 0;
-        float fz = 0.f, fy = 0.f, fx = 0.f;
-        if (ok) {
-            const unsigned pt = sval[i];
-            const unsigned pj = pt / (unsigned)g.ncols;
-            const int k = (int)(pt - pj * (unsigned)g.ncols);
-            const int p = (int)(pj / (unsigned)g.nrows), j = (int)(pj - (unsigned)p * (unsigned)g.nrows);
-            const Corner3 c = corner3(rot, p, j, k, g);
-            // the corner taken modulo nf, relative to the bin: in [0, bin edge)
-            tz = wrapi(c.lz, g.nf[0]) - c0[0];
-            ty = wrapi(c.ly, g.nf[1]) - c0[1];
-            tx = wrapi(c.lx, g.nf[2]) - c0[2];
-            fz = (float)((double)c.lz - c.gz);
-            fy = (float)((double)c.ly - c.gy);
-            fx = (float)((double)c.lx - c.gx);
-            cv = C[pt];
-        }
-        unsigned long long pts = __ballot(ok);
-        while (pts) {
-            const int s2 = __ffsll((long long)pts) - 1;
-            pts &= pts - 1;
-            const int pz0 = __builtin_amdgcn_readlane(tz, s2);
-            const int py0 = __builtin_amdgcn_readlane(ty, s2);
-            const int px0 = __builtin_amdgcn_readlane(tx, s2);
-            const float vr = rl_f32(cv.x, s2), vi = rl_f32(cv.y, s2);
-            const float wxy = es3(((float)dxl + rl_f32(fx, s2)) * ihw, g.beta) *
-                              es3(((float)dyl + rl_f32(fy, s2)) * ihw, g.beta);
-            // lane dz holds wz[dz]
-            const float wzl = es3(((float)dxl + rl_f32(fz, s2)) * ihw, g.beta);
-            const int base_idx = S::tidx(pz0, py0 + dyl, px0 + dxl);
 #pragma unroll
-            for (int dz = 0; dz < W3; ++dz) {
-                const float wgt = wxy * rl_f32(wzl, dz);
-                float2 &a = my[base_idx + dz * RY * PXS];
-                a.x += wgt * vr;
-                a.y += wgt * vi;
+    for (int i = 0; i < 4; ++i) {
+        const int r = 4 * h + i, d = (r - t) & (W3 - 1), slot = t + d;
+        const float w = es3(((float)d + f) * ihw, beta);
+#pragma unroll
+        for (int s = 0; s < SLOTS; s += W3) put(r + s, r + s == slot ? w : 0.f);
+    }
+}
+// smallest and largest corner row of the groups of G consecutive lanes
+template <int G> __device__ __forceinline__ void group_rows(int ty, bool ok, int &lo, int &hi) {
+    // (a corner on a bin's edge may round to the bin beside it: its weights are
+    // then dropped where they are smallest, and the rows stay in range)
+    ty = min(max(ty, 0), 63);
+    lo = ok ? ty : 127;
+    hi = ok ? ty : 0;
+#pragma unroll
+    for (int o = 1; o < G; o <<= 1) {
+        lo = min(lo, __shfl_xor(lo, o, 64));
+        hi = max(hi, __shfl_xor(hi, o, 64));
+    }
+}
+// first and last of wave w's rows (row w + 4 q -> q) that a group with corner
+// rows lo .. hi touches
+__device__ __forceinline__ int first_row(int lo, int w) { return max(0, (lo - w + 3) >> 2); }
+__device__ __forceinline__ int last_row(int hi, int w) { return (hi + W3 - 1 - w) >> 2; }
+
+// type 2: a block takes `chunk` consecutive sorted points; for each bin among
+// them the waves load their rows of the region into registers (they stay there
+// for all the bin's points).  Every point's sum depends on that point alone.
+// Masked points (sorted last) are not read.
+constexpr int XS = 20;                      // row stride of the x table
+__global__ void __launch_bounds__(256, 4)
+k_interp3d(const float2 *__restrict__ F, float2 *__restrict__ C, const double *__restrict__ rot,
+           const unsigned *__restrict__ skey, const unsigned *__restrict__ sval,
+           const unsigned *__restrict__ bend, unsigned npts, unsigned nbins, unsigned chunk, Grid3 g, Bins3 bn) {
+    using S = Shape3<16>;
+    __shared__ float Zt[BATCH * RGN], Yt[BATCH * RGN], Xt[BATCH * XS];   // [group][slot][16 points], x: [point][slot]
+    __shared__ float2 part[4][BATCH];
+    __shared__ int meta[BATCH / 16];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int p = threadIdx.x & (BATCH - 1), h = threadIdx.x >> 7;
+    const int n = lane & 15, k4 = lane >> 4;
+    unsigned a = blockIdx.x * chunk;
+    const unsigned stop = min(npts, a + chunk);
+    while (a < stop) {
+        const unsigned bin = __builtin_amdgcn_readfirstlane(skey[a] >> S::YB);
+        if (bin >= nbins) return;   // the masked points: all of the rest (the whole block agrees)
+        const unsigned e = min(stop, bend[bin]);
+        const int b[3] = {(int)(bin / (unsigned)(bn.nb[1] * bn.nb[2])), (int)(bin / (unsigned)bn.nb[2]) % bn.nb[1],
+                          (int)(bin % (unsigned)bn.nb[2])};
+        int s[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) s[i] = bin_first(b[i], g.nf[i], bn.nb[i]);
+        // lane (k4, n): x = n, z = 4 j + k4 of row y = w + 4 q
+        float fr[4][4], fi[4][4];
+        {
+            int xx = s[2] + n;
+            xx -= xx >= g.nf[2] ? g.nf[2] : 0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                int yy = s[1] + w + 4 * q;
+                yy -= yy >= g.nf[1] ? g.nf[1] : 0;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    int zz = s[0] + 4 * j + k4;
+                    zz -= zz >= g.nf[0] ? g.nf[0] : 0;
+                    const float2 v = F[((int64_t)zz * g.nf[1] + yy) * g.nf[2] + xx];
+                    fr[q][j] = v.x;
+                    fi[q][j] = v.y;
+                }
             }
         }
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < RZ * RY * RX; i += 64 * NW) {
-        const int z = i / (RY * RX), y = (i / RX) % RY, x = i % RX;
-        const int zz = c0[0] + z, yy = c0[1] + y, xx = c0[2] + x;
-        if (zz >= bn.pf[0] || yy >= bn.pf[1] || xx >= bn.pf[2]) continue;
-        const int li = S::tidx(z, y, x);
-        float2 s = acc[li];
-        for (int w = 1; w < NW; ++w) {
-            s.x += acc[w * PC + li].x;
-            s.y += acc[w * PC + li].y;
+        for (; a < e; a += BATCH) {
+            const int cnt = (int)min(e - a, (unsigned)BATCH);
+            const bool ok = p < cnt;
+            const unsigned pt = sval[ok ? a + p : a];
+            const Foot ft = foot3(rot, pt, g, s);
+            float *zt = Zt + (p >> 4) * 256 + (p & 15), *yt = Yt + (p >> 4) * 256 + (p & 15), *xt = Xt + p * XS;
+            axis_weights<RGN>(ft.t[0], ft.f[0], h, g.beta, [&](int sl, float v) { zt[16 * sl] = v; });
+            axis_weights<RGN>(ft.t[1], ft.f[1], h, g.beta, [&](int sl, float v) { yt[16 * sl] = v; });
+            axis_weights<RGN>(ft.t[2], ft.f[2], h, g.beta, [&](int sl, float v) { xt[sl] = v; });
+            int lo, hi;
+            group_rows<16>(ft.t[1], ok, lo, hi);
+            if ((threadIdx.x & 15) == 0 && h == 0) meta[p >> 4] = lo | hi << 8;
+            __syncthreads();
+            const int ng = (cnt + 15) >> 4;
+            const int mt = meta[lane & 7];
+            for (int gr = 0; gr < ng; ++gr) {
+                const int m = __builtin_amdgcn_readlane(mt, gr);
+                const int q0 = first_row(m & 255, w), q1 = last_row(m >> 8, w);
+                float zw[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) zw[j] = Zt[gr * 256 + (4 * j + k4) * 16 + n];
+                f32x4 ar = {0.f, 0.f, 0.f, 0.f}, ai = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (q < q0 || q > q1) continue;
+                    const float wy = Yt[gr * 256 + (w + 4 * q) * 16 + n];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float av = zw[j] * wy;
+                        ar = mfma4(av, fr[q][j], ar);
+                        ai = mfma4(av, fi[q][j], ai);
+                    }
+                }
+                // register q: point 4 k4 + q, x = n; summed over x in the 16 lanes
+                const float *xw = Xt + (gr * 16 + 4 * k4) * XS + n;
+                float2 o = make_float2(0.f, 0.f);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float wx = xw[q * XS];
+                    float vr = ar[q] * wx, vi = ai[q] * wx;
+#pragma unroll
+                    for (int d = 1; d < 16; d <<= 1) {
+                        vr += __shfl_xor(vr, d, 64);
+                        vi += __shfl_xor(vi, d, 64);
+                    }
+                    if (n == q) o = make_float2(vr, vi);
+                }
+                if (n < 4) part[w][gr * 16 + 4 * k4 + n] = o;
+            }
+            __syncthreads();
+            if (h == 0 && ok) {
+                const float2 v0 = part[0][p], v1 = part[1][p], v2 = part[2][p], v3 = part[3][p];
+                C[pt] = make_float2((v0.x + v1.x) + (v2.x + v3.x), (v0.y + v1.y) + (v2.y + v3.y));
+            }
         }
-        float2 &f = Fp[((int64_t)zz * bn.pf[1] + yy) * bn.pf[2] + xx];
-        f.x += s.x;
-        f.y += s.y;
+        a = e;
     }
 }
 
-// one wave per light bin of this phase (order: the phase's bins, fullest first)
+// Bins of more than B3_HEAVY points are spread by S::TEAMS teams of four
+// waves, each taking a consecutive part of the bin's points; their sums are
+// added in team order.  Whether a bin is heavy depends only on its own count.
+constexpr unsigned B3_HEAVY = 2048;
+
+// LDS of one team: tables [point][slot] of wz, c wx (re, im) and wy (its rows
+// reordered to [wave][row / 4]), the row strides padded against bank conflicts,
+// and the point groups' rows
+constexpr int ZS = RGN + 1;
+template <typename S> struct SpreadLds {
+    float z[BATCH * ZS], xr[BATCH * ZS], xi[BATCH * ZS];
+    float y[BATCH * (S::ROWS + 4)];
+    int meta[BATCH / 4];
+};
+
+// type 1: adds bin `bin`'s points to the fine grid F with TEAMS teams of four waves
+template <typename S, int TEAMS>
+__device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2 *__restrict__ F,
+                                            const double *__restrict__ rot, const unsigned *__restrict__ sval,
+                                            int bin, unsigned s0, unsigned s1, const Grid3 &g, const Bins3 &bn,
+                                            SpreadLds<S> *lds) {
+    constexpr int NQ = S::ROWS / 4, YS = S::ROWS + 4;
+    const int b[3] = {bin / (bn.nb[1] * bn.nb[2]), (bin / bn.nb[2]) % bn.nb[1], bin % bn.nb[2]};
+    int s[3], ext[3];   // the region's first cell and extent (the bin's corners + W3 - 1)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        s[i] = bin_first(b[i], g.nf[i], bn.nb[i]);
+        ext[i] = bin_first(b[i] + 1, g.nf[i], bn.nb[i]) - s[i] + W3 - 1;
+    }
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
+    const int team = TEAMS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const int p = threadIdx.x & (BATCH - 1), h = (threadIdx.x >> 7) & 1;
+    const int n = lane & 15, k4 = lane >> 4;
+    SpreadLds<S> &L = lds[team];
+    f32x4 ar[NQ], ai[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) ar[q] = ai[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // team t takes the t-th part of the bin's points, in order; every team
+    // runs the same number of batches
+    const unsigned per = ((s1 - s0 + TEAMS - 1) / TEAMS + BATCH - 1) / BATCH * BATCH;
+    const unsigned ws = min(s1, s0 + team * per), we = min(s1, ws + per);
+    const int nit = (int)(per / BATCH);
+    // the next batch's points are fetched during this one
+    auto index = [&](int it) -> unsigned {
+        const unsigned i = ws + (unsigned)it * BATCH + p;
+        return sval[i < we ? i : s0];
+    };
+    unsigned pt = index(0), ptn = nit > 1 ? index(1) : pt;
+    float2 cv = C[pt];
+    for (int it = 0; it < nit; ++it) {
+        const unsigned base = ws + (unsigned)it * BATCH;
+        const int cnt = base < we ? (int)min(we - base, (unsigned)BATCH) : 0;
+        const bool ok = p < cnt;
+        {
+            const Foot ft = foot3(rot, pt, g, s);
+            float *zt = L.z + p * ZS, *xr = L.xr + p * ZS, *xi = L.xi + p * ZS, *yt = L.y + p * YS;
+            const float cr = ok ? cv.x : 0.f, ci = ok ? cv.y : 0.f;
+            // past the last point every product is 0 x a stored weight
+            axis_weights<RGN>(ft.t[0], ft.f[0], h, g.beta, [&](int sl, float v) { zt[sl] = ok ? v : 0.f; });
+            axis_weights<S::ROWS>(ft.t[1], ft.f[1], h, g.beta,
+                                  [&](int sl, float v) { yt[(sl & 3) * NQ + (sl >> 2)] = v; });
+            axis_weights<RGN>(ft.t[2], ft.f[2], h, g.beta, [&](int sl, float v) {
+                xr[sl] = v * cr;
+                xi[sl] = v * ci;
+            });
+            int lo, hi;
+            group_rows<4>(ft.t[1], ok, lo, hi);
+            if ((p & 3) == 0 && h == 0) L.meta[p >> 2] = lo | hi << 8;
+        }
+        __syncthreads();
+        pt = ptn;
+        cv = C[pt];
+        if (it + 2 < nit) ptn = index(it + 2);
+        const int mt = L.meta[lane & 31];
+        const int ng = (cnt + 3) >> 2;
+        const float *zl = L.z + k4 * ZS + n, *xrl = L.xr + k4 * ZS + n, *xil = L.xi + k4 * ZS + n;
+        const float *yl = L.y + k4 * YS + w * NQ;
+        for (int gr = 0; gr < ng; ++gr) {
+            const int m = __builtin_amdgcn_readlane(mt, gr);
+            const int q0 = first_row(m & 255, w), q1 = last_row(m >> 8, w);
+            const float zw = zl[gr * 4 * ZS], br = xrl[gr * 4 * ZS], bi = xil[gr * 4 * ZS];
+            float wy[NQ];
+#pragma unroll
+            for (int q = 0; q < NQ; q += 4)
+                *reinterpret_cast<float4 *>(wy + q) = *reinterpret_cast<const float4 *>(yl + gr * 4 * YS + q);
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                if (q < q0 || q > q1) continue;
+                const float av = zw * wy[q];
+                ar[q] = mfma4(av, br, ar[q]);
+                ai[q] = mfma4(av, bi, ai[q]);
+            }
+        }
+        __syncthreads();
+    }
+    // register i of row slot q: cell (z, y, x) = (4 k4 + i, w + 4 q, n)
+    int xx = s[2] + n;
+    xx -= xx >= g.nf[2] ? g.nf[2] : 0;
+    auto cell = [&](int q, int i, bool &in) -> float2 * {
+        const int y = w + 4 * q, z = 4 * k4 + i;
+        in = y < ext[1] && z < ext[0] && n < ext[2];
+        int yy = s[1] + y, zz = s[0] + z;
+        yy -= yy >= g.nf[1] ? g.nf[1] : 0;
+        zz -= zz >= g.nf[0] ? g.nf[0] : 0;
+        return F + ((int64_t)zz * g.nf[1] + yy) * g.nf[2] + xx;
+    };
+    if constexpr (TEAMS == 1) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            float2 v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                bool in;
+                const float2 *f = cell(q, i, in);
+                if (in) v[i] = *f;
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                bool in;
+                float2 *f = cell(q, i, in);
+                if (in) *f = make_float2(v[i].x + ar[q][i], v[i].y + ai[q][i]);
+            }
+        }
+    } else {
+        // row slot by row slot through LDS (the tables' space): team q mod
+        // TEAMS adds the teams' sums in team order
+        f32x4 *ex = reinterpret_cast<f32x4 *>(lds);   // [team][wave][re, im][lane]
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            ex[((team * 4 + w) * 2) * 64 + lane] = ar[q];
+            ex[((team * 4 + w) * 2 + 1) * 64 + lane] = ai[q];
+            __syncthreads();
+            if (q % TEAMS == team) {
+                f32x4 sr = ex[(w * 2) * 64 + lane], si = ex[(w * 2 + 1) * 64 + lane];
+                for (int t = 1; t < TEAMS; ++t) {
+                    sr += ex[((t * 4 + w) * 2) * 64 + lane];
+                    si += ex[((t * 4 + w) * 2 + 1) * 64 + lane];
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    bool in;
+                    float2 *f = cell(q, i, in);
+                    if (in) {
+                        const float2 v = *f;
+                        *f = make_float2(v.x + sr[i], v.y + si[i]);
+                    }
+                }
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// one block per light bin of this phase (order: the phase's bins, fullest first)
 template <typename S>
-__global__ void __launch_bounds__(64)
-k_spread3d_bin(const float2 *__restrict__ C, float2 *__restrict__ Fp, const double *__restrict__ rot,
+__global__ void __launch_bounds__(256)
+k_spread3d_bin(const float2 *__restrict__ C, float2 *__restrict__ F, const double *__restrict__ rot,
                const unsigned *__restrict__ sval, const unsigned *__restrict__ bstart,
                const unsigned *__restrict__ bend, const unsigned *__restrict__ order, Grid3 g, Bins3 bn) {
-    const int bid = (int)order[blockIdx.x];
-    const unsigned s0 = bstart[bid], s1 = bend[bid];
+    const int bin = __builtin_amdgcn_readfirstlane(order[blockIdx.x]);
+    const unsigned s0 = bstart[bin], s1 = bend[bin];
     if (s0 >= s1 || s1 - s0 > B3_HEAVY) return;   // empty, or a heavy bin
-    spread3_bin<S, 1>(C, Fp, rot, sval, bid, s0, s1, g, bn, reinterpret_cast<float2 *>(lc_smem));
+    spread3_bin<S, 1>(C, F, rot, sval, bin, s0, s1, g, bn, reinterpret_cast<SpreadLds<S> *>(lc_smem));
 }
 
 // the phase's heavy bins (a prefix of its order): each block takes bins
 // j, j + gridDim.x, ... until the first light one
 template <typename S>
-__global__ void __launch_bounds__(64 * S::NWH)
-k_spread3d_bin_heavy(const float2 *__restrict__ C, float2 *__restrict__ Fp, const double *__restrict__ rot,
+__global__ void __launch_bounds__(256 * S::TEAMS)
+k_spread3d_bin_heavy(const float2 *__restrict__ C, float2 *__restrict__ F, const double *__restrict__ rot,
                      const unsigned *__restrict__ sval, const unsigned *__restrict__ bstart,
                      const unsigned *__restrict__ bend, const unsigned *__restrict__ order, unsigned nphase,
                      Grid3 g, Bins3 bn) {
     for (unsigned j = blockIdx.x; j < nphase; j += gridDim.x) {
-        const int bid = (int)order[j];
-        const unsigned s0 = bstart[bid], s1 = bend[bid];
+        const int bin = __builtin_amdgcn_readfirstlane(order[j]);
+        const unsigned s0 = bstart[bin], s1 = bend[bin];
         if (s1 - s0 <= B3_HEAVY) break;   // the order is fullest first: the rest are light
-        spread3_bin<S, S::NWH>(C, Fp, rot, sval, bid, s0, s1, g, bn, reinterpret_cast<float2 *>(lc_smem));
-        __syncthreads();   // the copies are cleared for the next bin only after every wave has flushed
+        spread3_bin<S, S::TEAMS>(C, F, rot, sval, bin, s0, s1, g, bn, reinterpret_cast<SpreadLds<S> *>(lc_smem));
     }
 }
 
@@ -436,36 +595,6 @@ __global__ void k_zero_u32(unsigned *p, int64_t n) {
 __global__ void k_zero2(float2 *p, int64_t n) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         p[i] = make_float2(0.f, 0.f);
-}
-
-// F = Fp wrapped onto the periodic fine grid: F[z][y][x] sums the (up to 8)
-// cells of Fp at (z + az nf0, y + ay nf1, x + ax nf2), az, ay, ax in {0, 1},
-// in that fixed order
-__global__ void k_fold3d(const float2 *__restrict__ Fp, float2 *__restrict__ F, Grid3 g, Bins3 bn) {
-    const int64_t n = (int64_t)g.nf[0] * g.nf[1] * g.nf[2];
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int z = (int)(i / ((int64_t)g.nf[1] * g.nf[2]));
-        const int64_t rem = i - (int64_t)z * g.nf[1] * g.nf[2];
-        const int y = (int)(rem / g.nf[2]), x = (int)(rem - (int64_t)y * g.nf[2]);
-        float2 s = make_float2(0.f, 0.f);
-        for (int az = 0; az < 2; ++az) {
-            const int zz = z + az * g.nf[0];
-            if (zz >= bn.pf[0]) break;
-            for (int ay = 0; ay < 2; ++ay) {
-                const int yy = y + ay * g.nf[1];
-                if (yy >= bn.pf[1]) break;
-                for (int ax = 0; ax < 2; ++ax) {
-                    const int xx = x + ax * g.nf[2];
-                    if (xx >= bn.pf[2]) break;
-                    const float2 v = Fp[((int64_t)zz * bn.pf[1] + yy) * bn.pf[2] + xx];
-                    s.x += v.x;
-                    s.y += v.y;
-                }
-            }
-        }
-        F[i] = s;
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -810,83 +939,77 @@ Grid3 grid3(const Geom3D &g, bool mask) {
 
 struct Work3 {
     float2 *C, *F, *V1, *V2;
-    // type 1 only: the spread's padded fine grid, the points' bin keys and
-    // indices (unsorted, sorted), the bins' runs and the sort's scratch
-    float2 *Fp;
+    // the points' keys and indices (unsorted, sorted), the bins' runs, the
+    // bins' launch order and the sorts' scratch
     unsigned *key_a, *key_b, *val_a, *val_b, *bstart, *bend;
-    unsigned *okey_a, *okey_b, *oval_a, *order;   // the bins' launch order
+    unsigned *okey_a, *okey_b, *oval_a, *order;
     void *sort_tmp;
     size_t sort_bytes;
 };
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-int bins_of(int nf, int b) { return (nf + b - 1) / b; }
-template <typename S> unsigned nbins_of(const int nf[3]) {
-    return (unsigned)bins_of(nf[0], S::BZ) * bins_of(nf[1], S::BY) * bins_of(nf[2], S::BX);
+template <typename S> Bins3 bins_of(const int nf[3]) {
+    const Bins3 bn{{bins_along(nf[0], BE), bins_along(nf[1], S::EY), bins_along(nf[2], BE)}};
+    const int edge[3] = {BE, S::EY, BE};
+    for (int a = 0; a < 3; ++a)
+        LC_REQUIRE(nf[a] >= RGN && ceil_div(nf[a], bn.nb[a]) <= edge[a], "3-D NUFFT: no bins for this fine grid");
+    return bn;
 }
-// the most bins any compiled shape makes of this grid (work buffers fit every shape)
+unsigned count_of(const Bins3 &bn) { return (unsigned)bn.nb[0] * bn.nb[1] * bn.nb[2]; }
+// the most bins any compiled shape makes of this grid, and the most values
+// their sort keys take (work buffers fit every shape)
 unsigned nbins_max(const int nf[3]) {
     unsigned m = 0;
-    for (int i = 0; i < N_SHAPES3; ++i) with_shape3(i, [&](auto sh) { m = std::max(m, nbins_of<decltype(sh)>(nf)); });
+    for (int i = 0; i < N_SHAPES3; ++i)
+        with_shape3(i, [&](auto sh) { m = std::max(m, count_of(bins_of<decltype(sh)>(nf))); });
     return m;
 }
 
-// bits of the sort key: bins 0 .. nbins - 1 and nbins for dropped points
-int key_bits(unsigned nbins) {
+// bits of the sort key: bins 0 .. nbins - 1 and nbins for dropped points, above
+// the yb bits of the corner row
+int key_bits(unsigned nbins, int yb) {
     int b = 1;
     while (b < 32 && (1ull << b) <= nbins) ++b;
-    return b;
+    LC_REQUIRE(b + yb <= 32, "3-D NUFFT: too many bins");
+    return b + yb;
 }
 
 size_t sort_tmp_bytes(int64_t npts, unsigned nbins) {
     size_t tb = 0, to = 0;
     LC_HIP(rocprim::radix_sort_pairs(nullptr, tb, (unsigned *)nullptr, (unsigned *)nullptr, (unsigned *)nullptr,
-                                     (unsigned *)nullptr, (size_t)npts, 0, key_bits(nbins), (hipStream_t)0));
+                                     (unsigned *)nullptr, (size_t)npts, 0, 32, (hipStream_t)0));
     LC_HIP(rocprim::radix_sort_pairs(nullptr, to, (unsigned *)nullptr, (unsigned *)nullptr, (unsigned *)nullptr,
-                                     (unsigned *)nullptr, (size_t)nbins, 0, MAX_ORDER_BITS, (hipStream_t)0));
+                                     (unsigned *)nullptr, (size_t)nbins, 0, ORDER_BITS, (hipStream_t)0));
     return std::max(tb, to);
 }
 
-// bytes of the type-1 spread's buffers beyond the fine grid
+// bytes of the sorted points' buffers
 size_t spread_bytes(int64_t npts, const int nf[3]) {
     const unsigned nbins = nbins_max(nf);
-    return align256(sizeof(float2) * (size_t)(nf[0] + W3 - 1) * (nf[1] + W3 - 1) * (nf[2] + W3 - 1)) +
-           4 * align256(sizeof(unsigned) * (size_t)npts) + 6 * align256(sizeof(unsigned) * (size_t)nbins) +
+    return 4 * align256(sizeof(unsigned) * (size_t)npts) + 6 * align256(sizeof(unsigned) * (size_t)nbins) +
            align256(sort_tmp_bytes(npts, nbins));
 }
 
-Work3 work3(Ctx &c, const Geom3D &g, bool spread = false) {
+Work3 work3(Ctx &c, const Geom3D &g) {
     const Nufft3D &u = g.nu;
     const int64_t npts = (int64_t)g.nproj * g.nrows * g.ncols;
+    LC_REQUIRE(npts < (int64_t)UINT32_MAX, "3-D projector: more than 2^32 detector points");
     const size_t bC = align256(sizeof(float2) * (size_t)npts);
     const size_t bF = align256(sizeof(float2) * (size_t)u.nf[0] * u.nf[1] * u.nf[2]);
     const size_t bV1 = align256(sizeof(float2) * (size_t)u.nf[0] * u.nf[1] * g.n3);
     const size_t bV2 = align256(sizeof(float2) * (size_t)u.nf[0] * g.n2 * g.n3);
     const size_t base = bC + bF + bV1 + bV2;
-    Work3 w{};
-    if (!spread) {
-        char *ws = reinterpret_cast<char *>(c.scratch(4, base));
-        w.C = reinterpret_cast<float2 *>(ws);
-        w.F = reinterpret_cast<float2 *>(ws + bC);
-        w.V1 = reinterpret_cast<float2 *>(ws + bC + bF);
-        w.V2 = reinterpret_cast<float2 *>(ws + bC + bF + bV1);
-        return w;
-    }
-    LC_REQUIRE(npts < (int64_t)UINT32_MAX, "backproj: more than 2^32 detector points");
     const unsigned nbins = nbins_max(u.nf);
-    const size_t bFp = align256(sizeof(float2) * (size_t)(u.nf[0] + W3 - 1) * (u.nf[1] + W3 - 1) * (u.nf[2] + W3 - 1));
     const size_t bK = align256(sizeof(unsigned) * (size_t)npts);
     const size_t bB = align256(sizeof(unsigned) * (size_t)nbins);
-    const size_t bT = sort_tmp_bytes(npts, nbins);
-    char *ws = reinterpret_cast<char *>(c.scratch(4, base + bFp + 4 * bK + 6 * bB + align256(bT)));
+    Work3 w{};
+    char *ws = reinterpret_cast<char *>(c.scratch(4, base + spread_bytes(npts, u.nf)));
     w.C = reinterpret_cast<float2 *>(ws);
     w.F = reinterpret_cast<float2 *>(ws + bC);
     w.V1 = reinterpret_cast<float2 *>(ws + bC + bF);
     w.V2 = reinterpret_cast<float2 *>(ws + bC + bF + bV1);
     char *q = ws + base;
-    w.Fp = reinterpret_cast<float2 *>(q);
-    q += bFp;
     w.key_a = reinterpret_cast<unsigned *>(q);
     w.key_b = reinterpret_cast<unsigned *>(q + bK);
     w.val_a = reinterpret_cast<unsigned *>(q + 2 * bK);
@@ -900,7 +1023,7 @@ Work3 work3(Ctx &c, const Geom3D &g, bool spread = false) {
     w.order = reinterpret_cast<unsigned *>(q + 5 * bB);
     q += 6 * bB;
     w.sort_tmp = q;
-    w.sort_bytes = bT;
+    w.sort_bytes = sort_tmp_bytes(npts, nbins);
     return w;
 }
 
@@ -988,6 +1111,28 @@ void det_axis(Ctx &c, const DetLine &d, const void *in, void *out, int64_t outer
     LC_HIP(hipGetLastError());
 }
 
+// orders the grid's points by the bins of shape S (w.key_b, w.val_b, w.bstart,
+// w.bend); drop: values of masked points are cleared there
+template <typename S> Bins3 sort_points(Ctx &c, const Geom3D &g, const Work3 &w, const Grid3 &gg, float2 *drop) {
+    const Bins3 bn = bins_of<S>(g.nu.nf);
+    const unsigned nbins = count_of(bn);
+    const int64_t npts = (int64_t)g.nproj * g.nrows * g.ncols;
+    const int bits = key_bits(nbins, S::YB);
+    hipLaunchKernelGGL(k_bin_keys<S>, dim3((unsigned)ceil_div(npts, 256)), dim3(256), 0, c.stream(),
+                       g.d_rot.as<double>(), gg, bn, w.key_a, w.val_a, npts, nbins, drop);
+    LC_HIP(hipGetLastError());
+    size_t tb = w.sort_bytes;
+    LC_HIP(rocprim::radix_sort_pairs(w.sort_tmp, tb, w.key_a, w.key_b, w.val_a, w.val_b, (size_t)npts, 0, bits,
+                                     c.stream()));
+    hipLaunchKernelGGL(k_zero_u32, dim3(1024), dim3(256), 0, c.stream(), w.bstart,
+                       (int64_t)(w.bend - w.bstart) + nbins);
+    hipLaunchKernelGGL(k_bin_ranges, dim3((unsigned)ceil_div(npts, 256)), dim3(256), 0, c.stream(), w.key_b,
+                       npts, w.bstart, w.bend, nbins, S::YB);
+    LC_HIP(hipGetLastError());
+    return bn;
+}
+
+// vol -> w.C; leaves the points sorted by the bins of Shape3<16>
 void type2_3d(Ctx &c, const Geom3D &g, const Work3 &w, const float *vol, bool mask) {
     const Nufft3D &u = g.nu;
     const int n1 = (int)g.n1, n2 = (int)g.n2, n3 = (int)g.n3;
@@ -1000,66 +1145,51 @@ void type2_3d(Ctx &c, const Geom3D &g, const Work3 &w, const float *vol, bool ma
     nu_axis<2, false, false>(c, w.V1, w.F, (int64_t)u.nf[0] * u.nf[1], 1, u.nf[2], n3,
                              corr + u.coff[2], 1.0f, u.plan[2]);
     const Grid3 gg = grid3(g, mask);
-    const int64_t npts = g.nproj * g.nrows * g.ncols;
-    // a wave of 64 points, four waves per block
-    hipLaunchKernelGGL(k_interp3d, dim3(ceil_div(ceil_div(npts, (int64_t)64), (int64_t)4)), dim3(256), 0,
-                       c.stream(), w.F, w.C, g.d_rot.as<double>(), gg);
+    const int64_t npts = (int64_t)g.nproj * g.nrows * g.ncols;
+    const Bins3 bn = sort_points<Shape3<16>>(c, g, w, gg, w.C);
+    // long runs read a bin's region once; short ones keep a small grid's blocks many
+    const unsigned chunk = (unsigned)std::min<int64_t>(1024, std::max<int64_t>(1, npts / (4096 * BATCH)) * BATCH);
+    hipLaunchKernelGGL(k_interp3d, dim3((unsigned)ceil_div(npts, chunk)), dim3(256), 0, c.stream(), w.F, w.C,
+                       g.d_rot.as<double>(), w.key_b, w.val_b, w.bend, (unsigned)npts, count_of(bn), chunk, gg, bn);
     LC_HIP(hipGetLastError());
 }
 
-// the sorted-bin spread with bin shape S: C -> Fp (padded, not yet folded)
-template <typename S> Bins3 spread3d(Ctx &c, const Geom3D &g, const Work3 &w, const Grid3 &gg) {
+// the sorted-bin spread with region shape S: w.C -> w.F (sorted: the points
+// are already in the order of S's bins)
+template <typename S> void spread3d(Ctx &c, const Geom3D &g, const Work3 &w, const Grid3 &gg, bool sorted) {
     const Nufft3D &u = g.nu;
-    Bins3 bn;
-    int64_t npad = 1;
-    const int edge[3] = {S::BZ, S::BY, S::BX};
-    for (int a = 0; a < 3; ++a) {
-        bn.nb[a] = bins_of(u.nf[a], edge[a]);
-        bn.pf[a] = u.nf[a] + W3 - 1;
-        npad *= bn.pf[a];
-    }
-    const unsigned nbins = (unsigned)bn.nb[0] * bn.nb[1] * bn.nb[2];
-    const int64_t npts = (int64_t)g.nproj * g.nrows * g.ncols;
-    // points ordered by bin, point order kept inside a bin
-    hipLaunchKernelGGL(k_bin_keys<S>, dim3((unsigned)ceil_div(npts, 256)), dim3(256), 0, c.stream(),
-                       g.d_rot.as<double>(), gg, bn, w.key_a, w.val_a, npts, nbins);
-    LC_HIP(hipGetLastError());
-    size_t tb = w.sort_bytes;
-    LC_HIP(rocprim::radix_sort_pairs(w.sort_tmp, tb, w.key_a, w.key_b, w.val_a, w.val_b, (size_t)npts, 0,
-                                     key_bits(nbins), c.stream()));
-    hipLaunchKernelGGL(k_zero_u32, dim3(1024), dim3(256), 0, c.stream(), w.bstart,
-                       (int64_t)(w.bend - w.bstart) + nbins);
-    hipLaunchKernelGGL(k_bin_ranges, dim3((unsigned)ceil_div(npts, 256)), dim3(256), 0, c.stream(), w.key_b,
-                       npts, w.bstart, w.bend, nbins);
-    hipLaunchKernelGGL(k_bin_order_keys<S>, dim3(ceil_div(nbins, 256)), dim3(256), 0, c.stream(), w.bstart,
+    const Bins3 bn = sorted ? bins_of<S>(u.nf) : sort_points<S>(c, g, w, gg, nullptr);
+    const unsigned nbins = count_of(bn);
+    hipLaunchKernelGGL(k_bin_order_keys, dim3(ceil_div(nbins, 256)), dim3(256), 0, c.stream(), w.bstart,
                        w.bend, bn, w.okey_a, w.oval_a, nbins);
     LC_HIP(hipGetLastError());
-    tb = w.sort_bytes;
+    size_t tb = w.sort_bytes;
     LC_HIP(rocprim::radix_sort_pairs(w.sort_tmp, tb, w.okey_a, w.okey_b, w.oval_a, w.order, (size_t)nbins, 0,
-                                     S::ORDER_BITS, c.stream()));
-    hipLaunchKernelGGL(k_zero2, dim3(2048), dim3(256), 0, c.stream(), w.Fp, npad);
+                                     ORDER_BITS, c.stream()));
+    hipLaunchKernelGGL(k_zero2, dim3(2048), dim3(256), 0, c.stream(), w.F,
+                       (int64_t)u.nf[0] * u.nf[1] * u.nf[2]);
     LC_HIP(hipGetLastError());
-    const size_t shs = sizeof(float2) * S::PC;
     int64_t first = 0;   // the phase's first entry in the launch order
-    for (int ph = 0; ph < S::NPH; ++ph) {
-        // phase (rz, ry, rx): the bins whose index along each axis is r mod P
-        const int r[3] = {ph / (S::PY * S::PX), (ph / S::PX) % S::PY, ph % S::PX}, per[3] = {S::PZ, S::PY, S::PX};
+    int per[3];
+    for (int a = 0; a < 3; ++a) per[a] = phases_along(bn.nb[a]);
+    for (int ph = 0; ph < per[0] * per[1] * per[2]; ++ph) {
+        // phase (rz, ry, rx): the bins whose index along each axis is r mod its phases
+        const int r[3] = {ph / (per[1] * per[2]), (ph / per[2]) % per[1], ph % per[2]};
         int nblk = 1;
-        for (int a = 0; a < 3; ++a) nblk *= std::max(0, (bn.nb[a] - r[a] + per[a] - 1) / per[a]);
-        if (nblk == 0) continue;
-        hipLaunchKernelGGL(k_spread3d_bin_heavy<S>, dim3(std::min(nblk, 256)), dim3(64 * S::NWH), shs * S::NWH,
-                           c.stream(), w.C, w.Fp, g.d_rot.as<double>(), w.val_b, w.bstart, w.bend, w.order + first,
-                           (unsigned)nblk, gg, bn);
-        hipLaunchKernelGGL(k_spread3d_bin<S>, dim3(nblk), dim3(64), shs, c.stream(), w.C, w.Fp,
+        for (int a = 0; a < 3; ++a) nblk *= (bn.nb[a] - r[a] + per[a] - 1) / per[a];
+        hipLaunchKernelGGL(k_spread3d_bin_heavy<S>, dim3(std::min(nblk, 256)), dim3(256 * S::TEAMS),
+                           sizeof(SpreadLds<S>) * S::TEAMS, c.stream(), w.C, w.F, g.d_rot.as<double>(), w.val_b,
+                           w.bstart, w.bend, w.order + first, (unsigned)nblk, gg, bn);
+        hipLaunchKernelGGL(k_spread3d_bin<S>, dim3(nblk), dim3(256), sizeof(SpreadLds<S>), c.stream(), w.C, w.F,
                            g.d_rot.as<double>(), w.val_b, w.bstart, w.bend, w.order + first, gg, bn);
         LC_HIP(hipGetLastError());
         first += nblk;
     }
-    return bn;
 }
 
+// sorted: type2_3d has just run on the same points
 void type1_3d(Ctx &c, const Geom3D &g, const Work3 &w, float *vol, bool mask, const double *shifts,
-              float scale) {
+              float scale, bool sorted) {
     const Nufft3D &u = g.nu;
     const int n1 = (int)g.n1, n2 = (int)g.n2, n3 = (int)g.n3;
     const Grid3 gg = grid3(g, mask);
@@ -1069,13 +1199,10 @@ void type1_3d(Ctx &c, const Geom3D &g, const Work3 &w, float *vol, bool mask, co
                            shifts, gg, np);
         LC_HIP(hipGetLastError());
     }
-    LC_REQUIRE(w.Fp != nullptr, "type1_3d: no spread buffers in the work area");
-    Bins3 bn;
-    with_shape3(c.nu3_shape(u.nf), [&](auto sh) { bn = spread3d<decltype(sh)>(c, g, w, gg); });
-    const int64_t nfine = (int64_t)u.nf[0] * u.nf[1] * u.nf[2];
-    hipLaunchKernelGGL(k_fold3d, dim3((unsigned)std::min<int64_t>(8192, ceil_div(nfine, 256))), dim3(256), 0,
-                       c.stream(), w.Fp, w.F, gg, bn);
-    LC_HIP(hipGetLastError());
+    with_shape3(c.nu3_shape(u.nf), [&](auto sh) {
+        using S = decltype(sh);
+        spread3d<S>(c, g, w, gg, sorted && S::ROWS == 16);
+    });
     const float *corr = g.nu.corr.as<float>();
     // x: rows (nf0*nf1, nf2) -> (nf0*nf1, n3)
     nu_axis<1, false, false>(c, w.F, w.V1, (int64_t)u.nf[0] * u.nf[1], 1, u.nf[2], n3,
@@ -1109,20 +1236,20 @@ void forward3d_dev(Ctx &c, Geom3D &g, const float *vol, float *proj) {
 // projection or nullptr
 void backproj3d_dev(Ctx &c, Geom3D &g, const float *proj, float *vol, const double *shifts) {
     nu3_check(c, g);
-    const Work3 w = work3(c, g, true);
+    const Work3 w = work3(c, g);
     const int nr = (int)g.nrows, nc = (int)g.ncols;
     // fftshift2 -> fft2 -> ifftshift2 along x then y
     det_axis<true, false>(c, g.nu.det_x, proj, w.C, g.nproj * nr, 1, nc / 2, nc / 2 + (nc & 1), -1, 1.0f);
     det_axis<false, false>(c, g.nu.det_y, w.C, w.C, g.nproj, nc, nr / 2, nr / 2 + (nr & 1), -1, 1.0f);
-    type1_3d(c, g, w, vol, true, shifts, 1.0f / ((float)nr * (float)nc));
+    type1_3d(c, g, w, vol, true, shifts, 1.0f / ((float)nr * (float)nc), false);
 }
 
 // sysmat(x, grid) (src/gradient.cpp:32-41): Re(T1(T2 x)) / (nrows ncols), no mask
 void sysmat3d_nufft_dev(Ctx &c, Geom3D &g, const float *x, float *y) {
     nu3_check(c, g);
-    const Work3 w = work3(c, g, true);
+    const Work3 w = work3(c, g);
     type2_3d(c, g, w, x, false);
-    type1_3d(c, g, w, y, false, nullptr, 1.0f / ((float)g.nrows * (float)g.ncols));
+    type1_3d(c, g, w, y, false, nullptr, 1.0f / ((float)g.nrows * (float)g.ncols), true);
 }
 
 // device bytes of a 3-D back-projection's spread beyond the fine grid (the

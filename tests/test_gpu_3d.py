@@ -227,6 +227,37 @@ def test_backproj3d_mid_size_matches_oracle(lc, orc64, dims, nproj, nrows, ncols
     assert np.array_equal(lc.backproj(proj, g, dims, sh), x)
 
 
+# (recon dims, nproj, nrows, ncols): fine grids of 16 .. 81 cells per axis, two,
+# three (24 and 27 cells) and more bins of 7 to 9 corners; the last one puts
+# over 2048 points into its bins, in no multiple of a table of points
+BIN_EDGES = [((8, 12, 13), 24, 11, 16), ((9, 13, 18), 24, 12, 15), ((12, 16, 40), 20, 16, 31),
+             ((13, 27, 24), 20, 17, 30), ((6, 16, 16), 331, 13, 35)]
+
+
+@pytest.mark.parametrize("dims,nproj,nrows,ncols", BIN_EDGES)
+def test_projectors3d_bin_edges_match_oracle(lc, orc64, dims, nproj, nrows, ncols):
+    announce(f"projectors3d bin edges dims={dims} det=({nrows},{ncols})")
+    rng = np.random.default_rng(61 + nproj)
+    th, ga, be = lamino_angles(nproj, -30.0)
+    g = lc.PolarGrid(th, ga, be, nrows, ncols)
+    vol, proj = rng.random(dims), rng.standard_normal((nproj, nrows, ncols))
+    yr = orc64.forward3d(vol, th, ga, be, nrows, ncols, tol=1e-12)
+    xr = orc64.backproj3d(proj, th, ga, be, dims, tol=1e-12)
+    assert rel_l2(lc.forward(vol, g), yr) < PROJ_TOL
+    ctx = lc.Context(0)
+    try:
+        psf = lc.PointSpreadFunction(g, dims, ctx=ctx, lazy=True)
+        for shape in range(3):
+            ctx.set_tuning3d(psf, shape)
+            x = lc.backproj(proj, g, dims, ctx=ctx)
+            err = rel_l2(x, xr)
+            print(f"shape {shape}: rel_l2 = {err:.3e}")
+            assert err < PROJ_TOL
+            assert np.array_equal(lc.backproj(proj, g, dims, ctx=ctx), x)
+    finally:
+        ctx.close()
+
+
 def test_backproj3d_bin_shapes_and_autotune(lc, orc64):
     # every compiled bin shape of the spread (0: 4x4x8, 1: 8x4x4, 2: 8x8x8
     # corner cells) gives the oracle's back-projection, deterministically;
