@@ -227,6 +227,34 @@ def test_backproj3d_mid_size_matches_oracle(lc, orc64, dims, nproj, nrows, ncols
     assert np.array_equal(lc.backproj(proj, g, dims, sh), x)
 
 
+# tilts per projection and the span of theta: one tilt over a full turn (opposite
+# projections coincide: even and odd counts), two tilts, a tilt per projection
+# (no two share a column direction), and repeated angles
+@pytest.mark.parametrize("kind,nproj", [("turn", 24), ("turn", 25), ("two", 24), ("each", 11), ("repeat", 12),
+                                        ("beta", 18)])
+def test_psf3d_projection_groups_match_oracle(lc, orc64, kind, nproj):
+    announce(f"psf3d groups {kind} nproj={nproj}")
+    dims, nrows, ncols = (5, 22, 22), 9, 21
+    th = np.arange(nproj) * (2 * np.pi / nproj)
+    ga, be = np.full(nproj, -np.pi / 6), np.zeros(nproj)
+    if kind == "two":
+        ga[nproj // 2:] = 0.3
+    elif kind == "each":
+        ga = np.linspace(-0.6, 0.2, nproj)
+    elif kind == "repeat":
+        th = np.repeat(th[::3], 3)
+    elif kind == "beta":
+        be[:] = 0.2
+    psf = lc.PointSpreadFunction(lc.PolarGrid(th, ga, be, nrows, ncols), dims)
+    P = orc64.psf3d(th, ga, be, nrows, ncols, dims, method=0)
+    x = np.random.default_rng(5).random(dims)
+    ref = P.convolve(x)
+    # FP32 operator: a few ulp of FP32; FP64 operator: phases of magnitude
+    # pi |m| < 200 in FP64 (3e-14), times the denominators' margin
+    assert rel_l2(psf.convolve(x.astype(np.float32)), ref) < 1e-6
+    assert rel_l2(psf.convolve(x), ref) < 1e-12
+
+
 # (recon dims, nproj, nrows, ncols): fine grids of 16 .. 81 cells per axis, two,
 # three (24 and 27 cells) and more bins of 7 to 9 corners; the last one puts
 # over 2048 points into its bins, in no multiple of a table of points
