@@ -19,8 +19,9 @@ struct Nufft2D {
     DBuf corr;            // float[N]
     DBuf cs;              // double2[nang]: (cos theta, sin theta), FP64
     FftPlan plan_nf{};    // fine-grid FFT
-    FftPlan plan_det{};   // detector FFT (valid if det_fast)
-    bool det_fast = false;
+    FftPlan plan_det{};   // detector FFT (det_fast: of the width; det_blue: Bluestein length)
+    bool det_fast = false, det_blue = false;
+    DBuf chirp;           // det_blue: double2 chirp[nrad], then its spectrum [plan_det.L]
     bool ready = false;
 };
 

@@ -19,6 +19,7 @@
 // one point at a time with the 8 x 8 footprint spread over the 64 lanes.  The
 // copies are summed in a fixed order at the end.
 #include <cmath>
+#include <complex>
 
 #include <rocprim/device/device_radix_sort.hpp>
 
@@ -119,7 +120,65 @@ k_det_fft(const float *__restrict__ real_in, const float2 *__restrict__ cplx_in,
     }
 }
 
-// direct DFT fallback for detector widths that are not 2^p 3^q
+// The same for widths that are not 2^p 3^q (up to 2048): Bluestein's algorithm
+// with a power-of-two length L >= 2 n - 1, in FP64 (as the direct sum below
+// accumulates; the FP64 rate equals that of unpacked FP32 and the rows are few):
+//   X_m = a_m sum_k (x_k a_k) b_{m-k},  a_k = e^{SIGN i pi k^2 / n},  b_k = conj(a_k)
+// chirp: e^{i pi k^2 / n}; bhat: FFT-(b) / L for SIGN -1 (b is even, so the
+// SIGN +1 spectrum is its conjugate).  Rows per block and slices as above.
+// 1440 rows of 511: 25 us against 516 us for the direct sum.
+template <int SIGN, int NT, int MAXE, int LC>
+__global__ void __launch_bounds__(NT)
+k_det_blue(const float *__restrict__ real_in, const float2 *__restrict__ cplx_in,
+           float2 *__restrict__ cplx_out, float *__restrict__ real_out, int nrows, int n, int nl,
+           FftPlan plan, const double2 *__restrict__ tw, const double2 *__restrict__ chirp,
+           const double2 *__restrict__ bhat, float scale) {
+    double2 *buf = reinterpret_cast<double2 *>(lc_smem);
+    const int L = LC > 0 ? LC : plan.L;
+    const int lrow0 = blockIdx.x * nl;
+    const int nloc = min(nl, nrows - lrow0);
+    const int64_t row0 = (int64_t)blockIdx.y * nrows + lrow0;
+    const int dfw = n / 2, dinv = n / 2 + (n & 1);
+    const int din = SIGN < 0 ? dfw : dinv, dout = SIGN < 0 ? dinv : dfw;
+    auto phase = [&](int k) { return SIGN < 0 ? cconj(chirp[k]) : chirp[k]; };
+    for (int idx = threadIdx.x; idx < nl * L; idx += NT) {
+        const int l = idx / L, k = idx - l * L;
+        double2 v = make_double2(0.0, 0.0);
+        if (l < nloc && k < n) {
+            int src = k + din;
+            if (src >= n) src -= n;
+            const int64_t q = (row0 + l) * n + src;
+            if constexpr (SIGN < 0) v = cscale(phase(k), (double)real_in[q]);
+            else v = cmul(phase(k), make_double2(cplx_in[q].x, cplx_in[q].y));
+        }
+        buf[lds_row(l, k, L)] = v;
+    }
+    __syncthreads();
+    auto fft = [&](auto sign) {
+        constexpr int SG = decltype(sign)::value;
+        if constexpr (LC > 0) fft_lds_ct<double, LC, SG, NT, MAXE, false>(buf, nl, 0, tw);
+        else fft_lds<double, SG, NT, MAXE, false>(buf, nl, L, plan, tw);
+    };
+    fft(std::integral_constant<int, -1>{});
+    for (int idx = threadIdx.x; idx < nl * L; idx += NT) {
+        const int l = idx / L, k = idx - l * L;
+        double2 *p = buf + lds_row(l, k, L);
+        *p = cmul(*p, SIGN < 0 ? bhat[k] : cconj(bhat[k]));
+    }
+    __syncthreads();
+    fft(std::integral_constant<int, 1>{});
+    for (int idx = threadIdx.x; idx < nloc * n; idx += NT) {
+        const int l = idx / n, k = idx - l * n;
+        int src = k + dout;
+        if (src >= n) src -= n;
+        const double2 v = cmul(buf[lds_row(l, src, L)], phase(src));
+        const int64_t q = (row0 + l) * n + k;
+        if constexpr (SIGN < 0) cplx_out[q] = make_float2((float)v.x, (float)v.y);
+        else real_out[q] = (float)v.x * scale;
+    }
+}
+
+// direct DFT for widths above 2048 that are not 2^p 3^q, or above 4096
 template <int SIGN>
 __global__ void k_det_dft(const float *__restrict__ real_in, const float2 *__restrict__ cplx_in,
                           float2 *__restrict__ cplx_out, float *__restrict__ real_out, int nrows,
@@ -762,6 +821,44 @@ int nufft2d_fine_n(int64_t N) {
     return (int)nf;
 }
 
+// longest detector line in LDS: NU_NT * NU_ME values
+constexpr int DET_FFT_MAX = 4096;
+
+// Bluestein tables of a detector of n columns: chirp and chirp spectrum in FP64
+static void det_blue_init(Ctx &c, Nufft2D &u, int n) {
+    int L = 16;
+    while (L < 2 * n - 1) L *= 2;
+    LC_REQUIRE(fft_make_plan(L, u.plan_det), "detector transform: no Bluestein length");
+    std::vector<double2> t(n + L);   // chirp, then b -> bhat
+    std::vector<std::complex<double>> b(L, 0.0);
+    for (int k = 0; k < n; ++k) {
+        const double ang = M_PI * (double)(((int64_t)k * k) % (2 * (int64_t)n)) / (double)n;
+        t[k] = make_double2(std::cos(ang), std::sin(ang));
+        b[k] = std::complex<double>(t[k].x, t[k].y);   // conj(a_k) of SIGN -1
+        if (k) b[L - k] = b[k];
+    }
+    // forward FFT on the host: radix-2, decimation in time
+    for (int i = 1, j = 0; i < L; ++i) {
+        int bit = L >> 1;
+        for (; j & bit; bit >>= 1) j ^= bit;
+        j ^= bit;
+        if (i < j) std::swap(b[i], b[j]);
+    }
+    std::vector<std::complex<double>> w(L / 2);
+    for (int q = 0; q < L / 2; ++q) w[q] = std::polar(1.0, -2.0 * M_PI * q / L);
+    for (int len = 2; len <= L; len *= 2)
+        for (int i = 0; i < L; i += len)
+            for (int k = 0; k < len / 2; ++k) {
+                const std::complex<double> p = b[i + k], q = b[i + k + len / 2] * w[k * (L / len)];
+                b[i + k] = p + q;
+                b[i + k + len / 2] = p - q;
+            }
+    for (int m = 0; m < L; ++m) t[n + m] = make_double2(b[m].real() / L, b[m].imag() / L);
+    u.chirp.alloc(sizeof(double2) * t.size());
+    LC_HIP(hipMemcpyAsync(u.chirp.as(), t.data(), sizeof(double2) * t.size(), hipMemcpyHostToDevice, c.stream()));
+    c.sync();
+}
+
 void nufft2d_init(Ctx &c, Geom2D &g) {
     Nufft2D &u = g.nu;
     u.cs.alloc(sizeof(double2) * g.nang);
@@ -786,7 +883,9 @@ void nufft2d_init(Ctx &c, Geom2D &g) {
     LC_HIP(hipMemcpyAsync(u.corr.as(), corr.data(), sizeof(float) * N, hipMemcpyHostToDevice, c.stream()));
     c.sync();
     LC_REQUIRE(fft_make_plan(u.nf, u.plan_nf), "nufft: fine grid size not 2^p 3^q");
-    u.det_fast = fft_make_plan((int)g.nrad, u.plan_det);
+    u.det_fast = g.nrad <= DET_FFT_MAX && fft_make_plan((int)g.nrad, u.plan_det);
+    u.det_blue = !u.det_fast && 2 * g.nrad - 1 <= DET_FFT_MAX;
+    if (u.det_blue) det_blue_init(c, u, (int)g.nrad);
     u.ready = true;
 }
 
@@ -822,9 +921,33 @@ SpreadGeom spread_geom(const Geom2D &g) {
 void det_transform(Ctx &c, const Geom2D &g, int sign, const float *real_in, const float2 *cplx_in,
                    float2 *cplx_out, float *real_out, int ns) {
     const int n = (int)g.nrad, nang = (int)g.nang, nrows = ns * nang;
-    const float2 *tw = c.twiddles<float>(n);
     const float scale = 1.0f / (float)n;
-    if (g.nu.det_fast && n <= NU_NT * NU_ME) {
+    static_assert(DET_FFT_MAX == NU_NT * NU_ME, "a detector line fits a block");
+    if (g.nu.det_blue) {
+        const int L = g.nu.plan_det.L, nl = std::max(1, std::min(DET_FFT_MAX / L, 64));
+        const double2 *tw = c.twiddles<double>(L), *chirp = g.nu.chirp.as<double2>();
+        const size_t sh = sizeof(double2) * lds_round(nl * L);
+        const dim3 grid(ceil_div(nang, nl), ns);
+        auto launch = [&](auto len) {
+            constexpr int LC = decltype(len)::value;
+            if (sign < 0)
+                hipLaunchKernelGGL((k_det_blue<-1, NU_NT, NU_ME, LC>), grid, dim3(NU_NT), sh, c.stream(), real_in,
+                                   cplx_in, cplx_out, real_out, nang, n, nl, g.nu.plan_det, tw, chirp, chirp + n,
+                                   scale);
+            else
+                hipLaunchKernelGGL((k_det_blue<1, NU_NT, NU_ME, LC>), grid, dim3(NU_NT), sh, c.stream(), real_in,
+                                   cplx_in, cplx_out, real_out, nang, n, nl, g.nu.plan_det, tw, chirp, chirp + n,
+                                   scale);
+        };
+        switch (L) {   // the lengths of common widths compiled, the rest by their plan
+        case 256: launch(std::integral_constant<int, 256>{}); break;
+        case 512: launch(std::integral_constant<int, 512>{}); break;
+        case 1024: launch(std::integral_constant<int, 1024>{}); break;
+        case 2048: launch(std::integral_constant<int, 2048>{}); break;
+        default: launch(std::integral_constant<int, 0>{});
+        }
+    } else if (g.nu.det_fast) {
+        const float2 *tw = c.twiddles<float>(n);
         const int nl = std::max(1, std::min(NU_NT * NU_ME / n, 64));
         const size_t sh = sizeof(float2) * lds_round(nl * n);
         const dim3 grid(ceil_div(nang, nl), ns);
@@ -839,6 +962,7 @@ void det_transform(Ctx &c, const Geom2D &g, int sign, const float *real_in, cons
         };
         if (!with_ct_len(n, launch)) launch(std::integral_constant<int, 0>{});
     } else {
+        const float2 *tw = c.twiddles<float>(n);
         dim3 grid(nrows);
         if (sign < 0)
             hipLaunchKernelGGL(k_det_dft<-1>, grid, dim3(128), 0, c.stream(), real_in, cplx_in,

@@ -74,6 +74,27 @@ def test_backproj2d_matches_oracle(lc, orc64, N, nang, nrad, ns, span):
     assert err < PROJ_TOL
 
 
+# detector widths that are not 2^p 3^q: the smallest, ones whose transform
+# length is compiled (256 .. 2048: several rows per block, a partial last
+# block, one row per two blocks) and ones around 1024 / 2048, where it changes
+@pytest.mark.parametrize("nrad,nang", [(5, 7), (95, 33), (130, 17), (511, 9), (1021, 5), (1025, 4), (2047, 3),
+                                       (2051, 2)])
+def test_detector_widths_match_oracle(lc, orc64, nrad, nang):
+    # both directions against the FP64 oracle; the projectors' own FP32 error is
+    # about 5e-7, so a wrong detector bin or phase (1 / nrad of the energy or
+    # more) shows.  A slice is the same alone and in a stack.
+    announce(f"detector widths nrad={nrad}")
+    rng = np.random.default_rng(nrad)
+    N = 24
+    th = uniform_theta(nang)
+    g = lc.PolarGrid2D(th, nrad)
+    x, y = rng.random((2, N, N)), rng.standard_normal((2, nang, nrad))
+    assert rel_l2(lc.forward2d(x, g), orc64.forward2d(x, th, nrad, tol=1e-12)) < 5e-6
+    b = lc.backproj2d(y, g, (2, N, N))
+    assert rel_l2(b, orc64.backproj2d(y, th, N, tol=1e-12)) < 5e-6
+    assert np.array_equal(lc.backproj2d(y[1:], g, (1, N, N)), b[1:])
+
+
 @pytest.mark.parametrize("N,nang,nrad", [(64, 50, 64), (96, 120, 128), (512, 360, 512)])
 def test_projectors_adjoint(lc, N, nang, nrad):
     # even nrad: fftshift == ifftshift, so backproj2d is the adjoint of forward2d
