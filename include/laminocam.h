@@ -428,8 +428,9 @@ int lc_get_tuning2d(lc_ctx ctx, int64_t image_n, int32_t *variant);
 /* ---- 3-D NUFFT spread bin shapes per grid (no reference counterpart) ----
  * The type-1 spread of lc_backproj3d sorts the points into bins of footprint
  * corners; the library is compiled for several bin shapes (shape 0, at most
- * 9 x 9 x 9 corner cells along z, y, x, is the default; 1 is 9 x 25 x 9, 2 is
- * 9 x 41 x 9).
+ * 9 x 9 x 9 corner cells along z, y, x, is the default; 1 is 9 x 25 x 9; 2 is
+ * the default's with dense bins shared out among more waves from 512 points
+ * instead of 2048).
  * lc_autotune3d times a back-projection of g's grid with each shape,
  * installs the fastest in the context for g's fine-grid shape (the volume's
  * dims, oversampled) and returns it, with the time of one back-projection in

@@ -48,15 +48,24 @@ __device__ __forceinline__ float es3(float z, float beta) {
     return s > 0.0f ? __expf(beta * (__builtin_amdgcn_sqrtf(s) - 1.0f)) : 0.0f;
 }
 
+// a modulo n for a in [-n, 2 n)
 __device__ __forceinline__ int wrapi(int a, int n) {
-    a %= n;
-    return a < 0 ? a + n : a;
+    a += a < 0 ? n : 0;
+    return a - (a >= n ? n : 0);
+}
+
+// a / b for inv = 1.0 / b: the FP64 product is within one of the quotient
+__device__ __forceinline__ unsigned div_by(unsigned a, unsigned b, double inv) {
+    const unsigned q = (unsigned)((double)a * inv);
+    const int r = (int)(a - q * b);
+    return r < 0 ? q - 1 : r >= (int)b ? q + 1 : q;
 }
 
 struct Grid3 {
     int nproj, nrows, ncols;
     int nf[3];          // fine grid (z, y, x)
     double dX, dY;      // lattice steps 2 pi / ncols, 2 pi / nrows
+    double icols, irows;   // 1 / ncols, 1 / nrows
     float beta;
     int mask;           // 1: drop points with any |coordinate| > pi
 };
@@ -92,8 +101,10 @@ constexpr int BE = RGN - W3 + 1;            // most corner cells of a bin along 
 
 // A compiled region shape: ROWS region rows along y (bins of ROWS - W3 + 1
 // corner rows).  More rows mean fewer bins, whose regions overlap less.
-template <int ROWS_> struct Shape3 {
+// A bin of more than HEAVY points is spread by several teams of waves.
+template <int ROWS_, unsigned HEAVY_ = 2048> struct Shape3 {
     static constexpr int ROWS = ROWS_;
+    static constexpr unsigned HEAVY = HEAVY_;
     static constexpr int EY = ROWS - W3 + 1;
     static constexpr int YB = EY <= 16 ? 4 : EY <= 32 ? 5 : 6;   // key bits of the corner row
     static constexpr int TEAMS = ROWS <= 16 ? 4 : 3;             // teams of a heavy bin (their tables fill the LDS)
@@ -105,7 +116,7 @@ constexpr int N_SHAPES3 = 3;
 template <typename F> void with_shape3(int i, F &&f) {
     switch (i) {
     case 1: f(Shape3<32>{}); break;
-    case 2: f(Shape3<48>{}); break;
+    case 2: f(Shape3<16, 512>{}); break;
     default: f(Shape3<16>{}); break;
     }
 }
@@ -123,7 +134,9 @@ __device__ __forceinline__ int bin_first(int i, int nf, int nb) { return (int)((
 // the bin of corner l: the largest i with bin_first(i) <= l
 __device__ __forceinline__ int bin_of(int l, int nf, int nb) { return (int)(((int64_t)(l + 1) * nb - 1) / nf); }
 
-// fine-grid position g, footprint corner l (unwrapped) of point (p, j, k)
+// fine-grid position g, footprint corner l (unwrapped) of point (p, j, k).
+// The columns of a rotation are orthonormal, so a coordinate is at most
+// sqrt(2) pi in size and a corner lies in [-nf, 2 nf).
 struct Corner3 {
     double gz, gy, gx;
     int lz, ly, lx;
@@ -144,9 +157,9 @@ __device__ __forceinline__ Corner3 corner3(const double *rot, int p, int j, int 
     return c;
 }
 __device__ __forceinline__ Corner3 corner3(const double *rot, unsigned pt, const Grid3 &g) {
-    const unsigned pj = pt / (unsigned)g.ncols;
+    const unsigned pj = div_by(pt, (unsigned)g.ncols, g.icols);
     const int k = (int)(pt - pj * (unsigned)g.ncols);
-    const int p = (int)(pj / (unsigned)g.nrows), j = (int)(pj - (unsigned)p * (unsigned)g.nrows);
+    const int p = (int)div_by(pj, (unsigned)g.nrows, g.irows), j = (int)(pj - (unsigned)p * (unsigned)g.nrows);
     return corner3(rot, p, j, k, g);
 }
 
@@ -241,10 +254,11 @@ __global__ void k_phase_shift3d(float2 *__restrict__ C, const double *__restrict
 // (twice the vector FMA rate, with no LDS access per cell) more than pays for.
 // Weights are computed once per point into LDS tables of BATCH points.
 // Measured: interpolating 23.1 M points (360 x 89 x 721 on 29 x 721^2) takes
-// 3.9 ms against 22.0 ms with a wave per point reading its 512 cells through
-// L1; spreading 47 M points (720 x 128 x 511 on 32 x 511^2) 7.5 ms against 13.5
+// 3.7 ms against 22.0 ms with a wave per point reading its 512 cells through
+// L1; spreading 47 M points (720 x 128 x 511 on 32 x 511^2) 6.8 ms against 13.5
 // ms with a wave per bin adding each point's cells to an LDS copy of a 4 x 4 x
-// 8 bin's region, and 2.9 M points (8 x 256^2) 1.28 against 2.61 ms.
+// 8 bin's region, and 2.9 M points (8 x 256^2) 1.15 against 2.61 ms.  Four waves
+// per SIMD (128 registers) matter: with three the spread takes 20% longer.
 // ---------------------------------------------------------------------------
 using f32x4 = __attribute__((ext_vector_type(4))) float;
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
@@ -252,8 +266,9 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
 }
 constexpr int BATCH = 128;                  // points per table; two threads fill a point's slots
 
-// footprint corner of a point relative to its bin, and the offset of its first
-// cell from the point (the weights' argument), per axis
+// footprint corner of a point relative to its bin, and the offset of its cell
+// W3 / 2 from the point, in [0, 1), per axis (the weights' arguments are exact
+// integers away from it: the largest weights get the smallest rounding)
 struct Foot {
     int t[3];
     float f[3];
@@ -264,9 +279,9 @@ __device__ __forceinline__ Foot foot3(const double *rot, unsigned pt, const Grid
     q.t[0] = wrapi(c.lz, g.nf[0]) - s[0];
     q.t[1] = wrapi(c.ly, g.nf[1]) - s[1];
     q.t[2] = wrapi(c.lx, g.nf[2]) - s[2];
-    q.f[0] = (float)((double)c.lz - c.gz);
-    q.f[1] = (float)((double)c.ly - c.gy);
-    q.f[2] = (float)((double)c.lx - c.gx);
+    q.f[0] = (float)((double)(c.lz + W3 / 2) - c.gz);
+    q.f[1] = (float)((double)(c.ly + W3 / 2) - c.gy);
+    q.f[2] = (float)((double)(c.lx + W3 / 2) - c.gx);
     return q;
 }
 
@@ -278,7 +293,7 @@ __device__ __forceinline__ void axis_weights(int t, float f, int h, float beta, 
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int r = 4 * h + i, d = (r - t) & (W3 - 1), slot = t + d;
-        const float w = es3(((float)d + f) * ihw, beta);
+        const float w = es3(((float)(d - W3 / 2) + f) * ihw, beta);
 #pragma unroll
         for (int s = 0; s < SLOTS; s += W3) put(r + s, r + s == slot ? w : 0.f);
     }
@@ -295,6 +310,13 @@ template <int G> __device__ __forceinline__ void group_rows(int ty, bool ok, int
         lo = min(lo, __shfl_xor(lo, o, 64));
         hi = max(hi, __shfl_xor(hi, o, 64));
     }
+}
+// v summed over its row of 16 lanes (every lane gets the sum)
+__device__ __forceinline__ float row_sum(float v) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, true));   // row_ror:1
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, true));
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true));
 }
 // first and last of wave w's rows (row w + 4 q -> q) that a group with corner
 // rows lo .. hi touches
@@ -347,18 +369,22 @@ k_interp3d(const float2 *__restrict__ F, float2 *__restrict__ C, const double *_
                 }
             }
         }
+        unsigned next = sval[min(a + p, e - 1)];   // this thread's point of the coming table
         for (; a < e; a += BATCH) {
             const int cnt = (int)min(e - a, (unsigned)BATCH);
             const bool ok = p < cnt;
-            const unsigned pt = sval[ok ? a + p : a];
-            const Foot ft = foot3(rot, pt, g, s);
-            float *zt = Zt + (p >> 4) * 256 + (p & 15), *yt = Yt + (p >> 4) * 256 + (p & 15), *xt = Xt + p * XS;
-            axis_weights<RGN>(ft.t[0], ft.f[0], h, g.beta, [&](int sl, float v) { zt[16 * sl] = v; });
-            axis_weights<RGN>(ft.t[1], ft.f[1], h, g.beta, [&](int sl, float v) { yt[16 * sl] = v; });
-            axis_weights<RGN>(ft.t[2], ft.f[2], h, g.beta, [&](int sl, float v) { xt[sl] = v; });
-            int lo, hi;
-            group_rows<16>(ft.t[1], ok, lo, hi);
-            if ((threadIdx.x & 15) == 0 && h == 0) meta[p >> 4] = lo | hi << 8;
+            const unsigned pt = next;
+            next = sval[min(a + BATCH + p, e - 1)];
+            if ((p & 64) < cnt) {   // (a wave whose points all lie past the end has none to place)
+                const Foot ft = foot3(rot, pt, g, s);
+                float *zt = Zt + (p >> 4) * 256 + (p & 15), *yt = Yt + (p >> 4) * 256 + (p & 15), *xt = Xt + p * XS;
+                axis_weights<RGN>(ft.t[0], ft.f[0], h, g.beta, [&](int sl, float v) { zt[16 * sl] = v; });
+                axis_weights<RGN>(ft.t[1], ft.f[1], h, g.beta, [&](int sl, float v) { yt[16 * sl] = v; });
+                axis_weights<RGN>(ft.t[2], ft.f[2], h, g.beta, [&](int sl, float v) { xt[sl] = v; });
+                int lo, hi;
+                group_rows<16>(ft.t[1], ok, lo, hi);
+                if ((threadIdx.x & 15) == 0 && h == 0) meta[p >> 4] = lo | hi << 8;
+            }
             __syncthreads();
             const int ng = (cnt + 15) >> 4;
             const int mt = meta[lane & 7];
@@ -368,7 +394,10 @@ k_interp3d(const float2 *__restrict__ F, float2 *__restrict__ C, const double *_
                 float zw[4];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) zw[j] = Zt[gr * 256 + (4 * j + k4) * 16 + n];
-                f32x4 ar = {0.f, 0.f, 0.f, 0.f}, ai = {0.f, 0.f, 0.f, 0.f};
+                // even and odd rows apart: each matrix instruction is a chain
+                // of rounded FMAs, and shorter chains round less
+                f32x4 ar[2], ai[2];
+                ar[0] = ar[1] = ai[0] = ai[1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     if (q < q0 || q > q1) continue;
@@ -376,22 +405,19 @@ k_interp3d(const float2 *__restrict__ F, float2 *__restrict__ C, const double *_
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         const float av = zw[j] * wy;
-                        ar = mfma4(av, fr[q][j], ar);
-                        ai = mfma4(av, fi[q][j], ai);
+                        ar[q & 1] = mfma4(av, fr[q][j], ar[q & 1]);
+                        ai[q & 1] = mfma4(av, fi[q][j], ai[q & 1]);
                     }
                 }
+                ar[0] += ar[1];
+                ai[0] += ai[1];
                 // register q: point 4 k4 + q, x = n; summed over x in the 16 lanes
                 const float *xw = Xt + (gr * 16 + 4 * k4) * XS + n;
                 float2 o = make_float2(0.f, 0.f);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const float wx = xw[q * XS];
-                    float vr = ar[q] * wx, vi = ai[q] * wx;
-#pragma unroll
-                    for (int d = 1; d < 16; d <<= 1) {
-                        vr += __shfl_xor(vr, d, 64);
-                        vi += __shfl_xor(vi, d, 64);
-                    }
+                    const float vr = row_sum(ar[0][q] * wx), vi = row_sum(ai[0][q] * wx);
                     if (n == q) o = make_float2(vr, vi);
                 }
                 if (n < 4) part[w][gr * 16 + 4 * k4 + n] = o;
@@ -406,10 +432,9 @@ k_interp3d(const float2 *__restrict__ F, float2 *__restrict__ C, const double *_
     }
 }
 
-// Bins of more than B3_HEAVY points are spread by S::TEAMS teams of four
+// Bins of more than S::HEAVY points are spread by S::TEAMS teams of four
 // waves, each taking a consecutive part of the bin's points; their sums are
 // added in team order.  Whether a bin is heavy depends only on its own count.
-constexpr unsigned B3_HEAVY = 2048;
 
 // LDS of one team: tables [point][slot] of wz, c wx (re, im) and wy (its rows
 // reordered to [wave][row / 4]), the row strides padded against bank conflicts,
@@ -440,9 +465,11 @@ __device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2
     const int p = threadIdx.x & (BATCH - 1), h = (threadIdx.x >> 7) & 1;
     const int n = lane & 15, k4 = lane >> 4;
     SpreadLds<S> &L = lds[team];
-    f32x4 ar[NQ], ai[NQ];
+    // sums over the batches so far (tr, ti) and within one: two levels keep the
+    // chains of rounded additions short where a bin holds thousands of points
+    f32x4 tr[NQ], ti[NQ];
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) ar[q] = ai[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int q = 0; q < NQ; ++q) tr[q] = ti[q] = f32x4{0.f, 0.f, 0.f, 0.f};
     // team t takes the t-th part of the bin's points, in order; every team
     // runs the same number of batches
     const unsigned per = ((s1 - s0 + TEAMS - 1) / TEAMS + BATCH - 1) / BATCH * BATCH;
@@ -459,7 +486,7 @@ __device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2
         const unsigned base = ws + (unsigned)it * BATCH;
         const int cnt = base < we ? (int)min(we - base, (unsigned)BATCH) : 0;
         const bool ok = p < cnt;
-        {
+        if ((p & 64) < cnt) {   // (a wave whose points all lie past the end has none to place)
             const Foot ft = foot3(rot, pt, g, s);
             float *zt = L.z + p * ZS, *xr = L.xr + p * ZS, *xi = L.xi + p * ZS, *yt = L.y + p * YS;
             const float cr = ok ? cv.x : 0.f, ci = ok ? cv.y : 0.f;
@@ -483,21 +510,39 @@ __device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2
         const int ng = (cnt + 3) >> 2;
         const float *zl = L.z + k4 * ZS + n, *xrl = L.xr + k4 * ZS + n, *xil = L.xi + k4 * ZS + n;
         const float *yl = L.y + k4 * YS + w * NQ;
+        f32x4 ar[NQ], ai[NQ];
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) ar[q] = ai[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // the next group's operands are read during this one's products
+        float zw = zl[0], br = xrl[0], bi = xil[0];
+        f32x4 wy[NQ / 4];
+#pragma unroll
+        for (int q = 0; q < NQ / 4; ++q) wy[q] = *reinterpret_cast<const f32x4 *>(yl + 4 * q);
         for (int gr = 0; gr < ng; ++gr) {
+            const int gn = min(gr + 1, BATCH / 4 - 1);
+            const float zn = zl[gn * 4 * ZS], brn = xrl[gn * 4 * ZS], bnx = xil[gn * 4 * ZS];
+            f32x4 wyn[NQ / 4];
+#pragma unroll
+            for (int q = 0; q < NQ / 4; ++q) wyn[q] = *reinterpret_cast<const f32x4 *>(yl + gn * 4 * YS + 4 * q);
             const int m = __builtin_amdgcn_readlane(mt, gr);
             const int q0 = first_row(m & 255, w), q1 = last_row(m >> 8, w);
-            const float zw = zl[gr * 4 * ZS], br = xrl[gr * 4 * ZS], bi = xil[gr * 4 * ZS];
-            float wy[NQ];
-#pragma unroll
-            for (int q = 0; q < NQ; q += 4)
-                *reinterpret_cast<float4 *>(wy + q) = *reinterpret_cast<const float4 *>(yl + gr * 4 * YS + q);
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
                 if (q < q0 || q > q1) continue;
-                const float av = zw * wy[q];
+                const float av = zw * wy[q / 4][q % 4];
                 ar[q] = mfma4(av, br, ar[q]);
                 ai[q] = mfma4(av, bi, ai[q]);
             }
+            zw = zn;
+            br = brn;
+            bi = bnx;
+#pragma unroll
+            for (int q = 0; q < NQ / 4; ++q) wy[q] = wyn[q];
+        }
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            tr[q] += ar[q];
+            ti[q] += ai[q];
         }
         __syncthreads();
     }
@@ -526,7 +571,7 @@ __device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2
             for (int i = 0; i < 4; ++i) {
                 bool in;
                 float2 *f = cell(q, i, in);
-                if (in) *f = make_float2(v[i].x + ar[q][i], v[i].y + ai[q][i]);
+                if (in) *f = make_float2(v[i].x + tr[q][i], v[i].y + ti[q][i]);
             }
         }
     } else {
@@ -535,8 +580,8 @@ __device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2
         f32x4 *ex = reinterpret_cast<f32x4 *>(lds);   // [team][wave][re, im][lane]
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
-            ex[((team * 4 + w) * 2) * 64 + lane] = ar[q];
-            ex[((team * 4 + w) * 2 + 1) * 64 + lane] = ai[q];
+            ex[((team * 4 + w) * 2) * 64 + lane] = tr[q];
+            ex[((team * 4 + w) * 2 + 1) * 64 + lane] = ti[q];
             __syncthreads();
             if (q % TEAMS == team) {
                 f32x4 sr = ex[(w * 2) * 64 + lane], si = ex[(w * 2 + 1) * 64 + lane];
@@ -561,13 +606,13 @@ __device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2
 
 // one block per light bin of this phase (order: the phase's bins, fullest first)
 template <typename S>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, S::ROWS <= 16 ? 4 : 1)
 k_spread3d_bin(const float2 *__restrict__ C, float2 *__restrict__ F, const double *__restrict__ rot,
                const unsigned *__restrict__ sval, const unsigned *__restrict__ bstart,
                const unsigned *__restrict__ bend, const unsigned *__restrict__ order, Grid3 g, Bins3 bn) {
     const int bin = __builtin_amdgcn_readfirstlane(order[blockIdx.x]);
     const unsigned s0 = bstart[bin], s1 = bend[bin];
-    if (s0 >= s1 || s1 - s0 > B3_HEAVY) return;   // empty, or a heavy bin
+    if (s0 >= s1 || s1 - s0 > S::HEAVY) return;   // empty, or a heavy bin
     spread3_bin<S, 1>(C, F, rot, sval, bin, s0, s1, g, bn, reinterpret_cast<SpreadLds<S> *>(lc_smem));
 }
 
@@ -582,7 +627,7 @@ k_spread3d_bin_heavy(const float2 *__restrict__ C, float2 *__restrict__ F, const
     for (unsigned j = blockIdx.x; j < nphase; j += gridDim.x) {
         const int bin = __builtin_amdgcn_readfirstlane(order[j]);
         const unsigned s0 = bstart[bin], s1 = bend[bin];
-        if (s1 - s0 <= B3_HEAVY) break;   // the order is fullest first: the rest are light
+        if (s1 - s0 <= S::HEAVY) break;   // the order is fullest first: the rest are light
         spread3_bin<S, S::TEAMS>(C, F, rot, sval, bin, s0, s1, g, bn, reinterpret_cast<SpreadLds<S> *>(lc_smem));
     }
 }
@@ -932,6 +977,8 @@ Grid3 grid3(const Geom3D &g, bool mask) {
     for (int a = 0; a < 3; ++a) r.nf[a] = g.nu.nf[a];
     r.dX = 2.0 * M_PI / (double)g.ncols;
     r.dY = 2.0 * M_PI / (double)g.nrows;
+    r.icols = 1.0 / (double)g.ncols;
+    r.irows = 1.0 / (double)g.nrows;
     r.beta = (float)g.nu.beta;
     r.mask = mask ? 1 : 0;
     return r;
