@@ -21,6 +21,11 @@ struct Nufft2D {
     FftPlan plan_nf{};    // fine-grid FFT
     FftPlan plan_det{};   // detector FFT (det_fast: of the width; det_blue: Bluestein length)
     bool det_fast = false, det_blue = false;
+    // the points of a slice sorted by corner bin (unsigned[nang * nrad], then
+    // int[bins + 1] starts) and the spread's tiles, fullest first, per tile
+    // shape: ntiles of them from tiles_off, the first nheavy heavy
+    DBuf points, tiles;
+    int tiles_off[2] = {0, 0}, ntiles[2] = {0, 0}, nheavy[2] = {0, 0};
     DBuf chirp;           // det_blue: double2 chirp[nrad], then its spectrum [plan_det.L]
     bool ready = false;
 };
@@ -249,7 +254,6 @@ int nufft3d_autotune(Ctx &c, Geom3D &g, double *best_ms);
 // the same for the 2-D spread, per fine-grid size, timed on nslices slices
 int nufft2d_num_shapes();
 int nufft2d_autotune(Ctx &c, Geom2D &g, int nslices, double *best_ms);
-size_t nufft2d_spread_bytes(int64_t ns, int64_t npts, int nf);
 // An odd image size N needs column blocks of at least two columns (the block
 // copies move pairs of complex values).  A column shape too small for 2 M
 // values is replaced by the first shape that holds them (block width then

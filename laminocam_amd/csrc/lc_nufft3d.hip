@@ -269,31 +269,32 @@ constexpr int BATCH = 128;                  // points per table; two threads fil
 // footprint corner of a point relative to its bin, and the offset of its cell
 // W3 / 2 from the point, in [0, 1), per axis (the weights' arguments are exact
 // integers away from it: the largest weights get the smallest rounding)
-struct Foot {
+template <typename T> struct Foot {
     int t[3];
-    float f[3];
+    T f[3];
 };
-__device__ __forceinline__ Foot foot3(const double *rot, unsigned pt, const Grid3 &g, const int s[3]) {
+template <typename T>
+__device__ __forceinline__ Foot<T> foot3(const double *rot, unsigned pt, const Grid3 &g, const int s[3]) {
     const Corner3 c = corner3(rot, pt, g);
-    Foot q;
+    Foot<T> q;
     q.t[0] = wrapi(c.lz, g.nf[0]) - s[0];
     q.t[1] = wrapi(c.ly, g.nf[1]) - s[1];
     q.t[2] = wrapi(c.lx, g.nf[2]) - s[2];
-    q.f[0] = (float)((double)(c.lz + W3 / 2) - c.gz);
-    q.f[1] = (float)((double)(c.ly + W3 / 2) - c.gy);
-    q.f[2] = (float)((double)(c.lx + W3 / 2) - c.gx);
+    q.f[0] = (T)((double)(c.lz + W3 / 2) - c.gz);
+    q.f[1] = (T)((double)(c.ly + W3 / 2) - c.gy);
+    q.f[2] = (T)((double)(c.lx + W3 / 2) - c.gx);
     return q;
 }
 
 // the slots congruent to 4 h .. 4 h + 3 modulo 8 of one axis's `slots` slots:
 // put(slot, weight), where one slot of each residue lies in the footprint
-template <int SLOTS, typename F>
-__device__ __forceinline__ void axis_weights(int t, float f, int h, float beta, F &&put) {
+template <int SLOTS, typename T, typename F>
+__device__ __forceinline__ void axis_weights(int t, T f, int h, float beta, F &&put) {
     const float ihw = 1.0f / (0.5f * W3);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int r = 4 * h + i, d = (r - t) & (W3 - 1), slot = t + d;
-        const float w = es3(((float)(d - W3 / 2) + f) * ihw, beta);
+        const float w = es3((float)((T)(d - W3 / 2) + f) * ihw, beta);
 #pragma unroll
         for (int s = 0; s < SLOTS; s += W3) put(r + s, r + s == slot ? w : 0.f);
     }
@@ -376,7 +377,7 @@ k_interp3d(const float2 *__restrict__ F, float2 *__restrict__ C, const double *_
             const unsigned pt = next;
             next = sval[min(a + BATCH + p, e - 1)];
             if ((p & 64) < cnt) {   // (a wave whose points all lie past the end has none to place)
-                const Foot ft = foot3(rot, pt, g, s);
+                const Foot<double> ft = foot3<double>(rot, pt, g, s);
                 float *zt = Zt + (p >> 4) * 256 + (p & 15), *yt = Yt + (p >> 4) * 256 + (p & 15), *xt = Xt + p * XS;
                 axis_weights<RGN>(ft.t[0], ft.f[0], h, g.beta, [&](int sl, float v) { zt[16 * sl] = v; });
                 axis_weights<RGN>(ft.t[1], ft.f[1], h, g.beta, [&](int sl, float v) { yt[16 * sl] = v; });
@@ -487,7 +488,7 @@ __device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2
         const int cnt = base < we ? (int)min(we - base, (unsigned)BATCH) : 0;
         const bool ok = p < cnt;
         if ((p & 64) < cnt) {   // (a wave whose points all lie past the end has none to place)
-            const Foot ft = foot3(rot, pt, g, s);
+            const Foot<float> ft = foot3<float>(rot, pt, g, s);
             float *zt = L.z + p * ZS, *xr = L.xr + p * ZS, *xi = L.xi + p * ZS, *yt = L.y + p * YS;
             const float cr = ok ? cv.x : 0.f, ci = ok ? cv.y : 0.f;
             // past the last point every product is 0 x a stored weight

@@ -141,6 +141,34 @@ def test_sysmat_nufft_matches_oracle_and_toeplitz(lc, orc64, N, nang, ns):
     assert rel_l2(y1, y2) < PROJ_TOL
 
 
+# fine grids of 16 cells (one tile, wrapped onto itself), 27 and 81 (partial
+# tiles and bins), 54 and 162, and 96 with over 512 points in its central tiles;
+# stacks of 1 to 7 slices share weights by 4, 2 and 1
+@pytest.mark.parametrize("N,nang,nrad,ns", [(8, 11, 9, 3), (13, 20, 16, 7), (27, 30, 40, 2), (41, 25, 37, 1),
+                                            (81, 40, 64, 6), (48, 333, 50, 5)])
+def test_projectors_tile_edges_match_oracle(lc, orc64, N, nang, nrad, ns):
+    announce(f"projector tile edges N={N} nang={nang} nrad={nrad} ns={ns}")
+    rng = np.random.default_rng(N * 5 + ns)
+    th = uniform_theta(nang, 2 * np.pi)
+    sino, vol = rng.standard_normal((ns, nang, nrad)).astype(np.float32), rng.random((ns, N, N))
+    xr = orc64.backproj2d(sino, th, N, tol=1e-12)
+    g = lc.PolarGrid2D(th, nrad)
+    assert rel_l2(lc.forward2d(vol, g), orc64.forward2d(vol, th, nrad, tol=1e-12)) < PROJ_TOL
+    ctx = lc.Context(0)
+    try:
+        psf = lc.PointSpreadFunction2D(g, N, ctx=ctx)
+        for shape in range(2):
+            ctx.set_tuning2d_nufft(psf, shape)
+            x = lc.backproj2d(sino, g, (ns, N, N), ctx=ctx)
+            err = rel_l2(x, xr)
+            print(f"shape {shape}: rel_l2 = {err:.3e}")
+            assert err < PROJ_TOL
+            for i in range(ns):
+                assert np.array_equal(lc.backproj2d(sino[i:i + 1], g, (1, N, N), ctx=ctx), x[i:i + 1])
+    finally:
+        ctx.close()
+
+
 def test_backproj2d_bin_shapes_and_autotune(lc, orc64):
     # both compiled bin sizes of the sorted-bin spread (16 and 32 corner
     # cells) give the oracle's back-projection; a slice is the same alone and
