@@ -34,6 +34,13 @@ namespace lc {
 // loads of each vector per thread)
 constexpr int CG_UPD_NT = 512;
 
+// outer Split-Bregman iterations per residual formed from A x (see sb_outer_t).
+// Over 15 solves of 4 to 30 outer iterations the error against 64 bits is that
+// of forming it every time (ratio 1.00) with 2, 1.06 with 3, 1.14 with 5; a 3-D
+// solve of 12 outer iterations on 13 x 145^2 takes 3.96 ms formed every time (by
+// the kernels before these), 2.32 with 2, 2.15 with 3, 2.05 with 5.
+constexpr int SB_REFRESH = 2;
+
 // CG iterations per replay of a batch's cached iteration graph
 constexpr int CG_GRAPH_ITERS = 8;
 
@@ -256,7 +263,7 @@ __global__ void k_cg_fin2(const ProbDev *__restrict__ pd, CgState *st, const dou
 }
 
 // ----------------------------------------------------------------------------
-// finite differences (per element of a problem's n1 x N x N stack)
+// finite differences per element, for the standalone operators
 // ----------------------------------------------------------------------------
 struct Idx3 {
     int s, a, b, n1, n2, n3;
@@ -351,33 +358,147 @@ __device__ __forceinline__ R lap_at(const A &u, const Idx3 &q, int boundary) {
     return acc;
 }
 
-// (s, a, b) of the element at global offset i of a problem (one 64-bit
-// division pair per thread); step() advances it by NT elements
-__device__ __forceinline__ Idx3 idx_of(const ProbDev &d, int64_t i) {
-    const int64_t loc = i - d.off;
-    Idx3 q;
-    q.n2 = d.N;
-    q.n3 = d.N;
-    q.n1 = d.ns;
-    const int64_t nn = (int64_t)d.N * d.N;
-    q.s = (int)(loc / nn);
-    const int64_t rem = loc - (int64_t)q.s * nn;
-    q.a = (int)(rem / d.N);
-    q.b = (int)(rem - (int64_t)q.a * d.N);
+// ----------------------------------------------------------------------------
+// finite differences in the solver: four consecutive elements of a problem's
+// n1 x N x N stack per thread.  Row ends fall anywhere in a group of four when
+// N is odd (padded sizes always are), so neighbours are read as unaligned
+// four-wide loads at the flat offsets +-1, +-2, +-N, ... and every element
+// keeps or drops its own.  One position per group (an FP64 reciprocal each for
+// the slice and the row in place of 64-bit divisions and a walk along rows) and
+// wide loads in place of one element, its indices and its 4-byte loads per
+// thread, which kept the vector ALU busier than the memory:
+// batch of 64 slices (16.9 M elements): Laplacian 108 -> 57 us, shrink 221 -> 134
+// us, right-hand side 160 us and the residual after it 77 us -> 142 us for both.
+// ----------------------------------------------------------------------------
+template <typename R> using ua4 = R __attribute__((ext_vector_type(4), aligned(sizeof(R))));
+
+struct Quad {
+    int s[4], a[4], b[4];   // the elements' slice, row, column
+};
+// positions of the four elements from offset loc of a problem (inn = 1 / N^2, iN = 1 / N)
+__device__ __forceinline__ Quad quad_of(int64_t loc, int N, double inn, double iN) {
+    const int nn = N * N;
+    int s = (int)((double)loc * inn);
+    int rem = (int)(loc - (int64_t)s * nn);   // within one of the quotient
+    const int ds = rem < 0 ? -1 : rem >= nn ? 1 : 0;
+    s += ds;
+    rem -= ds * nn;
+    int a = (int)((double)rem * iN), b = rem - a * N;
+    const int da = b < 0 ? -1 : b >= N ? 1 : 0;
+    a += da;
+    b -= da * N;
+    Quad q;
+    if (N < 4) {   // a group may cross more than one row end
+        for (int e = 0; e < 4; ++e) {
+            const int64_t l = loc + e;
+            q.s[e] = (int)(l / nn);
+            const int m = (int)(l - (int64_t)q.s[e] * nn);
+            q.a[e] = m / N;
+            q.b[e] = m - q.a[e] * N;
+        }
+        return q;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const bool w = b + e >= N;
+        const int ae = a + w;
+        const bool w2 = ae >= N;
+        q.b[e] = b + e - (w ? N : 0);
+        q.a[e] = w2 ? 0 : ae;
+        q.s[e] = s + w2;
+    }
     return q;
 }
-__device__ __forceinline__ void step(Idx3 &q, int n) {
-    q.b += n;
-    while (q.b >= q.n3) {
-        q.b -= q.n3;
-        if (++q.a >= q.n2) {
-            q.a = 0;
-            ++q.s;
+
+// four values of u from offset i, where [lo, hi) may be read; need: some
+// element's neighbour lies there (others' values are dropped by the caller)
+template <typename R>
+__device__ __forceinline__ ua4<R> load4(const R *__restrict__ u, int64_t i, int64_t lo, int64_t hi, bool need) {
+    ua4<R> v = {(R)0, (R)0, (R)0, (R)0};
+    if (!need) return v;
+    if (i >= lo && i + 4 <= hi) return *reinterpret_cast<const ua4<R> *>(u + i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (i + e >= lo && i + e < hi) v[e] = u[i + e];
+    return v;
+}
+// four streamed values from a group's own offset (16-byte aligned), cnt of them present
+template <typename R> __device__ __forceinline__ ua4<R> own4(const R *__restrict__ u, int64_t i, int cnt) {
+    if (cnt == 4) {
+        const vec4<R> t = ld_stream(reinterpret_cast<const vec4<R> *>(u + i));
+        return ua4<R>{t.x, t.y, t.z, t.w};
+    }
+    ua4<R> v = {(R)0, (R)0, (R)0, (R)0};
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (e < cnt) v[e] = u[i + e];
+    return v;
+}
+template <typename R> __device__ __forceinline__ void put4(R *__restrict__ u, int64_t i, int cnt, const ua4<R> &v) {
+    if (cnt == 4) {
+        st_stream(reinterpret_cast<vec4<R> *>(u + i), vmake4<vec4<R>>(v[0], v[1], v[2], v[3]));
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (e < cnt) u[i + e] = v[e];
+}
+
+// The neighbours of a group at distance D (1 or 2) along each axis; vol: the
+// stack has neighbouring slices.  col[e + D -+ D] are element e's along a row.
+template <typename R, int D> struct Near {
+    ua4<R> up[2], dn[2];   // [0] slices, [1] rows
+    R col[4 + 2 * D];
+};
+template <int D, typename R>
+__device__ __forceinline__ void near_load(Near<R, D> &w, const R *__restrict__ u, int64_t i, int64_t lo, int64_t hi,
+                                          const Quad &q, int n1, int N, bool vol, bool rows, bool cols) {
+    const int64_t nn = (int64_t)N * N;
+    if (vol) {
+        w.up[0] = load4(u, i + D * nn, lo, hi, q.s[0] + D < n1);
+        w.dn[0] = load4(u, i - D * nn, lo, hi, q.s[3] - D >= 0);
+    }
+    if (rows) {
+        w.up[1] = load4(u, i + (int64_t)D * N, lo, hi, true);
+        w.dn[1] = load4(u, i - (int64_t)D * N, lo, hi, true);
+    }
+    if (cols) {
+        const ua4<R> a = load4(u, i - D, lo, hi, true), b = load4(u, i + D, lo, hi, true);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            w.col[e] = a[e];
+            w.col[e + 2 * D] = b[e];
         }
     }
 }
 
-// Ap -= mu * lap(p); partial <p, Ap> (Split-Bregman operator, src/bregman.cpp:55)
+// neighbour at +D and -D of element e along axis c, 0 outside the stack
+template <typename R, int D>
+__device__ __forceinline__ void near_at(const Near<R, D> &w, const Quad &q, int e, int c, int n1, int N, R &up, R &dn,
+                                        bool &in1, bool &im1) {
+    const int v = c == 0 ? q.s[e] : c == 1 ? q.a[e] : q.b[e], n = c == 0 ? n1 : N;
+    in1 = v + 1 < n;
+    im1 = v >= 1;
+    up = v + D < n ? (c == 2 ? w.col[e + 2 * D] : w.up[c][e]) : (R)0;
+    dn = v >= D ? (c == 2 ? w.col[e] : w.dn[c][e]) : (R)0;
+}
+__device__ __forceinline__ bool interior4(const Quad &q, int e, int n1, int N) {
+    return q.s[e] >= 1 && q.s[e] + 1 < n1 && q.a[e] >= 1 && q.a[e] + 1 < N && q.b[e] >= 1 && q.b[e] + 1 < N;
+}
+
+// runs f(i, cnt, quad) over a chunk's groups of four
+template <int NT, typename F>
+__device__ __forceinline__ void for_quads(const ChunkRef &c, const ProbDev &d, F &&f) {
+    const double iN = 1.0 / (double)d.N, inn = iN * iN;
+    static_assert(CHUNK % (4 * NT) == 0, "a whole chunk is a whole number of groups per thread");
+    for (int64_t i = c.begin + 4 * threadIdx.x; i < c.end; i += 4 * NT)
+        f(i, (int)min((int64_t)4, c.end - i), quad_of(i - d.off, d.N, inn, iN));
+}
+
+// Ap -= mu * lap(p); partial <p, Ap> (Split-Bregman operator, src/bregman.cpp:55).
+// lap = div(grad): along an axis (G(v + 1) - G(v - 1)) / 2 with G(v) =
+// (p(v + 1) - p(v - 1)) / 2, p and G zero outside (boundary 1), or G and the
+// result zero off the interior (boundary 0)
 template <typename R, int NT>
 __global__ void __launch_bounds__(NT)
 k_sb_lapdot(const ChunkRef *__restrict__ ch, const ProbDev *__restrict__ pd,
@@ -386,41 +507,38 @@ k_sb_lapdot(const ChunkRef *__restrict__ ch, const ProbDev *__restrict__ pd,
     const ChunkRef c = ch[blockIdx.x];
     if (st && !st[c.prob].active) return;
     const ProbDev d = pd[c.prob];
-    const int64_t nn = (int64_t)d.N * d.N;
+    const bool vol = d.ns > 1;
+    const int64_t lo = d.off, hi = d.off + d.n;
     double acc = 0.0;
-    Idx3 q = idx_of(d, c.begin + threadIdx.x);
-    // UE elements per thread per step (i, i + NT, ...): the stencil loads of
-    // all of them are issued before any result is used, so a wave keeps UE
-    // elements' loads in flight instead of one; acc sums in the same order
-    constexpr int UE = 4;
-    auto run = [&](auto full) {
-        constexpr bool FULL = decltype(full)::value;
-        for (int64_t i0 = c.begin + threadIdx.x; i0 < c.end; i0 += UE * NT) {
-            R l[UE], a[UE], pv[UE];
+    for_quads<NT>(c, d, [&](int64_t i, int cnt, const Quad &q) {
+        Near<R, 2> w;
+        near_load<2>(w, p, i, lo, hi, q, d.ns, d.N, vol, true, true);
+        ua4<R> a = own4(ap, i, cnt);
 #pragma unroll
-            for (int u = 0; u < UE; ++u) {
-                const int64_t i = i0 + u * NT;
-                if (FULL || i < c.end) {
-                    l[u] = lap_at<R>(Rel<R>{p + i, nn, d.N}, q, d.boundary);
-                    a[u] = __builtin_nontemporal_load(ap + i);
-                    pv[u] = p[i];
-                }
-                step(q, NT);
-            }
+        for (int e = 0; e < 4; ++e) {
+            const R u0 = w.col[e + 2];
+            R l = (R)0;
 #pragma unroll
-            for (int u = 0; u < UE; ++u) {
-                const int64_t i = i0 + u * NT;
-                if (FULL || i < c.end) {
-                    const R v = a[u] - l[u] * (R)d.mu;
-                    __builtin_nontemporal_store(v, ap + i);
-                    acc += (double)pv[u] * v;
+            for (int k = 0; k < 3; ++k) {
+                if (k == 0 && !vol) continue;
+                R up, dn;
+                bool ip, im;
+                near_at(w, q, e, k, d.ns, d.N, up, dn, ip, im);
+                // boundary 0: q inside, so G(v + 1) counts when v + 2 does
+                if (d.boundary == 0) {
+                    const int v = k == 0 ? q.s[e] : k == 1 ? q.a[e] : q.b[e], n = k == 0 ? d.ns : d.N;
+                    ip = v + 2 < n;
+                    im = v >= 2;
                 }
+                const R gp = ip ? (R)0.5 * (up - u0) : (R)0, gm = im ? (R)0.5 * (u0 - dn) : (R)0;
+                l += (R)0.5 * (gp - gm);
             }
+            if (d.boundary == 0 && !interior4(q, e, d.ns, d.N)) l = (R)0;
+            a[e] -= l * (R)d.mu;
+            if (e < cnt) acc += (double)u0 * a[e];
         }
-    };
-    static_assert(CHUNK % (UE * NT) == 0, "a whole chunk is a whole number of steps");
-    if (c.end - c.begin == CHUNK) run(std::true_type{});
-    else run(std::false_type{});
+        put4(ap, i, cnt, a);
+    });
     if (dot) {
         __shared__ double sh[NT / 64];
         const double t = block_sum<NT>(acc, sh);
@@ -428,31 +546,77 @@ k_sb_lapdot(const ChunkRef *__restrict__ ch, const ProbDev *__restrict__ pd,
     }
 }
 
-// rhs = y0 - mu * div(d - b)   (src/bregman.cpp:58-61); d - b is formed at
-// each stencil point as it is read (component stride = total), rounded
-// exactly as a stored d - b would be
-template <typename R, int NT>
+// rhs = y0 - mu * div(d - b)   (src/bregman.cpp:58-61); d - b is formed as it is
+// read (component stride = total), rounded exactly as a stored d - b would be.
+// A single slice has no neighbours along the first axis: its component 0 stays
+// zero and is not read.  RES: also r += rhs - (the rhs of the last outer
+// iteration), the residual of the new right-hand side at the current x, and
+// the partials <r, r>, <rhs, rhs>
+template <typename R, int NT, bool RES>
 __global__ void __launch_bounds__(NT)
 k_sb_rhs(const ChunkRef *__restrict__ ch, const ProbDev *__restrict__ pd,
          const SbState *__restrict__ sb, const R *__restrict__ y0, R *__restrict__ rhs,
-         const R *__restrict__ D, const R *__restrict__ Bv, int64_t total) {
+         const R *__restrict__ D, const R *__restrict__ Bv, R *__restrict__ r, double *__restrict__ cpart,
+         int64_t total) {
     const ChunkRef c = ch[blockIdx.x];
     if (!sb[c.prob].active) return;
     const ProbDev d = pd[c.prob];
-    const int64_t nn = (int64_t)d.N * d.N;
-    Idx3 q = idx_of(d, c.begin + threadIdx.x);
-    for (int64_t i = c.begin + threadIdx.x; i < c.end; i += NT, step(q, NT)) {
-        auto dmb = [&](int k, int ds, int da, int db) {
-            const int64_t o = k * total + i + ds * nn + (int64_t)(da * d.N + db);
-            return D[o] - Bv[o];
-        };
-        const R dv = div_gen<R>(dmb, q, d.boundary);
-        __builtin_nontemporal_store(__builtin_nontemporal_load(y0 + i) - dv * (R)d.mu, rhs + i);
+    const bool vol = d.ns > 1;
+    const int64_t lo = d.off, hi = d.off + d.n;
+    double rr = 0.0, yy = 0.0;
+    for_quads<NT>(c, d, [&](int64_t i, int cnt, const Quad &q) {
+        Near<R, 1> wd[3], wb[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            if (k == 0 && !vol) continue;
+            near_load<1>(wd[k], D + k * total, i, lo, hi, q, d.ns, d.N, k == 0, k == 1, k == 2);
+            near_load<1>(wb[k], Bv + k * total, i, lo, hi, q, d.ns, d.N, k == 0, k == 1, k == 2);
+        }
+        const ua4<R> y = own4(y0, i, cnt);
+        ua4<R> o, rv, t;
+        if constexpr (RES) {
+            o = own4(rhs, i, cnt);
+            rv = own4(r, i, cnt);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            R dv = (R)0;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                if (k == 0 && !vol) continue;
+                R du, dd, bu, bd;
+                bool ip, im;
+                near_at(wd[k], q, e, k, d.ns, d.N, du, dd, ip, im);
+                near_at(wb[k], q, e, k, d.ns, d.N, bu, bd, ip, im);
+                dv += (R)0.5 * ((du - bu) - (dd - bd));
+            }
+            if (d.boundary == 0 && !interior4(q, e, d.ns, d.N)) dv = (R)0;
+            t[e] = y[e] - dv * (R)d.mu;
+            if constexpr (RES) {
+                rv[e] += t[e] - o[e];
+                if (e < cnt) {
+                    rr += (double)rv[e] * rv[e];
+                    yy += (double)t[e] * t[e];
+                }
+            }
+        }
+        put4(rhs, i, cnt, t);
+        if constexpr (RES) put4(r, i, cnt, rv);
+    });
+    if constexpr (RES) {
+        __shared__ double sh[NT / 64];
+        const double a = block_sum<NT>(rr, sh);
+        const double b = block_sum<NT>(yy, sh);
+        if (threadIdx.x == 0) {
+            cpart[blockIdx.x * 4 + 0] = a;
+            cpart[blockIdx.x * 4 + 1] = b;
+        }
     }
 }
 
 // isotropic (or per-component) shrink and Bregman update
-// (src/bregman.cpp:64-84); partials ||x - x_old||^2, ||x_old||^2; x_old = x
+// (src/bregman.cpp:64-84); partials ||x - x_old||^2, ||x_old||^2; x_old = x.
+// A single slice's component 0 is zero before and after: it is left alone.
 template <typename R, int NT>
 __global__ void __launch_bounds__(NT)
 k_sb_shrink(const ChunkRef *__restrict__ ch, const ProbDev *__restrict__ pd,
@@ -463,42 +627,62 @@ k_sb_shrink(const ChunkRef *__restrict__ ch, const ProbDev *__restrict__ pd,
     const SbState S = sb[c.prob];
     if (!S.active) return;
     const ProbDev d = pd[c.prob];
-    const int64_t nn = (int64_t)d.N * d.N;
+    const bool vol = d.ns > 1;
+    const int64_t lo = d.off, hi = d.off + d.n;
     const R thr = (R)(S.lambda / S.mu);
     double dn = 0.0, on = 0.0;
-    Idx3 q = idx_of(d, c.begin + threadIdx.x);
-    for (int64_t i = c.begin + threadIdx.x; i < c.end; i += NT, step(q, NT)) {
-        const Rel<R> xr{x + i, nn, d.N};
-        // streaming (nontemporal) accesses for the fields only this
-        // element touches; x keeps ordinary loads (its neighbours are reread)
-        R g[3], v[3], bk[3];
+    for_quads<NT>(c, d, [&](int64_t i, int cnt, const Quad &q) {
+        Near<R, 1> w;
+        near_load<1>(w, x, i, lo, hi, q, d.ns, d.N, vol, true, true);
+        ua4<R> bk[3], dk[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            g[k] = grad_c<R>(xr, q, k, 0, 0, 0, d.boundary);
-            bk[k] = __builtin_nontemporal_load(Bv + k * total + i);
-            v[k] = g[k] + bk[k];
+            if (k == 0 && !vol) bk[k] = ua4<R>{(R)0, (R)0, (R)0, (R)0};
+            else bk[k] = own4(Bv + k * total, i, cnt);
         }
-        if (!aniso) {
-            const R sk = sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-            const R sh = fmax((R)0, sk - thr);
+        const ua4<R> xo = own4(xold, i, cnt);
+        ua4<R> xi;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            xi[e] = w.col[e + 1];
+            R g[3], v[3];
+            const bool in = d.boundary != 0 || interior4(q, e, d.ns, d.N);
+#pragma unroll
             for (int k = 0; k < 3; ++k) {
-                const R dk = sh * (v[k] / (sk + (R)1e-8));
-                __builtin_nontemporal_store(dk, D + k * total + i);
-                __builtin_nontemporal_store(bk[k] + (g[k] - dk), Bv + k * total + i);
+                g[k] = (R)0;
+                if (k != 0 || vol) {
+                    R up, dw;
+                    bool ip, im;
+                    near_at(w, q, e, k, d.ns, d.N, up, dw, ip, im);
+                    g[k] = in ? (R)0.5 * (up - dw) : (R)0;
+                }
+                v[k] = g[k] + bk[k][e];
             }
-        } else {
-            for (int k = 0; k < 3; ++k) {
-                const R sh = fmax((R)0, fabs(v[k]) - thr);
-                const R dk = copysign(sh, v[k]);
-                __builtin_nontemporal_store(dk, D + k * total + i);
-                __builtin_nontemporal_store(bk[k] + (g[k] - dk), Bv + k * total + i);
+            if (!aniso) {
+                const R sk = sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+                const R sh = fmax((R)0, sk - thr);
+#pragma unroll
+                for (int k = 0; k < 3; ++k) dk[k][e] = sh * (v[k] / (sk + (R)1e-8));
+            } else {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) dk[k][e] = copysign(fmax((R)0, fabs(v[k]) - thr), v[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < 3; ++k) bk[k][e] += g[k] - dk[k][e];
+            if (e < cnt) {
+                const R df = xi[e] - xo[e];
+                dn += (double)df * (double)df;
+                on += (double)xo[e] * xo[e];
             }
         }
-        const R xi = x[i], xo = __builtin_nontemporal_load(xold + i);
-        dn += (double)(xi - xo) * (double)(xi - xo);
-        on += (double)xo * xo;
-        __builtin_nontemporal_store(xi, xold + i);
-    }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            if (k == 0 && !vol) continue;
+            put4(D + k * total, i, cnt, dk[k]);
+            put4(Bv + k * total, i, cnt, bk[k]);
+        }
+        put4(xold, i, cnt, xi);
+    });
     __shared__ double sh[NT / 64];
     const double a = block_sum<NT>(dn, sh);
     const double b = block_sum<NT>(on, sh);
@@ -1091,21 +1275,40 @@ void Batch2D::cg(const std::vector<int> &max_iter, double tol, double xtol, bool
     c_.sync();
 }
 
-// one Split-Bregman outer iteration (src/bregman.cpp:58-88) for every active problem
+// one Split-Bregman outer iteration (src/bregman.cpp:58-88) for every active
+// problem.  The inner solve starts from the x of the last one under a new
+// right-hand side, and that solve left r = rhs_old - A x; so r + rhs - rhs_old
+// is its starting residual without an operator apply, half of an outer
+// iteration's at one inner iteration.  The first outer iteration and every
+// SB_REFRESH-th after it (`full`) form r = rhs - A x, so the roundings of the
+// updates do not add up; zero: x = 0, so r = rhs.
 template <typename R>
 void Batch2D::sb_outer_t(bool hsync, double tol, double xtol, int inner, const int *dmi,
-                         const std::vector<int> &mi) {
+                         const std::vector<int> &mi, bool full, bool zero) {
     const int np = nprob();
     const SbState *sbs = dsb_.as<SbState>();
-    // rhs = y0 - mu div(d - b)
-    hipLaunchKernelGGL((k_sb_rhs<R, 256>), dim3(nchunk_), dim3(256), 0, c_.stream(),
-                       dchunk_.as<ChunkRef>(), dprob_.as<ProbDev>(), sbs, Y0_.as<R>(), Y_.as<R>(),
-                       Dv_.as<R>(), Bv_.as<R>(), total_);
-    LC_HIP(hipGetLastError());
+    auto arm = [&] {
+        hipLaunchKernelGGL(k_cg_arm, dim3(ceil_div(np, 64)), dim3(64), 0, c_.stream(), dstate_.as<CgState>(), sbs,
+                           dmi, tol, xtol, np);
+    };
+    auto rhs = [&](auto res) {   // rhs = y0 - mu div(d - b)
+        hipLaunchKernelGGL((k_sb_rhs<R, 256, decltype(res)::value>), dim3(nchunk_), dim3(256), 0, c_.stream(),
+                           dchunk_.as<ChunkRef>(), dprob_.as<ProbDev>(), sbs, Y0_.as<R>(), Y_.as<R>(), Dv_.as<R>(),
+                           Bv_.as<R>(), R_.as<R>(), cpartial_.as<double>(), total_);
+        LC_HIP(hipGetLastError());
+    };
     // x = cgsolver(A - mu lap, rhs, x, inner)
-    hipLaunchKernelGGL(k_cg_arm, dim3(ceil_div(np, 64)), dim3(64), 0, c_.stream(),
-                       dstate_.as<CgState>(), sbs, dmi, tol, xtol, np);
-    cg_setup(false, true, mi, tol, xtol);
+    if (full) {
+        rhs(std::false_type{});
+        arm();
+        cg_setup(zero, true, mi, tol, xtol);
+    } else {
+        arm();
+        rhs(std::true_type{});
+        hipLaunchKernelGGL(k_cg_fin0, dim3(np), dim3(FIN_NT), 0, c_.stream(), dprob_.as<ProbDev>(),
+                           dstate_.as<CgState>(), cpartial_.as<double>());
+        LC_HIP(hipGetLastError());
+    }
     for (int it = 0; it < inner; ++it) cg_iteration_t<R>(hsync, true);
     // shrink + Bregman update + convergence
     hipLaunchKernelGGL((k_sb_shrink<R, 256>), dim3(nchunk_), dim3(256), 0, c_.stream(),
@@ -1164,17 +1367,32 @@ void Batch2D::split_bregman(const std::vector<float> &lambda, const std::vector<
     DBuf dmi(sizeof(int) * np);
     LC_HIP(hipMemcpyAsync(dmi.as(), mi.data(), sizeof(int) * np, hipMemcpyHostToDevice,
                           c_.stream()));
-    auto outer_iter = [&](bool hsync) {
+    auto outer_iter = [&](bool hsync, int it) {
         LC_ETYPE([&](auto z) {
-            sb_outer_t<decltype(z)>(hsync, tol, xtol, inner, dmi.as<int>(), mi);
+            sb_outer_t<decltype(z)>(hsync, tol, xtol, inner, dmi.as<int>(), mi, it % SB_REFRESH == 0,
+                                    it == 0 && x0_zero);
         });
     };
     if (graph && !host_sync) {
-        CapturedGraph gr(c_, [&] { outer_iter(false); });
-        for (int it = 0; it < outer; ++it) gr.launch();
+        // the first outer iteration, then SB_REFRESH at a time from a graph
+        // (once captured, worth two replays), the rest one by one
+        std::unique_ptr<CapturedGraph> gr;
+        for (int it = 0; it < outer;) {
+            const int left = (outer - it) / SB_REFRESH;
+            if (it % SB_REFRESH == 1 && left >= (gr ? 1 : 2)) {
+                if (!gr)
+                    gr = std::make_unique<CapturedGraph>(c_, [&] {
+                        for (int k = 0; k < SB_REFRESH; ++k) outer_iter(false, it + k);
+                    });
+                gr->launch();
+                it += SB_REFRESH;
+            } else {
+                outer_iter(false, it++);
+            }
+        }
     } else {
         for (int it = 0; it < outer; ++it) {
-            outer_iter(host_sync);
+            outer_iter(host_sync, it);
             if (host_sync) {
                 std::vector<SbState> h = sb_state();
                 bool any = false;

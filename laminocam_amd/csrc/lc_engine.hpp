@@ -369,7 +369,8 @@ class Batch2D {
     // middle pass of a class: 2-D column pass or the 3-D slice-coupled pass
     template <typename R> void toep_mid(const ToepClass &k, const CgState *st, cpx<R> *U);
     template <typename R> void sb_outer_t(bool hsync, double tol, double xtol, int inner,
-                                          const int *dmi, const std::vector<int> &mi);
+                                          const int *dmi, const std::vector<int> &mi, bool full,
+                                          bool zero);
 
     Ctx &c_;
     bool f64_ = false;

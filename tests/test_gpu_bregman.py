@@ -55,6 +55,33 @@ def test_split_bregman_tv_active_matches_oracle(lc, orc64, zero_pad, aniso):
     assert rel_l2(x64, xr) < 1e-9
 
 
+# the vector kernels take four consecutive elements per thread: slices of 2 and 3
+# columns (a group crosses several rows), odd sizes (groups cross row and slice
+# ends), a single slice (no slice axis), more than one 4096-element chunk with a
+# partial group at its end; odd and even numbers of outer iterations
+@pytest.mark.parametrize("ns,N,outer,inner", [(1, 2, 3, 1), (3, 2, 2, 1), (4, 3, 5, 1), (1, 5, 4, 2), (3, 7, 6, 1),
+                                              (2, 47, 5, 1), (1, 66, 7, 1), (5, 31, 1, 3)])
+@pytest.mark.parametrize("zero_pad", [False, True])
+def test_split_bregman_sizes_match_oracle(lc, orc64, ns, N, outer, inner, zero_pad):
+    announce(f"sb sizes ns={ns} N={N} outer={outer} inner={inner} zero_pad={zero_pad}")
+    rng = np.random.default_rng(17 * N + ns)
+    th = np.arange(30) * np.pi / 30
+    P = orc64.psf2d(th, max(N, 8), N, method=0)
+    rhs, x0 = P.convolve(rng.random((ns, N, N))), 0.1 * rng.random((ns, N, N))
+    psf = lc.PointSpreadFunction2D(lc.PolarGrid2D(th, max(N, 8)), N)
+    for start in (np.zeros_like(x0), x0):
+        xr, rr = orc64.split_bregman(P, rhs, start, 0.3, 8.0, outer, inner, 0.0, 0.0, boundary=int(zero_pad))
+        for graph in (False, True):
+            x, rep = lc.split_bregman(psf, rhs, start, 0.3, 8.0, outer, inner, 0.0, 0.0, zero_pad=zero_pad,
+                                      graph=graph)
+            assert rep["outer"] == rr["outer"]
+            # FP64 rounding through at most 8 well-conditioned steps
+            assert rel_l2(x, xr) < 1e-9
+        x32, _ = lc.split_bregman(psf, rhs.astype(np.float32), start.astype(np.float32), 0.3, 8.0, outer, inner,
+                                  0.0, 0.0, zero_pad=zero_pad)
+        assert rel_l2(x32, xr) < 1e-3
+
+
 def test_mbir2d_sanity_split_bregman_gpu(lc, orc64):
     """tests/test_mbir2d_sanity.cpp:98-205 on the GPU path: forward2d,
     backproj2d, Split-Bregman (lambda 0.1, mu 5, 50 x 25, tol = xtol = 1e-5)
