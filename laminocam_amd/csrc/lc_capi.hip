@@ -1,6 +1,7 @@
 // extern "C" boundary of the library (include/laminocam.h).
 #include <atomic>
 #include <cstring>
+#include <optional>
 #include <string>
 
 #include "laminocam.h"
@@ -182,13 +183,44 @@ template <typename T>
 static void sysmat_psf(lc_ctx ctx, ProbSpec ps, const T *x, T *y, uint32_t flags) {
     std::lock_guard<std::mutex> lk(ctx->c.mu);
     ctx->c.set_current();
-    Batch2D b(ctx->c, {ps}, sizeof(T) == 8);
-    const size_t bytes = sizeof(T) * (size_t)b.size(0);   // exactly the problem's size
+    Ctx &c = ctx->c;
+    constexpr bool f64 = sizeof(T) == 8;
+    // the operator alone, on the caller's vectors where the kernels can read
+    // them (device memory, 16-byte aligned pairs), else on staged copies
+    const int64_t n = ps.g3 ? ps.g3->n1 * ps.g3->N * ps.g3->N : ps.ns * ps.g->N * ps.g->N;
+    const size_t bytes = sizeof(T) * (size_t)n, pad = (bytes + 255) & ~(size_t)255;
     const bool dev = flags & LC_DEVICE_PTRS;
-    copy_in(ctx->c, b.Xv(), x, bytes, dev);
-    b.toeplitz(b.Xv(), b.APv());
-    copy_out(ctx->c, y, b.APv(), bytes, dev);
-    ctx->c.sync();
+    const bool direct = dev && (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) % 16 == 0;
+    // small stacks: the intermediate and the tables in context scratch, no allocation
+    // (what must not live there, the spectrum and the twiddles, comes first)
+    Arena ar;
+    struct Off { ~Off() { tl_arena = nullptr; } };
+    std::optional<Off> off;
+    if (!ps.g3) {
+        const size_t need = 2 * sizeof(T) * (size_t)ps.ns * (size_t)((ps.g->H + 16) * ps.g->N + 2) +
+                            sizeof(SliceRef) * (size_t)ps.ns + sizeof(ProbDev) + 1024;
+        if (need <= ((size_t)64 << 20)) {
+            if (f64 ? !ps.g->psf64_ready : !ps.g->psf_ready) geom2d_build_psf(c, *ps.g, f64);
+            if (f64) c.template twiddles<double>((int)ps.g->M);
+            else c.template twiddles<float>((int)ps.g->M);
+            ar.base = static_cast<char *>(c.scratch(6, need));
+            ar.cap = need;
+            ar.who = "lc_sysmat2d_psf";
+        }
+    }
+    char *st = direct ? nullptr : static_cast<char *>(c.scratch(2, 2 * pad));
+    if (!direct) copy_in(c, st, x, bytes, dev);
+    if (ar.base) {
+        tl_arena = &ar;
+        off.emplace();
+    }
+    Batch2D b(c, {ps}, f64, true, true);
+    off.reset();
+    b.toeplitz(direct ? static_cast<const void *>(x) : st, direct ? static_cast<void *>(y) : st + pad);
+    if (!direct) {
+        copy_out(c, y, st + pad, bytes, dev);
+        c.sync();
+    }
 }
 
 extern "C" {

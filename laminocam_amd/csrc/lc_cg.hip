@@ -785,8 +785,8 @@ void fd_launch(Ctx &c, int op, const double *in, double *out, int n1, int n2, in
 // ----------------------------------------------------------------------------
 // Batch2D
 // ----------------------------------------------------------------------------
-Batch2D::Batch2D(Ctx &c, const std::vector<ProbSpec> &probs, bool f64, bool class_streams)
-    : c_(c), f64_(f64), probs_(probs) {
+Batch2D::Batch2D(Ctx &c, const std::vector<ProbSpec> &probs, bool f64, bool class_streams, bool op_only)
+    : c_(c), f64_(f64), op_only_(op_only), probs_(probs) {
     LC_REQUIRE(!probs.empty(), "batch: no problems");
     build();
     const char *e = std::getenv("LC_CLASS_STREAMS");
@@ -831,7 +831,7 @@ void Batch2D::build() {
     int64_t off = 0, uoff = 0;
     int chunk = 0, slot = 0;
     // host tables stay alive until the uploads below have completed
-    std::vector<std::vector<SliceRef>> keep;
+    auto &keep = hslices_;
     // classes
     for (auto &kv : groups) {
         auto k = std::make_unique<ToepClass>();
@@ -917,14 +917,18 @@ void Batch2D::build() {
     total_u_ = uoff;
     nchunk_ = chunk;
     nslot_ = slot;
+    U_.alloc(cb * (size_t)total_u_);
+    dprob_.alloc(sizeof(ProbDev) * np);
+    if (op_only_) {   // (null states: every problem active)
+        LC_HIP(hipMemcpyAsync(dprob_.as(), hprob_.data(), sizeof(ProbDev) * np, hipMemcpyHostToDevice, c_.stream()));
+        return;
+    }
     const size_t fb = esize() * (size_t)total_;
     X_.alloc(fb);
     R_.alloc(fb);
     P_.alloc(fb);
     AP_.alloc(fb);
     Y_.alloc(fb);
-    U_.alloc(cb * (size_t)total_u_);
-    dprob_.alloc(sizeof(ProbDev) * np);
     dchunk_.alloc(sizeof(ChunkRef) * hchunk_.size());
     dstate_.alloc(sizeof(CgState) * np);
     dsb_.alloc(sizeof(SbState) * np);
@@ -946,6 +950,7 @@ void Batch2D::build() {
     LC_HIP(hipMemcpyAsync(dsb_.as(), zs.data(), sizeof(SbState) * np, hipMemcpyHostToDevice,
                           c_.stream()));
     c_.sync();
+    hslices_.clear();
 }
 
 // The Toeplitz passes of the size classes touch disjoint parts of the batch
@@ -992,6 +997,11 @@ void Batch2D::apply_op(const void *src, void *dst, bool sb, bool dot) {
 }
 
 void Batch2D::toeplitz(const void *src, void *dst) {
+    if (op_only_) {
+        apply_op(src, dst, false, false);
+        c_.sync();
+        return;
+    }
     // all problems: arm every state active with no iterations
     std::vector<int> one(probs_.size(), 1);
     DBuf mi(sizeof(int) * one.size());

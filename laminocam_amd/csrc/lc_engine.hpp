@@ -2,6 +2,7 @@
 // engine.
 #pragma once
 
+#include <complex>
 #include <vector>
 
 #include "lc_runtime.hpp"
@@ -45,6 +46,14 @@ struct Geom2D {
     bool psf_ready = false, psf64_ready = false;
     Nufft2D nu;
 };
+
+// deconvolution factors (-1)^m / psi_hat(2 pi m / nf), m = -n/2 .. n - n/2 - 1, of the
+// width-w kernel on an nf-cell fine grid
+void es_correction(int n, int nf, int w, double beta, float *corr);
+// Bluestein tables of an n-point transform by length L >= 2 n - 1 (2^p 3^q):
+// chirp e^{i pi k^2 / n} and FFT-(its even extension) / L
+void bluestein_tables(int n, int L, std::vector<std::complex<double>> &chirp,
+                      std::vector<std::complex<double>> &bhat);
 
 // NUFFT projectors on device buffers (src/projection.cpp:146-182):
 // forward2d: vol (ns x N x N) -> sino (ns x nang x nrad); backproj2d: reverse
@@ -303,7 +312,9 @@ class Batch2D {
     // class_streams: run the size classes' Toeplitz passes on the context's
     // auxiliary streams side by side (off where several contexts share the
     // device's hardware queues, as the server's lanes do)
-    Batch2D(Ctx &c, const std::vector<ProbSpec> &probs, bool f64 = false, bool class_streams = true);
+    // op_only: no vectors, no solver state; toeplitz() alone, on the caller's vectors
+    Batch2D(Ctx &c, const std::vector<ProbSpec> &probs, bool f64 = false, bool class_streams = true,
+            bool op_only = false);
     bool f64() const { return f64_; }
     size_t esize() const { return f64_ ? sizeof(double) : sizeof(float); }
     int nprob() const { return (int)probs_.size(); }
@@ -373,7 +384,8 @@ class Batch2D {
                                           bool zero);
 
     Ctx &c_;
-    bool f64_ = false;
+    bool f64_ = false, op_only_ = false;
+    std::vector<std::vector<SliceRef>> hslices_;   // host tables of pending uploads
     std::vector<ProbSpec> probs_;
     std::vector<ProbDev> hprob_;
     std::vector<ChunkRef> hchunk_;

@@ -710,47 +710,95 @@ k_fine_rows_t2(const float2 *__restrict__ V, float2 *__restrict__ fine, int nf, 
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-// Gauss-Legendre quadrature of the kernel's Fourier transform (FP64):
+// the kernel's Fourier transform by 96-point Gauss-Legendre quadrature (FP64):
 // Psi(xi) = (w/2) int_{-pi/2}^{pi/2} e^{beta (cos t - 1)} cos(xi (w/2) sin t) cos t dt
-static double es_phihat(double beta, int w, double xi) {
-    static double gx[96], gw[96];
-    static bool ready = false;
-    const int n = 96;
-    if (!ready) {
-        for (int i = 0; i < n; ++i) {
-            double x = std::cos(M_PI * (i + 0.75) / (n + 0.5));
+// The integrand is even, so 48 nodes; what does not depend on xi is tabulated.
+namespace {
+struct EsNodes {
+    static constexpr int N = 96;
+    double x[N / 2], w[N / 2];   // nodes in (0, 1) and weights
+    EsNodes() {
+        for (int i = 0; i < N / 2; ++i) {
+            double v = std::cos(M_PI * (i + 0.75) / (N + 0.5)), dp = 0.0;
             for (int it = 0; it < 100; ++it) {
-                double p0 = 1.0, p1 = x;
-                for (int k = 2; k <= n; ++k) {
-                    double p2 = ((2.0 * k - 1.0) * x * p1 - (k - 1.0) * p0) / k;
+                double p0 = 1.0, p1 = v;
+                for (int k = 2; k <= N; ++k) {
+                    const double p2 = ((2.0 * k - 1.0) * v * p1 - (k - 1.0) * p0) / k;
                     p0 = p1;
                     p1 = p2;
                 }
-                double dp = n * (x * p1 - p0) / (x * x - 1.0);
-                double dx = p1 / dp;
-                x -= dx;
+                dp = N * (v * p1 - p0) / (v * v - 1.0);
+                const double dx = p1 / dp;
+                v -= dx;
                 if (std::fabs(dx) < 1e-16) break;
             }
-            double p0 = 1.0, p1 = x;
-            for (int k = 2; k <= n; ++k) {
-                double p2 = ((2.0 * k - 1.0) * x * p1 - (k - 1.0) * p0) / k;
+            double p0 = 1.0, p1 = v;
+            for (int k = 2; k <= N; ++k) {
+                const double p2 = ((2.0 * k - 1.0) * v * p1 - (k - 1.0) * p0) / k;
                 p0 = p1;
                 p1 = p2;
             }
-            double dp = n * (x * p1 - p0) / (x * x - 1.0);
-            gx[i] = x;
-            gw[i] = 2.0 / ((1.0 - x * x) * dp * dp);
+            dp = N * (v * p1 - p0) / (v * v - 1.0);
+            x[i] = v;
+            w[i] = 2.0 / ((1.0 - v * v) * dp * dp);
         }
-        ready = true;
     }
+};
+} // namespace
+
+void es_correction(int n, int nf, int w, double beta, float *corr) {
+    static const EsNodes q;
+    constexpr int NQ = EsNodes::N / 2;
     const double hw = 0.5 * w;
-    double s = 0.0;
-    for (int i = 0; i < n; ++i) {
-        const double t = 0.5 * M_PI * gx[i];
-        const double ct = std::cos(t);
-        s += gw[i] * std::exp(beta * (ct - 1.0)) * std::cos(xi * hw * std::sin(t)) * ct;
+    double arg[NQ], amp[NQ];
+    for (int i = 0; i < NQ; ++i) {
+        const double t = 0.5 * M_PI * q.x[i], ct = std::cos(t);
+        arg[i] = hw * std::sin(t) * 2.0 * M_PI / (double)nf;
+        amp[i] = 2.0 * q.w[i] * std::exp(beta * (ct - 1.0)) * ct;
     }
-    return hw * 0.5 * M_PI * s;
+    for (int m = 0; m <= n / 2; ++m) {
+        double s = 0.0;
+        for (int i = 0; i < NQ; ++i) s += amp[i] * std::cos((double)m * arg[i]);
+        const float c = (float)(((m & 1) ? -1.0 : 1.0) / (hw * 0.5 * M_PI * s));
+        corr[n / 2 - m] = c;
+        if (n / 2 + m < n) corr[n / 2 + m] = c;
+    }
+}
+
+// y[0 .. n) = DFT_- of x[0], x[step], ... (n = 2^p 3^q), recursively by radix 2 and 3
+static void host_dft(const std::complex<double> *x, int n, int step, std::complex<double> *y) {
+    if (n == 1) {
+        y[0] = x[0];
+        return;
+    }
+    const int r = n % 2 == 0 ? 2 : 3, m = n / r;
+    for (int j = 0; j < r; ++j) host_dft(x + j * step, m, step * r, y + j * m);
+    for (int k = 0; k < m; ++k) {
+        const std::complex<double> a = y[k], b = y[m + k] * std::polar(1.0, -2.0 * M_PI * k / n);
+        if (r == 2) {
+            y[k] = a + b;
+            y[m + k] = a - b;
+        } else {
+            const std::complex<double> c = y[2 * m + k] * std::polar(1.0, -4.0 * M_PI * k / n);
+            const std::complex<double> s = b + c, d = std::complex<double>(0.0, -std::sqrt(0.75)) * (b - c);
+            y[k] = a + s;
+            y[m + k] = a - 0.5 * s + d;
+            y[2 * m + k] = a - 0.5 * s - d;
+        }
+    }
+}
+
+void bluestein_tables(int n, int L, std::vector<std::complex<double>> &chirp, std::vector<std::complex<double>> &bhat) {
+    chirp.resize(n);
+    std::vector<std::complex<double>> b(L, 0.0);
+    for (int k = 0; k < n; ++k) {
+        const double ang = M_PI * (double)(((int64_t)k * k) % (2 * (int64_t)n)) / (double)n;
+        b[k] = chirp[k] = std::complex<double>(std::cos(ang), std::sin(ang));
+        if (k) b[L - k] = b[k];
+    }
+    bhat.resize(L);
+    host_dft(b.data(), L, 1, bhat.data());
+    for (auto &v : bhat) v /= (double)L;
 }
 
 // (cos, sin) of every projection angle, FP64, once per geometry: the spread
@@ -779,31 +827,11 @@ static void det_blue_init(Ctx &c, Nufft2D &u, int n) {
     int L = 16;
     while (L < 2 * n - 1) L *= 2;
     LC_REQUIRE(fft_make_plan(L, u.plan_det), "detector transform: no Bluestein length");
-    std::vector<double2> t(n + L);   // chirp, then b -> bhat
-    std::vector<std::complex<double>> b(L, 0.0);
-    for (int k = 0; k < n; ++k) {
-        const double ang = M_PI * (double)(((int64_t)k * k) % (2 * (int64_t)n)) / (double)n;
-        t[k] = make_double2(std::cos(ang), std::sin(ang));
-        b[k] = std::complex<double>(t[k].x, t[k].y);   // conj(a_k) of SIGN -1
-        if (k) b[L - k] = b[k];
-    }
-    // forward FFT on the host: radix-2, decimation in time
-    for (int i = 1, j = 0; i < L; ++i) {
-        int bit = L >> 1;
-        for (; j & bit; bit >>= 1) j ^= bit;
-        j ^= bit;
-        if (i < j) std::swap(b[i], b[j]);
-    }
-    std::vector<std::complex<double>> w(L / 2);
-    for (int q = 0; q < L / 2; ++q) w[q] = std::polar(1.0, -2.0 * M_PI * q / L);
-    for (int len = 2; len <= L; len *= 2)
-        for (int i = 0; i < L; i += len)
-            for (int k = 0; k < len / 2; ++k) {
-                const std::complex<double> p = b[i + k], q = b[i + k + len / 2] * w[k * (L / len)];
-                b[i + k] = p + q;
-                b[i + k + len / 2] = p - q;
-            }
-    for (int m = 0; m < L; ++m) t[n + m] = make_double2(b[m].real() / L, b[m].imag() / L);
+    std::vector<std::complex<double>> ch, bh;
+    bluestein_tables(n, L, ch, bh);
+    std::vector<double2> t;
+    for (const auto &v : ch) t.push_back(make_double2(v.real(), v.imag()));
+    for (const auto &v : bh) t.push_back(make_double2(v.real(), v.imag()));
     u.chirp.alloc(sizeof(double2) * t.size());
     LC_HIP(hipMemcpyAsync(u.chirp.as(), t.data(), sizeof(double2) * t.size(), hipMemcpyHostToDevice, c.stream()));
     c.sync();
@@ -892,12 +920,7 @@ void nufft2d_init(Ctx &c, Geom2D &g) {
     u.w = NU_W;
     u.beta = 2.30 * NU_W;
     std::vector<float> corr(N);
-    for (int a = 0; a < N; ++a) {
-        const int m = a - N / 2;
-        const double ph = es_phihat(u.beta, NU_W, (double)m * 2.0 * M_PI / (double)nf);
-        const double sgn = (m & 1) ? -1.0 : 1.0;   // (-1)^m from the centred fine grid
-        corr[a] = (float)(sgn / ph);
-    }
+    es_correction(N, (int)nf, NU_W, u.beta, corr.data());   // (-1)^m from the centred fine grid
     u.corr.alloc(sizeof(float) * N);
     // stream-ordered copy: a legacy-stream copy would have to wait on other
     // threads' streams, some of which may be capturing graphs

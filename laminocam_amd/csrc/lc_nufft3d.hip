@@ -838,48 +838,6 @@ int fine_size(int64_t n) {
     return (int)f;
 }
 
-// psi_hat of the width-8 kernel by 96-point Gauss-Legendre quadrature (FP64)
-double es_phihat3(double beta, double xi) {
-    static double gx[96], gw[96];
-    static bool ready = false;
-    const int n = 96;
-    if (!ready) {
-        for (int i = 0; i < n; ++i) {
-            double x = std::cos(M_PI * (i + 0.75) / (n + 0.5));
-            for (int it = 0; it < 100; ++it) {
-                double p0 = 1.0, p1 = x;
-                for (int k = 2; k <= n; ++k) {
-                    double p2 = ((2.0 * k - 1.0) * x * p1 - (k - 1.0) * p0) / k;
-                    p0 = p1;
-                    p1 = p2;
-                }
-                double dp = n * (x * p1 - p0) / (x * x - 1.0);
-                double dx = p1 / dp;
-                x -= dx;
-                if (std::fabs(dx) < 1e-16) break;
-            }
-            double p0 = 1.0, p1 = x;
-            for (int k = 2; k <= n; ++k) {
-                double p2 = ((2.0 * k - 1.0) * x * p1 - (k - 1.0) * p0) / k;
-                p0 = p1;
-                p1 = p2;
-            }
-            double dp = n * (x * p1 - p0) / (x * x - 1.0);
-            gx[i] = x;
-            gw[i] = 2.0 / ((1.0 - x * x) * dp * dp);
-        }
-        ready = true;
-    }
-    const double hw = 0.5 * W3;
-    double s = 0.0;
-    for (int i = 0; i < n; ++i) {
-        const double t = 0.5 * M_PI * gx[i];
-        const double ct = std::cos(t);
-        s += gw[i] * std::exp(beta * (ct - 1.0)) * std::cos(xi * hw * std::sin(t)) * ct;
-    }
-    return hw * 0.5 * M_PI * s;
-}
-
 } // namespace
 
 int nufft3d_fine_n(int64_t n) { return fine_size(n); }
@@ -905,35 +863,17 @@ void det_line_init(Ctx &c, DetLine &d, int n) {
     LC_REQUIRE(L <= LN_NT * LN_ME, "detector transform: width too large");
     LC_REQUIRE(fft_make_plan((int)L, d.plan), "detector transform: no Bluestein length");
     d.blue = true;
-    // chirp a_k = e^{+i pi k^2 / n} (the kernel conjugates it for sign -1)
-    std::vector<float2> ch(n);
-    std::vector<std::complex<double>> a(n);
-    for (int k = 0; k < n; ++k) {
-        const int64_t q = ((int64_t)k * k) % (2 * (int64_t)n);
-        const double ang = M_PI * (double)q / (double)n;
-        a[k] = std::complex<double>(std::cos(ang), std::sin(ang));
-        ch[k] = make_float2((float)a[k].real(), (float)a[k].imag());
-    }
-    // bhat for sign s: b_k = conj(a_k^s) = e^{-s i pi k^2/n} on k and L-k
-    // (L >= 2n - 1, so the two runs do not meet); bhat = FFT-(b) / L in FP64,
-    // [sign -1 | sign +1].  b_k = b_{L-k} pairs e^{-2 pi i k m / L} with its
-    // conjugate: bhat_m = (b_0 + sum_{0<k<n} b_k 2 cos(2 pi k m / L)) / L, a
-    // real combination of the b_k, so the sign +1 table is the conjugate of
-    // the sign -1 one.  cos(2 pi q / L) comes from a table over q = k m mod L.
-    std::vector<double> cq(L);
-    for (int64_t q = 0; q < L; ++q) cq[q] = std::cos(2.0 * M_PI * (double)q / (double)L);
-    std::vector<float2> bh(2 * L);
+    // chirp a_k = e^{+i pi k^2 / n} (the kernel conjugates it for sign -1); bhat
+    // for sign s is FFT-(b) / L with b_k = conj(a_k^s) on k and L - k (L >= 2n - 1,
+    // so the two runs do not meet), [sign -1 | sign +1]: b is even, so the sign +1
+    // table is the conjugate of the sign -1 one
+    std::vector<std::complex<double>> ch64, bh64;
+    bluestein_tables(n, (int)L, ch64, bh64);
+    std::vector<float2> ch(n), bh(2 * L);
+    for (int k = 0; k < n; ++k) ch[k] = make_float2((float)ch64[k].real(), (float)ch64[k].imag());
     for (int64_t m = 0; m < L; ++m) {
-        std::complex<double> acc = a[0];
-        int64_t q = 0;
-        for (int k = 1; k < n; ++k) {
-            q += m;
-            if (q >= L) q -= L;
-            acc += a[k] * (2.0 * cq[q]);
-        }
-        acc /= (double)L;
-        bh[m] = make_float2((float)acc.real(), (float)acc.imag());
-        bh[L + m] = make_float2((float)acc.real(), (float)-acc.imag());
+        bh[m] = make_float2((float)bh64[m].real(), (float)bh64[m].imag());
+        bh[L + m] = make_float2((float)bh64[m].real(), (float)-bh64[m].imag());
     }
     d.chirp.alloc(sizeof(float2) * n);
     d.bhat.alloc(sizeof(float2) * 2 * L);
@@ -953,11 +893,8 @@ void nufft3d_init(Ctx &c, Geom3D &g) {
         LC_REQUIRE(u.nf[a] <= LN_NT * LN_ME, "3-D NUFFT: fine grid too large");
         LC_REQUIRE(fft_make_plan(u.nf[a], u.plan[a]), "3-D NUFFT: fine size not 2^p 3^q");
         u.coff[a] = (int)corr.size();
-        for (int64_t i = 0; i < nm[a]; ++i) {
-            const int64_t m = i - nm[a] / 2;
-            const double ph = es_phihat3(beta, (double)m * 2.0 * M_PI / (double)u.nf[a]);
-            corr.push_back((float)(((m & 1) ? -1.0 : 1.0) / ph));
-        }
+        corr.resize(corr.size() + nm[a]);
+        es_correction((int)nm[a], u.nf[a], W3, beta, corr.data() + u.coff[a]);
     }
     u.corr.alloc(sizeof(float) * corr.size());
     LC_HIP(hipMemcpyAsync(u.corr.as(), corr.data(), sizeof(float) * corr.size(), hipMemcpyHostToDevice,
