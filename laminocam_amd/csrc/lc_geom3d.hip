@@ -183,37 +183,81 @@ k_psf3d_gen(double2 *P, const double *rot, int nproj, int nrows, int ncols, int 
     }
 }
 
-// s[j] += w D_n(t0 + j dt) along a run; stp = (cos, sin)(pi dt), (cos, sin)(pi dt / n).
-// Terms whose denominator is below thr are evaluated directly afterwards: out
-// of the unrolled loop they cost it neither registers nor instructions.
-__device__ __forceinline__ void dirichlet_run(double (&s)[P3_RUN], double t0, double dt, int n, double inv_n,
-                                              double4 stp, double w, double thr) {
-    double ar, ai, br, bi;   // numerator (times w) and denominator phases
-    sincospi(t0, &ai, &ar);
-    sincospi(t0 * inv_n, &bi, &br);
-    ar *= w;
-    ai *= w;
-    unsigned direct = 0;
+// Pair j of a run of RUN values lies j + 1/2 steps on either side of its middle.
+// tab[i RUN/2 + j] = (w cos, w sin)((j + 1/2) pi dt_i), (cos, sin)((j + 1/2) pi dt_i / n)
+// for the row directions v (weight w), then for the groups' column directions u.
+template <int RUN>
+__global__ void k_psf3d_steps(double4 *tab, const double4 *__restrict__ v, int nv, const double *__restrict__ gu,
+                              int ngroups, int nrows, int ncols) {
+    const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = id / (RUN / 2);
+    if (i >= nv + ngroups) return;
+    const double o = (double)(id - i * (RUN / 2)) + 0.5;
+    const double dt = i < nv ? v[i].x : gu[3 * (i - nv)], w = i < nv ? v[i].w : 1.0;
+    const double inv_n = 1.0 / (double)(i < nv ? nrows : ncols);
+    double s, c, sd, cd;
+    sincospi(o * dt, &s, &c);
+    sincospi(o * dt * inv_n, &sd, &cd);
+    tab[id] = make_double4(w * c, w * s, cd, sd);
+}
+
+// s[k] += w D_n(tc + (k - (RUN-1)/2) dt), or s[k] *= D_n (MUL, w = 1).  Both sines of
+// a pair come from the middle's sine and cosine by the addition theorem, three
+// operations per pair and free of a recurrence's growing error, and the two
+// denominators share one hardware reciprocal, refined by a Newton step (the FP64
+// operator's error against 64 bits falls by a sixth over ten geometries).  Terms
+// whose denominator is below thr are evaluated directly afterwards: out of the
+// unrolled loop they cost it neither registers nor instructions.
+template <int RUN, bool MUL>
+__device__ __forceinline__ void dirichlet_run(double (&s)[RUN], double tc, double dt, int n, double inv_n,
+                                              const double4 *__restrict__ tab, double w, double thr) {
+    double sa, ca, sb, cb;
+    sincospi(tc, &sa, &ca);
+    sincospi(tc * inv_n, &sb, &cb);
+    bool direct = false;
 #pragma unroll
-    for (int j = 0; j < P3_RUN; ++j) {
-        // the hardware reciprocal refined by one Newton step, as above
-        double r = __builtin_amdgcn_rcp(bi);
-        r = fma(r, fma(-bi, r, 1.0), r);
-        const bool f = fabs(bi) > thr;
-        s[j] = f ? fma(ai, r, s[j]) : s[j];
-        direct |= f ? 0u : 1u << j;
-        const double a = ar * stp.x - ai * stp.y, b = br * stp.z - bi * stp.w;
-        ai = ar * stp.y + ai * stp.x;
-        bi = br * stp.w + bi * stp.z;
-        ar = a;
-        br = b;
+    for (int j = 0; j < RUN / 2; ++j) {
+        const double4 T = tab[j];
+        const int kp = RUN / 2 + j, km = RUN / 2 - 1 - j;
+        const double pa = sa * T.x, ap = fma(ca, T.y, pa), am = fma(-ca, T.y, pa);
+        const double pb = sb * T.z, bp = fma(cb, T.w, pb), bm = fma(-cb, T.w, pb);
+        const bool fp = fabs(bp) > thr, fm = fabs(bm) > thr;
+        // 2^300 in place of a small denominator: its quotient vanishes, the other stays exact
+        const double dp = __hiloint2double(fp ? __double2hiint(bp) : 0x52b00000, __double2loint(bp));
+        const double dm = __hiloint2double(fm ? __double2hiint(bm) : 0x52b00000, __double2loint(bm));
+        const double den = dp * dm;
+        double r = __builtin_amdgcn_rcp(den);
+        r = fma(r, fma(-den, r, 1.0), r);
+        if (MUL) {
+            s[kp] *= fp ? ap * (r * dm) : 1.0;
+            s[km] *= fm ? am * (r * dp) : 1.0;
+        } else {
+            s[kp] = fma(ap, r * dm, s[kp]);
+            s[km] = fma(am, r * dp, s[km]);
+        }
+        direct |= !(fp && fm);
     }
-    while (direct) {
-        const int j = __ffs(direct) - 1;
-        direct &= direct - 1;
-        const double d = w * dirichlet_d(fma((double)j, dt, t0), n, inv_n);
+    if (!direct) return;
+    // which ones: the same operations once more, kept apart from the first time's
+    // so that no value of those stays in a register for this
+    asm volatile("" : "+v"(sb), "+v"(cb));
+    unsigned at = 0;
 #pragma unroll
-        for (int k = 0; k < P3_RUN; ++k) s[k] += k == j ? d : 0.0;
+    for (int j = 0; j < RUN / 2; ++j) {
+        const double4 T = tab[j];
+        const double pb = sb * T.z;
+        at |= fabs(fma(cb, T.w, pb)) > thr ? 0u : 1u << (RUN / 2 + j);
+        at |= fabs(fma(-cb, T.w, pb)) > thr ? 0u : 1u << (RUN / 2 - 1 - j);
+    }
+    while (at) {
+        const int k = __ffs(at) - 1;
+        at &= at - 1;
+        const double d = w * dirichlet_d(fma((double)k - 0.5 * (RUN - 1), dt, tc), n, inv_n);
+#pragma unroll
+        for (int i = 0; i < RUN; ++i) {
+            if (MUL) s[i] *= i == k ? d : 1.0;
+            else s[i] += i == k ? d : 0.0;
+        }
     }
 }
 
@@ -221,63 +265,49 @@ __device__ __forceinline__ void dirichlet_run(double (&s)[P3_RUN], double t0, do
 // projections of one tilt (gamma, beta) do: group q's projections are
 // v[goff[q]] .. v[goff[q + 1] - 1] (x, y, z, weight), and its terms are
 // D_ncols(m.u) sum_i w_i D_nrows(m.v_i), one Dirichlet factor per projection
-// in place of two.  Runs follow mx from -M/2 upwards, so none wraps.  The PSF
-// of the laminography shape (64 x 1536^2, 360 projections of 89 x 721) takes
-// 12.0 ms against 47.8 ms with both factors per projection (12 FP64 operations
-// and a reciprocal per term in place of 25; a full turn's projections halve).
-__global__ void __launch_bounds__(256, 4)
-k_psf3d_gen_grouped(double2 *P, const double4 *__restrict__ v, const int *__restrict__ goff,
-                    const double *__restrict__ gu, int ngroups, int nrows, int ncols, int M1, int M, double thr) {
-    __shared__ double4 vs[P3_CHUNK], stp[P3_CHUNK];
+// in place of two.  Runs follow mx from -M/2 upwards, so none wraps.  FP64
+// arithmetic bounds it: per term 3 operations for the sines, 4 and half a
+// reciprocal for the quotient, and 1/RUN of the middle's two sincospi.  The
+// tables' uniform addresses make them scalar loads.  The PSF of the
+// laminography shape (64 x 1536^2, 360 projections of 89 x 721) takes 7.5 ms
+// against 12.0 ms with the sines by recurrence in runs of 16 and 47.8 ms with
+// both factors per projection.
+template <int RUN>
+__global__ void __launch_bounds__(256, RUN == 32 ? 3 : 4)
+k_psf3d_gen_grouped(double2 *__restrict__ P, const double4 *__restrict__ v, const int *__restrict__ goff,
+                    const double *__restrict__ gu, const double4 *__restrict__ tab, int ngroups, int nrows, int ncols,
+                    int M1, int M, double thr) {
     const double inv_c = 1.0 / (double)ncols, inv_r = 1.0 / (double)nrows;
-    const int runs = (M + P3_RUN - 1) / P3_RUN;
+    const int runs = (M + RUN - 1) / RUN;
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t per_z = (int64_t)M * runs;
     const int iz = (int)(gid / per_z);
     const int rem = (int)(gid - (int64_t)iz * per_z);
-    const int iy = rem / runs, x0 = (rem - iy * runs) * P3_RUN;
-    const bool valid = iz <= M1 / 2;   // no early return: the block synchronises below
+    const int iy = rem / runs, x0 = (rem - iy * runs) * RUN;
+    if (iz > M1 / 2) return;
     const double mz = (double)(iz < (M1 + 1) / 2 ? iz : iz - M1);
-    const double my = (double)(iy < (M + 1) / 2 ? iy : iy - M), mx = (double)(x0 - M / 2);
+    const double my = (double)(iy < (M + 1) / 2 ? iy : iy - M);
+    const double mc = (double)(x0 - M / 2) + 0.5 * (RUN - 1);   // the run's middle
+    const int nv = goff[ngroups];
     for (int q = 0; q < ngroups; ++q) {
-        double s[P3_RUN];
+        double s[RUN];
 #pragma unroll
-        for (int j = 0; j < P3_RUN; ++j) s[j] = 0.0;
-        for (int a0 = goff[q], a1 = goff[q + 1]; a0 < a1; a0 += P3_CHUNK) {
-            const int na = min(P3_CHUNK, a1 - a0);
-            __syncthreads();
-            for (int i = threadIdx.x; i < na; i += blockDim.x) {
-                const double4 d = v[a0 + i];
-                double4 st;
-                sincospi(d.x, &st.y, &st.x);
-                sincospi(d.x * inv_r, &st.w, &st.z);
-                vs[i] = d;
-                stp[i] = st;
-            }
-            __syncthreads();
-            if (!valid) continue;
-            for (int i = 0; i < na; ++i) {
-                const double4 d = vs[i];
-                dirichlet_run(s, mx * d.x + my * d.y + mz * d.z, d.x, nrows, inv_r, stp[i], d.w,
-                              thr);
-            }
+        for (int j = 0; j < RUN; ++j) s[j] = 0.0;
+        for (int i = goff[q]; i < goff[q + 1]; ++i) {
+            const double4 d = v[i];
+            dirichlet_run<RUN, false>(s, mc * d.x + my * d.y + mz * d.z, d.x, nrows, inv_r,
+                                      tab + (size_t)i * (RUN / 2), d.w, thr);
         }
-        if (!valid) continue;
-        const double ux = gu[3 * q], t0 = mx * ux + my * gu[3 * q + 1] + mz * gu[3 * q + 2];
-        double c[P3_RUN];
-#pragma unroll
-        for (int j = 0; j < P3_RUN; ++j) c[j] = 0.0;
-        double4 st;
-        sincospi(ux, &st.y, &st.x);
-        sincospi(ux * inv_c, &st.w, &st.z);
-        dirichlet_run(c, t0, ux, ncols, inv_c, st, 1.0, thr);
+        const double ux = gu[3 * q];
+        dirichlet_run<RUN, true>(s, mc * ux + my * gu[3 * q + 1] + mz * gu[3 * q + 2], ux, ncols, inv_c,
+                                 tab + (size_t)(nv + q) * (RUN / 2), 1.0, thr);
         const bool mirror = iz >= 1 && 2 * iz < M1;
 #pragma unroll
-        for (int j = 0; j < P3_RUN; ++j) {
+        for (int j = 0; j < RUN; ++j) {
             if (x0 + j >= M) break;
             const int m = x0 + j - M / 2, ix = m < 0 ? m + M : m;
             double2 *p = P + ((size_t)iz * M + iy) * M + ix;
-            const double t = c[j] * s[j] + (q ? p->x : 0.0);
+            const double t = s[j] + (q ? p->x : 0.0);
             *p = make_double2(t, 0.0);
             if (mirror) P[((size_t)(M1 - iz) * M + (M - iy) % M) * M + (M - ix) % M] = make_double2(t, 0.0);
         }
@@ -412,22 +442,37 @@ void geom3d_build_psf(Ctx &c, Geom3D &g, bool f64) {
     double2 *P = reinterpret_cast<double2 *>(c.scratch(0, sizeof(double2) * np));
     const int64_t threads = (int64_t)(M1 / 2 + 1) * M * ceil_div(M, P3_RUN);
     const PsfGroups gr = psf_groups(g, !f64);
-    DBuf dgr;   // v, u, off
+    DBuf dgr;   // the runs' tables, v, u, off
     if (gr.off.size() > 1 && 2 * (gr.off.size() - 1) <= (size_t)g.nproj) {
-        const size_t bv = sizeof(double4) * gr.v.size(), bu = sizeof(double) * gr.u.size(),
-                     bo = sizeof(int) * gr.off.size();
+        const int ng = (int)gr.off.size() - 1, nv = (int)gr.v.size();
+        // runs of 32 share the middle's sines among more terms; runs of 16 where
+        // those would leave the chip below three waves per SIMD
+        const int run = (int64_t)(M1 / 2 + 1) * M * ceil_div(M, 32) >= 3 * 1024 * 64 ? 32 : 16;
+        const size_t bv = sizeof(double4) * gr.v.size(), bt = sizeof(double4) * (size_t)(nv + ng) * (run / 2),
+                     bu = sizeof(double) * gr.u.size(), bo = sizeof(int) * gr.off.size();
         std::vector<char> host(bv + bu + bo);
         std::memcpy(host.data(), gr.v.data(), bv);
         std::memcpy(host.data() + bv, gr.u.data(), bu);
         std::memcpy(host.data() + bv + bu, gr.off.data(), bo);
-        dgr.alloc(host.size());
-        LC_HIP(hipMemcpyAsync(dgr.as(), host.data(), host.size(), hipMemcpyHostToDevice, c.stream()));
+        dgr.alloc(bt + host.size());
+        char *d = dgr.as<char>();
+        LC_HIP(hipMemcpyAsync(d + bt, host.data(), host.size(), hipMemcpyHostToDevice, c.stream()));
         c.sync();
-        const char *d = dgr.as<char>();
-        hipLaunchKernelGGL(k_psf3d_gen_grouped, dim3(ceil_div(threads, 256)), dim3(256), 0, c.stream(), P,
-                           reinterpret_cast<const double4 *>(d), reinterpret_cast<const int *>(d + bv + bu),
-                           reinterpret_cast<const double *>(d + bv), (int)gr.off.size() - 1, (int)g.nrows,
-                           (int)g.ncols, M1, M, f64 ? 1e-3 : 1e-4);
+        double4 *dt = reinterpret_cast<double4 *>(d);
+        const double4 *dv = reinterpret_cast<const double4 *>(d + bt);
+        const double *du = reinterpret_cast<const double *>(d + bt + bv);
+        const int *doff = reinterpret_cast<const int *>(d + bt + bv + bu);
+        auto gen = [&](auto run_c) {
+            constexpr int RUN = decltype(run_c)::value;
+            hipLaunchKernelGGL(k_psf3d_steps<RUN>, dim3(ceil_div((int64_t)(nv + ng) * (RUN / 2), 256)), dim3(256), 0,
+                               c.stream(), dt, dv, nv, du, ng, (int)g.nrows, (int)g.ncols);
+            LC_HIP(hipGetLastError());
+            const int64_t n = (int64_t)(M1 / 2 + 1) * M * ceil_div(M, RUN);
+            hipLaunchKernelGGL(k_psf3d_gen_grouped<RUN>, dim3(ceil_div(n, 256)), dim3(256), 0, c.stream(), P, dv, doff,
+                               du, dt, ng, (int)g.nrows, (int)g.ncols, M1, M, f64 ? 1e-3 : 1e-4);
+        };
+        if (run == 32) gen(std::integral_constant<int, 32>{});
+        else gen(std::integral_constant<int, 16>{});
     } else {
         hipLaunchKernelGGL(k_psf3d_gen, dim3(ceil_div(threads, 256)), dim3(256), 0, c.stream(), P,
                            g.d_rot.as<double>(), (int)g.nproj, (int)g.nrows, (int)g.ncols, M1, M, 0);

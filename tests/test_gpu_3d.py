@@ -255,6 +255,23 @@ def test_psf3d_projection_groups_match_oracle(lc, orc64, kind, nproj):
     assert rel_l2(psf.convolve(x), ref) < 1e-12
 
 
+# a PSF large enough for runs of 32 values (the sizes above take 16), the last
+# run of a row partly empty; detectors of fewer rows than a run crosses have
+# several removable zeros in one run
+@pytest.mark.parametrize("nrows", [5, 40])
+def test_psf3d_long_runs_match_oracle(lc, orc64, nrows):
+    announce(f"psf3d long runs nrows={nrows}")
+    dims, nproj = (9, 401, 401), 6
+    th = np.arange(nproj) * (2 * np.pi / nproj)
+    ga = np.repeat([-np.pi / 6, 0.3], nproj // 2)
+    psf = lc.PointSpreadFunction(lc.PolarGrid(th, ga, np.zeros(nproj), nrows, 401), dims)
+    x = np.random.default_rng(6).random(dims)
+    ref = orc64.psf3d(th, ga, np.zeros(nproj), nrows, 401, dims, method=0).convolve(x)
+    # as above; phases of magnitude pi |m| < 2200 (3e-13)
+    assert rel_l2(psf.convolve(x.astype(np.float32)), ref) < 1e-6
+    assert rel_l2(psf.convolve(x), ref) < 1e-11
+
+
 # (recon dims, nproj, nrows, ncols): fine grids of 16 .. 81 cells per axis, two,
 # three (24 and 27 cells) and more bins of 7 to 9 corners; the last one puts
 # over 2048 points into its bins, in no multiple of a table of points
