@@ -976,11 +976,19 @@ size_t spread_bytes(int64_t npts, const int nf[3]) {
            align256(sort_tmp_bytes(npts, nbins));
 }
 
-Work3 work3(Ctx &c, const Geom3D &g) {
+// projections that the forward projector sorts at a time: up to 2^27 points
+// (2 GiB of keys and indexes; the 23 M points of 360 projections of 89 x 721
+// are one range), so its sort's memory and 32-bit indexes bound no sinogram
+int64_t range_of(const Geom3D &g) {
+    return std::min<int64_t>(g.nproj, std::max<int64_t>(1, ((int64_t)1 << 27) / ((int64_t)g.nrows * g.ncols)));
+}
+
+// nsort: projections sorted at a time
+Work3 work3(Ctx &c, const Geom3D &g, int64_t nsort) {
     const Nufft3D &u = g.nu;
-    const int64_t npts = (int64_t)g.nproj * g.nrows * g.ncols;
+    const int64_t npts = nsort * g.nrows * g.ncols;
     LC_REQUIRE(npts < (int64_t)UINT32_MAX, "3-D projector: more than 2^32 detector points");
-    const size_t bC = align256(sizeof(float2) * (size_t)npts);
+    const size_t bC = align256(sizeof(float2) * (size_t)g.nproj * g.nrows * g.ncols);
     const size_t bF = align256(sizeof(float2) * (size_t)u.nf[0] * u.nf[1] * u.nf[2]);
     const size_t bV1 = align256(sizeof(float2) * (size_t)u.nf[0] * u.nf[1] * g.n3);
     const size_t bV2 = align256(sizeof(float2) * (size_t)u.nf[0] * g.n2 * g.n3);
@@ -1096,15 +1104,17 @@ void det_axis(Ctx &c, const DetLine &d, const void *in, void *out, int64_t outer
     LC_HIP(hipGetLastError());
 }
 
-// orders the grid's points by the bins of shape S (w.key_b, w.val_b, w.bstart,
-// w.bend); drop: values of masked points are cleared there
-template <typename S> Bins3 sort_points(Ctx &c, const Geom3D &g, const Work3 &w, const Grid3 &gg, float2 *drop) {
+// orders the points of np projections from p0 on by the bins of shape S
+// (w.key_b, w.val_b, w.bstart, w.bend); drop: the values of masked points among
+// them are cleared there
+template <typename S>
+Bins3 sort_points(Ctx &c, const Geom3D &g, const Work3 &w, const Grid3 &gg, float2 *drop, int64_t p0, int64_t np) {
     const Bins3 bn = bins_of<S>(g.nu.nf);
     const unsigned nbins = count_of(bn);
-    const int64_t npts = (int64_t)g.nproj * g.nrows * g.ncols;
+    const int64_t npts = np * g.nrows * g.ncols;
     const int bits = key_bits(nbins, S::YB);
     hipLaunchKernelGGL(k_bin_keys<S>, dim3((unsigned)ceil_div(npts, 256)), dim3(256), 0, c.stream(),
-                       g.d_rot.as<double>(), gg, bn, w.key_a, w.val_a, npts, nbins, drop);
+                       g.d_rot.as<double>() + 6 * p0, gg, bn, w.key_a, w.val_a, npts, nbins, drop);
     LC_HIP(hipGetLastError());
     size_t tb = w.sort_bytes;
     LC_HIP(rocprim::radix_sort_pairs(w.sort_tmp, tb, w.key_a, w.key_b, w.val_a, w.val_b, (size_t)npts, 0, bits,
@@ -1117,8 +1127,9 @@ template <typename S> Bins3 sort_points(Ctx &c, const Geom3D &g, const Work3 &w,
     return bn;
 }
 
-// vol -> w.C; leaves the points sorted by the bins of Shape3<16>
-void type2_3d(Ctx &c, const Geom3D &g, const Work3 &w, const float *vol, bool mask) {
+// vol -> w.C, nsort projections at a time; leaves the last ones' points sorted
+// by the bins of Shape3<16>
+void type2_3d(Ctx &c, const Geom3D &g, const Work3 &w, const float *vol, bool mask, int64_t nsort) {
     const Nufft3D &u = g.nu;
     const int n1 = (int)g.n1, n2 = (int)g.n2, n3 = (int)g.n3;
     const float *corr = g.nu.corr.as<float>();
@@ -1130,20 +1141,25 @@ void type2_3d(Ctx &c, const Geom3D &g, const Work3 &w, const float *vol, bool ma
     nu_axis<2, false, false>(c, w.V1, w.F, (int64_t)u.nf[0] * u.nf[1], 1, u.nf[2], n3,
                              corr + u.coff[2], 1.0f, u.plan[2]);
     const Grid3 gg = grid3(g, mask);
-    const int64_t npts = (int64_t)g.nproj * g.nrows * g.ncols;
-    const Bins3 bn = sort_points<Shape3<16>>(c, g, w, gg, w.C);
-    // long runs read a bin's region once; short ones keep a small grid's blocks many
-    const unsigned chunk = (unsigned)std::min<int64_t>(1024, std::max<int64_t>(1, npts / (4096 * BATCH)) * BATCH);
-    hipLaunchKernelGGL(k_interp3d, dim3((unsigned)ceil_div(npts, chunk)), dim3(256), 0, c.stream(), w.F, w.C,
-                       g.d_rot.as<double>(), w.key_b, w.val_b, w.bend, (unsigned)npts, count_of(bn), chunk, gg, bn);
-    LC_HIP(hipGetLastError());
+    for (int64_t p0 = 0; p0 < g.nproj; p0 += nsort) {
+        const int64_t np = std::min<int64_t>(nsort, g.nproj - p0), npts = np * g.nrows * g.ncols;
+        float2 *C = w.C + p0 * g.nrows * g.ncols;
+        const Bins3 bn = sort_points<Shape3<16>>(c, g, w, gg, C, p0, np);
+        // long runs read a bin's region once; short ones keep a small grid's blocks many
+        const unsigned chunk =
+            (unsigned)std::min<int64_t>(1024, std::max<int64_t>(1, npts / (4096 * BATCH)) * BATCH);
+        hipLaunchKernelGGL(k_interp3d, dim3((unsigned)ceil_div(npts, chunk)), dim3(256), 0, c.stream(), w.F, C,
+                           g.d_rot.as<double>() + 6 * p0, w.key_b, w.val_b, w.bend, (unsigned)npts, count_of(bn),
+                           chunk, gg, bn);
+        LC_HIP(hipGetLastError());
+    }
 }
 
 // the sorted-bin spread with region shape S: w.C -> w.F (sorted: the points
 // are already in the order of S's bins)
 template <typename S> void spread3d(Ctx &c, const Geom3D &g, const Work3 &w, const Grid3 &gg, bool sorted) {
     const Nufft3D &u = g.nu;
-    const Bins3 bn = sorted ? bins_of<S>(u.nf) : sort_points<S>(c, g, w, gg, nullptr);
+    const Bins3 bn = sorted ? bins_of<S>(u.nf) : sort_points<S>(c, g, w, gg, nullptr, 0, g.nproj);
     const unsigned nbins = count_of(bn);
     hipLaunchKernelGGL(k_bin_order_keys, dim3(ceil_div(nbins, 256)), dim3(256), 0, c.stream(), w.bstart,
                        w.bend, bn, w.okey_a, w.oval_a, nbins);
@@ -1208,8 +1224,9 @@ void nu3_check(Ctx &c, Geom3D &g) {
 // forward (src/projection.cpp:42-64): vol {n1, N, N} -> proj {nproj, nrows, ncols}
 void forward3d_dev(Ctx &c, Geom3D &g, const float *vol, float *proj) {
     nu3_check(c, g);
-    const Work3 w = work3(c, g);
-    type2_3d(c, g, w, vol, true);
+    const int64_t nsort = range_of(g);
+    const Work3 w = work3(c, g, nsort);
+    type2_3d(c, g, w, vol, true, nsort);
     const int nr = (int)g.nrows, nc = (int)g.ncols;
     // fftshift2 -> ifft2 -> ifftshift2 along x then y; real part / (nrows ncols)
     det_axis<false, false>(c, g.nu.det_x, w.C, w.C, g.nproj * nr, 1, nc / 2, nc / 2 + (nc & 1), 1, 1.0f);
@@ -1221,7 +1238,7 @@ void forward3d_dev(Ctx &c, Geom3D &g, const float *vol, float *proj) {
 // projection or nullptr
 void backproj3d_dev(Ctx &c, Geom3D &g, const float *proj, float *vol, const double *shifts) {
     nu3_check(c, g);
-    const Work3 w = work3(c, g);
+    const Work3 w = work3(c, g, g.nproj);
     const int nr = (int)g.nrows, nc = (int)g.ncols;
     // fftshift2 -> fft2 -> ifftshift2 along x then y
     det_axis<true, false>(c, g.nu.det_x, proj, w.C, g.nproj * nr, 1, nc / 2, nc / 2 + (nc & 1), -1, 1.0f);
@@ -1232,8 +1249,8 @@ void backproj3d_dev(Ctx &c, Geom3D &g, const float *proj, float *vol, const doub
 // sysmat(x, grid) (src/gradient.cpp:32-41): Re(T1(T2 x)) / (nrows ncols), no mask
 void sysmat3d_nufft_dev(Ctx &c, Geom3D &g, const float *x, float *y) {
     nu3_check(c, g);
-    const Work3 w = work3(c, g);
-    type2_3d(c, g, w, x, false);
+    const Work3 w = work3(c, g, g.nproj);
+    type2_3d(c, g, w, x, false, g.nproj);
     type1_3d(c, g, w, y, false, nullptr, 1.0f / ((float)g.nrows * (float)g.ncols), true);
 }
 

@@ -255,6 +255,23 @@ def test_psf3d_projection_groups_match_oracle(lc, orc64, kind, nproj):
     assert rel_l2(psf.convolve(x), ref) < 1e-12
 
 
+# a sinogram of more points than the forward projector sorts at a time (2^27):
+# the projections on either side of the boundary, and the last ones, against a
+# grid of these alone
+def test_forward3d_ranges_match_a_small_grid(lc):
+    announce("forward3d in ranges")
+    dims, nrows, ncols = (6, 16, 16), 48, 64
+    per = (1 << 27) // (nrows * ncols)
+    nproj = per + 70
+    th = np.arange(nproj) * (2 * np.pi / nproj)
+    ga = np.full(nproj, -np.pi / 6)
+    vol = np.random.default_rng(7).random(dims).astype(np.float32)
+    pick = np.r_[0:3, per - 3:per + 3, nproj - 3:nproj]
+    all_of = lc.forward(vol, lc.PolarGrid(th, ga, np.zeros(nproj), nrows, ncols))[pick]
+    few = lc.forward(vol, lc.PolarGrid(th[pick], ga[pick], np.zeros(len(pick)), nrows, ncols))
+    assert rel_l2(all_of, few) < 1e-6   # the same FP32 operations per point
+
+
 # a PSF large enough for runs of 32 values (the sizes above take 16), the last
 # run of a row partly empty; detectors of fewer rows than a run crosses have
 # several removable zeros in one run
