@@ -1254,8 +1254,8 @@ void sysmat3d_nufft_dev(Ctx &c, Geom3D &g, const float *x, float *y) {
     type1_3d(c, g, w, y, false, nullptr, 1.0f / ((float)g.nrows * (float)g.ncols), true);
 }
 
-// device bytes of a 3-D back-projection's spread beyond the fine grid (the
-// padded grid, the sort of the points by bin and its scratch)
+// device bytes of a 3-D back-projection's spread beyond the fine grid (the sort
+// of the points by bin and its scratch)
 size_t nufft3d_spread_bytes(int64_t npts, const int nf[3]) { return spread_bytes(npts, nf); }
 
 int nufft3d_num_shapes() { return N_SHAPES3; }
