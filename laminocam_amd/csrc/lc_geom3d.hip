@@ -314,12 +314,25 @@ k_psf3d_gen_grouped(double2 *__restrict__ P, const double4 *__restrict__ v, cons
     }
 }
 
+// The PSF's FP64 line passes, LC > 0: at a compiled length (unrolled stages; the
+// columns of a block are a power of two, 1 << lsh), LC = 0: by the run-time
+// plan.  At 64 x 1536^2 the compiled passes take 1.20 / 1.09 / 0.92 ms (x, y, z)
+// against 1.96 / 1.37 / 0.97 ms by the run-time plan (110-125 registers in place
+// of 224-255, index arithmetic folded); x moves its 4.8 GB at 4.0 TB/s, y and z
+// are held by their 32-byte and 1-KiB pieces.
+template <int NT, int MAXE, int LC, bool COL>
+__device__ __forceinline__ void psf3_fft(double2 *buf, int nl, int lsh, const FftPlan &plan,
+                                         const double2 *__restrict__ tw) {
+    if constexpr (LC > 0) fft_lds_ct<double, LC, -1, NT, MAXE, COL>(buf, nl, lsh, tw);
+    else fft_lds<double, -1, NT, MAXE, COL>(buf, nl, COL ? 0 : plan.L, plan, tw);
+}
+
 // in-place FP64 FFT of contiguous lines of length L (nl lines per block)
-template <int SIGN, int NT, int MAXE>
+template <int NT, int MAXE, int LC>
 __global__ void __launch_bounds__(NT)
 k_psf3_rows(double2 *data, int64_t nlines, int nl, FftPlan plan, const double2 *__restrict__ tw) {
     double2 *buf = reinterpret_cast<double2 *>(lc_smem);
-    const int L = plan.L;
+    const int L = LC > 0 ? LC : plan.L;
     const int64_t row0 = (int64_t)blockIdx.x * nl;
     const int nloc = (int)min((int64_t)nl, nlines - row0);
     for (int idx = threadIdx.x; idx < nl * L; idx += NT) {
@@ -327,7 +340,7 @@ k_psf3_rows(double2 *data, int64_t nlines, int nl, FftPlan plan, const double2 *
         buf[lds_row(l, e, L)] = (l < nloc) ? data[(row0 + l) * L + e] : make_double2(0.0, 0.0);
     }
     __syncthreads();
-    fft_lds<double, SIGN, NT, MAXE, false>(buf, nl, L, plan, tw);
+    psf3_fft<NT, MAXE, LC, false>(buf, nl, 0, plan, tw);
     for (int idx = threadIdx.x; idx < nloc * L; idx += NT) {
         const int l = idx / L, e = idx - l * L;
         data[(row0 + l) * L + e] = buf[lds_row(l, e, L)];
@@ -336,10 +349,11 @@ k_psf3_rows(double2 *data, int64_t nlines, int nl, FftPlan plan, const double2 *
 
 // in-place FP64 FFT along y (stride M) for columns x < ncol of every z plane;
 // B columns per block.  grid (ceil(ncol / B), M1)
-template <int SIGN, int NT, int MAXE>
+template <int NT, int MAXE, int LC>
 __global__ void __launch_bounds__(NT)
-k_psf3_cols(double2 *P, int M, int ncol, int B, FftPlan plan, const double2 *__restrict__ tw) {
+k_psf3_cols(double2 *P, int ncol, int lsh, int nb, FftPlan plan, const double2 *__restrict__ tw) {
     double2 *buf = reinterpret_cast<double2 *>(lc_smem);
+    const int M = LC > 0 ? LC : plan.L, B = LC > 0 ? 1 << lsh : nb;
     const int x0 = blockIdx.x * B;
     double2 *pl = P + (size_t)blockIdx.y * M * M;
     for (int idx = threadIdx.x; idx < M * B; idx += NT) {
@@ -347,7 +361,7 @@ k_psf3_cols(double2 *P, int M, int ncol, int B, FftPlan plan, const double2 *__r
         buf[lds_col(c, i, B)] = (x0 + c < ncol) ? pl[(size_t)i * M + x0 + c] : make_double2(0.0, 0.0);
     }
     __syncthreads();
-    fft_lds<double, SIGN, NT, MAXE, true>(buf, B, 0, plan, tw);
+    psf3_fft<NT, MAXE, LC, true>(buf, B, lsh, plan, tw);
     for (int idx = threadIdx.x; idx < M * B; idx += NT) {
         const int i = idx / B, c = idx - i * B;
         if (x0 + c < ncol) pl[(size_t)i * M + x0 + c] = buf[lds_col(c, i, B)];
@@ -357,11 +371,12 @@ k_psf3_cols(double2 *P, int M, int ncol, int B, FftPlan plan, const double2 *__r
 // FP64 FFT along z of columns (k2, k3 < H), real part x scale -> khat3 in
 // column blocks of width KB: value (z, k2, k3) at ((k3 / KB) M1 + z) M KB +
 // k2 KB + k3 % KB (OT: float or double).  grid (ceil(H / B), M)
-template <typename OT, int NT, int MAXE>
+template <typename OT, int NT, int MAXE, int LC>
 __global__ void __launch_bounds__(NT)
-k_psf3_slices(const double2 *P, OT *khat3, int M1, int M, int H, int B, int KB, FftPlan plan,
+k_psf3_slices(const double2 *P, OT *khat3, int M, int H, int lsh, int nb, int KB, FftPlan plan,
               const double2 *__restrict__ tw, double scale) {
     double2 *buf = reinterpret_cast<double2 *>(lc_smem);
+    const int M1 = LC > 0 ? LC : plan.L, B = LC > 0 ? 1 << lsh : nb;
     const int k30 = blockIdx.x * B;
     const int k2 = blockIdx.y;
     for (int idx = threadIdx.x; idx < M1 * B; idx += NT) {
@@ -369,7 +384,7 @@ k_psf3_slices(const double2 *P, OT *khat3, int M1, int M, int H, int B, int KB, 
         buf[lds_col(c, z, B)] = (k30 + c < H) ? P[((size_t)z * M + k2) * M + k30 + c] : make_double2(0.0, 0.0);
     }
     __syncthreads();
-    fft_lds<double, -1, NT, MAXE, true>(buf, B, 0, plan, tw);
+    psf3_fft<NT, MAXE, LC, true>(buf, B, lsh, plan, tw);
     for (int idx = threadIdx.x; idx < M1 * B; idx += NT) {
         const int z = idx / B, c = idx - z * B;
         const int k3 = k30 + c;
@@ -432,6 +447,28 @@ PsfGroups psf_groups(const Geom3D &g, bool merge) {
 }
 } // namespace
 
+constexpr int PSF_NT = 256, PSF_ME = 16;   // line passes: up to 4096 values per block
+
+// FP64 transforms of the M1 planes of M x M: along x, then along y for kx < H
+// (only those are needed further on)
+static void psf3_xy(Ctx &c, double2 *P, int M1, int M, int H, const FftPlan &plan, const double2 *tw) {
+    const int most = std::max(1, PSF_NT * PSF_ME / M);
+    auto pass = [&](auto lc) {
+        constexpr int LC = decltype(lc)::value;
+        const int64_t nlines = (int64_t)M1 * M;
+        hipLaunchKernelGGL((k_psf3_rows<PSF_NT, PSF_ME, LC>), dim3(ceil_div(nlines, most)), dim3(PSF_NT),
+                           sizeof(double2) * lds_round(most * M), c.stream(), P, nlines, most, plan, tw);
+        LC_HIP(hipGetLastError());
+        int lsh = 0;
+        while ((2 << lsh) <= most) ++lsh;
+        const int B = LC > 0 ? 1 << lsh : most;
+        hipLaunchKernelGGL((k_psf3_cols<PSF_NT, PSF_ME, LC>), dim3(ceil_div(H, B), M1), dim3(PSF_NT),
+                           sizeof(double2) * lds_round(B * M), c.stream(), P, H, lsh, B, plan, tw);
+        LC_HIP(hipGetLastError());
+    };
+    if (!with_ct_len(M, pass)) pass(std::integral_constant<int, 0>{});
+}
+
 void geom3d_build_psf(Ctx &c, Geom3D &g, bool f64) {
     if (g.n2 != g.n3)
         throw Error(LC_EUNSUP, "3-D Toeplitz operator: recon dims n2 != n3 are not supported");
@@ -478,45 +515,35 @@ void geom3d_build_psf(Ctx &c, Geom3D &g, bool f64) {
                            g.d_rot.as<double>(), (int)g.nproj, (int)g.nrows, (int)g.ncols, M1, M, 0);
     }
     LC_HIP(hipGetLastError());
-    constexpr int NT = 256, MAXE = 16;
     const double2 *tw = c.twiddles<double>(M);
     const double2 *tw1 = c.twiddles<double>(M1);
-    // x: every row of length M
-    {
-        const int nl = std::max(1, NT * MAXE / M);
-        const int64_t nlines = (int64_t)M1 * M;
-        hipLaunchKernelGGL((k_psf3_rows<-1, NT, MAXE>), dim3(ceil_div(nlines, nl)), dim3(NT),
-                           sizeof(double2) * lds_round(nl * M), c.stream(), P, nlines, nl, plan, tw);
-        LC_HIP(hipGetLastError());
-    }
-    // y: only the columns kx < H are needed further on
-    {
-        const int B = std::max(1, NT * MAXE / M);
-        hipLaunchKernelGGL((k_psf3_cols<-1, NT, MAXE>), dim3(ceil_div(H, B), M1), dim3(NT),
-                           sizeof(double2) * lds_round(B * M), c.stream(), P, M, H, B, plan, tw);
-        LC_HIP(hipGetLastError());
-    }
+    psf3_xy(c, P, M1, M, H, plan, tw);
     // z + extraction
     {
-        const int B = std::max(1, std::min(NT * MAXE / M1, 64));
         const double scale = 1.0 / ((double)M1 * M * M * (double)g.N * (double)g.N);
-        const size_t sh = sizeof(double2) * lds_round(B * M1);
-        const dim3 grid(ceil_div(H, B), M);
         // the 3-D Toeplitz class's column block width; k3 in [H, nblk KB) stays zero
         const int KB = toep3d_block_width((int)g.N, M, f64);
         const size_t nk = (size_t)ceil_div(H, KB) * KB * M * M1;
         DBuf &kh = f64 ? g.khat3_64 : g.khat3;
         kh.alloc((f64 ? sizeof(double) : sizeof(float)) * nk);
         LC_HIP(hipMemsetAsync(kh.as(), 0, (f64 ? sizeof(double) : sizeof(float)) * nk, c.stream()));
-        if (f64) {
-            g.kB64 = KB;
-            hipLaunchKernelGGL((k_psf3_slices<double, NT, MAXE>), grid, dim3(NT), sh, c.stream(), P,
-                               g.khat3_64.as<double>(), M1, M, H, B, KB, plan1, tw1, scale);
-        } else {
-            g.kB = KB;
-            hipLaunchKernelGGL((k_psf3_slices<float, NT, MAXE>), grid, dim3(NT), sh, c.stream(), P,
-                               g.khat3.as<float>(), M1, M, H, B, KB, plan1, tw1, scale);
-        }
+        if (f64) g.kB64 = KB;
+        else g.kB = KB;
+        auto slices = [&](auto lc) {
+            constexpr int LC = decltype(lc)::value;
+            int lsh = 0, B = std::max(1, std::min(PSF_NT * PSF_ME / M1, 64));
+            while ((2 << lsh) <= B) ++lsh;
+            if (LC > 0) B = 1 << lsh;
+            const dim3 grid(ceil_div(H, B), M);
+            const size_t sh = sizeof(double2) * lds_round(B * M1);
+            if (f64)
+                hipLaunchKernelGGL((k_psf3_slices<double, PSF_NT, PSF_ME, LC>), grid, dim3(PSF_NT), sh, c.stream(), P,
+                                   g.khat3_64.as<double>(), M, H, lsh, B, KB, plan1, tw1, scale);
+            else
+                hipLaunchKernelGGL((k_psf3_slices<float, PSF_NT, PSF_ME, LC>), grid, dim3(PSF_NT), sh, c.stream(), P,
+                                   g.khat3.as<float>(), M, H, lsh, B, KB, plan1, tw1, scale);
+        };
+        if (!with_ct_len(M1, slices)) slices(std::integral_constant<int, 0>{});
         LC_HIP(hipGetLastError());
     }
     c.sync();
@@ -571,19 +598,7 @@ template <typename OT> void geom3d_kernel_hat(Ctx &c, Geom3D &g, OT *out_host) {
     constexpr int NT = 256, MAXE = 16;
     const double2 *tw = c.twiddles<double>(M);
     const double2 *tw1 = c.twiddles<double>(M1);
-    {
-        const int nl = std::max(1, NT * MAXE / M);
-        const int64_t nlines = (int64_t)M1 * M;
-        hipLaunchKernelGGL((k_psf3_rows<-1, NT, MAXE>), dim3(ceil_div(nlines, nl)), dim3(NT),
-                           sizeof(double2) * lds_round(nl * M), c.stream(), P, nlines, nl, plan, tw);
-        LC_HIP(hipGetLastError());
-    }
-    {
-        const int B = std::max(1, NT * MAXE / M);
-        hipLaunchKernelGGL((k_psf3_cols<-1, NT, MAXE>), dim3(ceil_div(H, B), M1), dim3(NT),
-                           sizeof(double2) * lds_round(B * M), c.stream(), P, M, H, B, plan, tw);
-        LC_HIP(hipGetLastError());
-    }
+    psf3_xy(c, P, M1, M, H, plan, tw);
     const size_t n = (size_t)M1 * M * H;
     cpx<OT> *tmp = reinterpret_cast<cpx<OT> *>(c.scratch(1, sizeof(cpx<OT>) * n));
     {

@@ -255,6 +255,22 @@ def test_psf3d_projection_groups_match_oracle(lc, orc64, kind, nproj):
     assert rel_l2(psf.convolve(x), ref) < 1e-12
 
 
+# PSF sizes along z and along x / y with compiled line passes (16, 32, 64, 128,
+# 192, 384) and with the run-time plan (24, 27, 36, 48), in both combinations
+@pytest.mark.parametrize("dims", [(8, 24, 24), (12, 96, 96), (14, 64, 64), (16, 18, 18), (32, 180, 180)])
+def test_psf3d_line_lengths_match_oracle(lc, orc64, dims):
+    announce(f"psf3d line lengths {dims}")
+    nproj, nrows, ncols = 7, 11, dims[2] + 1
+    th = np.arange(nproj) * (np.pi / nproj)
+    args = (th, np.full(nproj, -np.pi / 6), np.zeros(nproj))
+    psf = lc.PointSpreadFunction(lc.PolarGrid(*args, nrows, ncols), dims)
+    x = np.random.default_rng(8).random(dims)
+    ref = orc64.psf3d(*args, nrows, ncols, dims, method=0).convolve(x)
+    # as for the projection groups; phases of magnitude pi |m| < 700 (1e-13)
+    assert rel_l2(psf.convolve(x.astype(np.float32)), ref) < 1e-6
+    assert rel_l2(psf.convolve(x), ref) < 1e-11
+
+
 # a sinogram of more points than the forward projector sorts at a time (2^27):
 # the projections on either side of the boundary, and the last ones, against a
 # grid of these alone
