@@ -339,7 +339,8 @@ __global__ void k_tile_keys(const int *__restrict__ start, unsigned *__restrict_
 // most runs of a tile: its own rows of bins and the wrapped ones, in two pieces
 template <typename S> constexpr int max_runs() { return 2 * ((S::T + NU_W - 2) / CB + 2 + 2); }
 
-template <typename S, int SC> struct SpreadLds2 {
+// (a multiple of 16 bytes: every wave's tables start where 16-byte accesses may)
+template <typename S, int SC> struct alignas(16) SpreadLds2 {
     float x[TAB * TS], y[S::M][TAB * TS];
     float2 c[SC][TAB];
     int rbeg[max_runs<S>()], rpos[max_runs<S>() + 1], roff[max_runs<S>()];
@@ -474,6 +475,7 @@ __device__ __forceinline__ void spread2_tile(const float2 *__restrict__ C, float
     } else {
         // summed in wave order, through the tables' space
         static_assert(sizeof(L.x) >= sizeof(f32x4) * 2 * 64, "the exchange fits the tables");
+        static_assert(alignof(SpreadLds2<S, SC>) >= alignof(f32x4), "and starts where f32x4 may, in every wave");
 #pragma unroll
         for (int s = 0; s < SC; ++s)
 #pragma unroll

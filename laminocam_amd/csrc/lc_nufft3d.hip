@@ -441,9 +441,9 @@ k_interp3d(const float2 *__restrict__ F, float2 *__restrict__ C, const double *_
 // reordered to [wave][row / 4]), the row strides padded against bank conflicts,
 // and the point groups' rows
 constexpr int ZS = RGN + 1;
-template <typename S> struct SpreadLds {
+template <typename S> struct alignas(16) SpreadLds {
     float z[BATCH * ZS], xr[BATCH * ZS], xi[BATCH * ZS];
-    float y[BATCH * (S::ROWS + 4)];
+    alignas(16) float y[BATCH * (S::ROWS + 4)];   // read four rows at a time
     int meta[BATCH / 4];
 };
 
