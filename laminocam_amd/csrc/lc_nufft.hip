@@ -251,8 +251,12 @@ struct Foot2 {
     float fy, fx;   // rounded
 };
 __device__ __forceinline__ Foot2 foot2(double2 t, int k, const Grid2 &g) {   // t: (cos, sin), k: radial index
-    const double r = ((double)k + 0.5) * g.dr - M_PI;
-    const double gx = 0.5 * g.nf + g.sc * r * t.x, gy = 0.5 * g.nf + g.sc * r * t.y;
+    // the fused multiply-adds are explicit, so the kernel that sorts the points
+    // and the one that spreads them take the same corner: positions that are
+    // whole numbers up to rounding are common (angles 0 and pi / 2 with nrad = N),
+    // and one on the two sides of the periodic edge would be lost
+    const double r = __builtin_fma((double)k + 0.5, g.dr, -M_PI);
+    const double gx = __builtin_fma(g.sc * r, t.x, 0.5 * g.nf), gy = __builtin_fma(g.sc * r, t.y, 0.5 * g.nf);
     const double hw = 0.5 * NU_W;
     Foot2 f;
     f.lx = (int)ceil(gx - hw);

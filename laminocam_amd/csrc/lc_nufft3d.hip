@@ -70,14 +70,21 @@ struct Grid3 {
     int mask;           // 1: drop points with any |coordinate| > pi
 };
 
+// The operations of a point's position are written out, with every fused
+// multiply-add explicit: positions that are whole numbers up to rounding are
+// common (an untilted scan with ncols = n has no others along x), and kernels
+// that let the compiler contract these products each in its own way took
+// different corners for them, on the two sides of the periodic edge at worst.
+__device__ __forceinline__ double lattice_coord(int k, double step) {   // (k + 1/2) step - pi
+    return __builtin_fma((double)k + 0.5, step, -M_PI);
+}
 __device__ __forceinline__ void point3(const double *rot, int p, int j, int k, const Grid3 &g,
                                        double &x, double &y, double &z) {
     const double *r = rot + 6 * (int64_t)p;
-    const double qx = ((double)k + 0.5) * g.dX - M_PI;
-    const double qy = ((double)j + 0.5) * g.dY - M_PI;
-    x = qx * r[0] + qy * r[3];
-    y = qx * r[1] + qy * r[4];
-    z = qx * r[2] + qy * r[5];
+    const double qx = lattice_coord(k, g.dX), qy = lattice_coord(j, g.dY);
+    x = __builtin_fma(qy, r[3], qx * r[0]);
+    y = __builtin_fma(qy, r[4], qx * r[1]);
+    z = __builtin_fma(qy, r[5], qx * r[2]);
 }
 
 __device__ __forceinline__ bool inside_pi(double x, double y, double z) {
@@ -148,9 +155,9 @@ __device__ __forceinline__ Corner3 corner3(const double *rot, int p, int j, int 
     point3(rot, p, j, k, g, x, y, z);
     c.ok = !g.mask || inside_pi(x, y, z);
     const double hw = 0.5 * W3;
-    c.gz = 0.5 * g.nf[0] + z * (g.nf[0] / (2.0 * M_PI));
-    c.gy = 0.5 * g.nf[1] + y * (g.nf[1] / (2.0 * M_PI));
-    c.gx = 0.5 * g.nf[2] + x * (g.nf[2] / (2.0 * M_PI));
+    c.gz = __builtin_fma(z, g.nf[0] / (2.0 * M_PI), 0.5 * g.nf[0]);
+    c.gy = __builtin_fma(y, g.nf[1] / (2.0 * M_PI), 0.5 * g.nf[1]);
+    c.gx = __builtin_fma(x, g.nf[2] / (2.0 * M_PI), 0.5 * g.nf[2]);
     c.lz = (int)ceil(c.gz - hw);
     c.ly = (int)ceil(c.gy - hw);
     c.lx = (int)ceil(c.gx - hw);
@@ -229,8 +236,7 @@ __global__ void k_phase_shift3d(float2 *__restrict__ C, const double *__restrict
     const int64_t pj = i / g.ncols;
     const int kk = (int)(i - pj * g.ncols);
     const int pp = (int)(pj / g.nrows), jj = (int)(pj - (int64_t)pp * g.nrows);
-    const double qx = ((double)kk + 0.5) * g.dX - M_PI;
-    const double qy = ((double)jj + 0.5) * g.dY - M_PI;
+    const double qx = lattice_coord(kk, g.dX), qy = lattice_coord(jj, g.dY);
     double s, c;
     sincos(qx * shifts[2 * pp] + qy * shifts[2 * pp + 1], &s, &c);
     const float cr = (float)c, si = (float)-s;
@@ -266,9 +272,10 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
 }
 constexpr int BATCH = 128;                  // points per table; two threads fill a point's slots
 
-// footprint corner of a point relative to its bin, and the offset of its cell
-// W3 / 2 from the point, in [0, 1), per axis (the weights' arguments are exact
-// integers away from it: the largest weights get the smallest rounding)
+// footprint corner of a point relative to its bin (inside it: corner3 gives
+// every kernel the same corner), and the offset of its cell W3 / 2 from the
+// point, in [0, 1), per axis (the weights' arguments are exact integers away
+// from it: the largest weights get the smallest rounding)
 template <typename T> struct Foot {
     int t[3];
     T f[3];
@@ -301,9 +308,6 @@ __device__ __forceinline__ void axis_weights(int t, T f, int h, float beta, F &&
 }
 // smallest and largest corner row of the groups of G consecutive lanes
 template <int G> __device__ __forceinline__ void group_rows(int ty, bool ok, int &lo, int &hi) {
-    // (a corner on a bin's edge may round to the bin beside it: its weights are
-    // then dropped where they are smallest, and the rows stay in range)
-    ty = min(max(ty, 0), 63);
     lo = ok ? ty : 127;
     hi = ok ? ty : 0;
 #pragma unroll

@@ -336,6 +336,39 @@ def test_projectors3d_bin_edges_match_oracle(lc, orc64, dims, nproj, nrows, ncol
         ctx.close()
 
 
+# Points on the lattice of the fine grid: without a tilt, with ncols = n and a
+# fine grid of 2 n cells, every point's position along x is an odd whole number
+# and that of detector column 1 is 3, whose footprint starts at the periodic
+# edge (cell -1 or 0, as the FP64 position rounds); tilted, a detector row does
+# so where theta = 90 degrees and nrows = 3 n1.  Every kernel has to take the same
+# corner, or the whole column or row is lost (4e-3 and more of the norm).
+LATTICE = [((8, 96, 96), 16, 16, 96, 0.0), ((8, 128, 128), 24, 32, 128, 0.0), ((6, 288, 288), 8, 12, 288, 0.0),
+           ((8, 384, 384), 6, 16, 384, 0.0), ((32, 128, 128), 50, 128, 128, 0.0), ((16, 128, 128), 4, 48, 128, -30.0)]
+
+
+@pytest.mark.parametrize("dims,nproj,nrows,ncols,tilt", LATTICE)
+def test_projectors3d_lattice_points_match_oracle(lc, orc64, dims, nproj, nrows, ncols, tilt):
+    announce(f"projectors3d lattice points dims={dims} det=({nrows},{ncols}) tilt={tilt}")
+    rng = np.random.default_rng(dims[2] + nrows)
+    th, ga, be = lamino_angles(nproj, tilt)
+    g = lc.PolarGrid(th, ga, be, nrows, ncols)
+    vol = rng.standard_normal(dims).astype(np.float32)
+    proj = rng.standard_normal((nproj, nrows, ncols)).astype(np.float32)
+    # the projectors' FP32 error is about 5e-7
+    assert rel_l2(lc.forward(vol, g), orc64.forward3d(vol, th, ga, be, nrows, ncols, tol=1e-12)) < 5e-6
+    xr = orc64.backproj3d(proj, th, ga, be, dims, tol=1e-12)
+    sr = orc64.sysmat3d_nufft(vol, th, ga, be, nrows, ncols, tol=1e-12)
+    ctx = lc.Context(0)
+    try:
+        psf = lc.PointSpreadFunction(g, dims, ctx=ctx, lazy=True)
+        for shape in range(3):
+            ctx.set_tuning3d(psf, shape)
+            assert rel_l2(lc.backproj(proj, g, dims, ctx=ctx), xr) < 5e-6
+            assert rel_l2(lc.sysmat(vol, g, ctx=ctx), sr) < 5e-6
+    finally:
+        ctx.close()
+
+
 def test_backproj3d_bin_shapes_and_autotune(lc, orc64):
     # every compiled bin shape of the spread (0: 4x4x8, 1: 8x4x4, 2: 8x8x8
     # corner cells) gives the oracle's back-projection, deterministically;

@@ -169,6 +169,21 @@ def test_projectors_tile_edges_match_oracle(lc, orc64, N, nang, nrad, ns):
         ctx.close()
 
 
+# points on the lattice of the fine grid (2 N cells, nrad = N, rows along the
+# axes): one per row at cell 3, whose footprint starts at the periodic edge and
+# is lost if the sort and the spread take its corner on different sides of it
+@pytest.mark.parametrize("N", [48, 96, 128, 384])
+def test_projectors_lattice_points_match_oracle(lc, orc64, N):
+    announce(f"projector lattice points N={N}")
+    rng = np.random.default_rng(N)
+    th = np.arange(8) * np.pi / 4
+    g = lc.PolarGrid2D(th, N)
+    vol, sino = rng.standard_normal((2, N, N)), rng.standard_normal((2, 8, N))
+    # the projectors' own FP32 error is about 5e-7
+    assert rel_l2(lc.forward2d(vol, g), orc64.forward2d(vol, th, N, tol=1e-12)) < 5e-6
+    assert rel_l2(lc.backproj2d(sino, g, (2, N, N)), orc64.backproj2d(sino, th, N, tol=1e-12)) < 5e-6
+
+
 def test_backproj2d_bin_shapes_and_autotune(lc, orc64):
     # both compiled bin sizes of the sorted-bin spread (16 and 32 corner
     # cells) give the oracle's back-projection; a slice is the same alone and
