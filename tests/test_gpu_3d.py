@@ -336,6 +336,27 @@ def test_projectors3d_bin_edges_match_oracle(lc, orc64, dims, nproj, nrows, ncol
         ctx.close()
 
 
+# the forward projector interpolates few points in their own order and more in
+# sorted order: (recon dims, nproj, nrows, ncols) with fine grids of 16 .. 81 cells
+# per axis (two, three and more bins) on either side of that line, 450000 points
+# and two for every bin, with masked points in both
+FORWARD_LINE = [((6, 16, 16), 331, 34, 39), ((6, 16, 16), 331, 34, 41), ((9, 13, 18), 400, 31, 37),
+                ((12, 16, 40), 400, 31, 37), ((13, 27, 24), 300, 41, 38)]
+
+
+@pytest.mark.parametrize("dims,nproj,nrows,ncols", FORWARD_LINE)
+def test_forward3d_sorted_and_unsorted_match_oracle(lc, orc64, dims, nproj, nrows, ncols):
+    announce(f"forward3d line dims={dims} points={nproj * nrows * ncols}")
+    vol = np.random.default_rng(nproj + ncols).random(dims)
+    th, ga, be = lamino_angles(nproj, -30.0)
+    y = lc.forward(vol, lc.PolarGrid(th, ga, be, nrows, ncols))
+    # the projectors' FP32 error is about 5e-7
+    assert rel_l2(y, orc64.forward3d(vol, th, ga, be, nrows, ncols, tol=1e-12)) < 5e-6
+    # the first projections alone are few points: the other kernel or the same one
+    few = lc.forward(vol, lc.PolarGrid(th[:5], ga[:5], be[:5], nrows, ncols))
+    assert rel_l2(few, y[:5]) < 1e-6
+
+
 # Points on the lattice of the fine grid: without a tilt, with ncols = n and a
 # fine grid of 2 n cells, every point's position along x is an odd whole number
 # and that of detector column 1 is 3, whose footprint starts at the periodic
