@@ -524,13 +524,17 @@ k_spread2d(const float2 *__restrict__ C, float2 *__restrict__ fine, const double
 }
 
 // ---------------------------------------------------------------------------
-// Type-2 interpolation.  A wave takes 64 consecutive points of a slice: lane l
+// Type-2 interpolation.  A wave takes PW consecutive points of a slice: lane l
 // first finds the footprint and the weights of point l, then the wave takes
 // the points two at a time, 32 lanes each: 8 rows x 4 lanes of two adjacent
 // cells, so a footprint row is one 64-byte piece read by 16-byte loads.  (One
 // lane per point reads the same cells as 64 8-byte loads whose lanes all fall
 // on different cache lines.)  The 32 lanes are summed in a fixed order.
 // 4 slices of 511^2, 360 x 511 points: 38 us against 201 us with a lane per point.
+// PW is 64, or 16 where that leaves too few waves (type2; the same sums): a
+// forward projection of 64^2 from 60 angles 52.6 -> 43.9 us (50.6 with a lane
+// per point), 512^2 from 360 66.1 -> 58.8 us (2880 waves of 64), but two such
+// slices 68.4 -> 72.1 us (5760).
 // ---------------------------------------------------------------------------
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(8)));   // two cells
 
@@ -545,6 +549,7 @@ __device__ __forceinline__ float sum32(float v) {
 }
 
 constexpr int IW = 4;                       // waves per interpolation block
+template <int PW>                           // points of a wave
 __global__ void __launch_bounds__(64 * IW)
 k_interp2d(const float2 *__restrict__ fine, float2 *__restrict__ C, const double2 *__restrict__ cs, Grid2 g,
            int npts) {
@@ -553,7 +558,7 @@ k_interp2d(const float2 *__restrict__ fine, float2 *__restrict__ C, const double
     __shared__ int2 tpos[IW][64];
     __shared__ float2 res[IW][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int base = (blockIdx.x * IW + wave) * 64;
+    const int base = (blockIdx.x * IW + wave) * PW;
     if (base >= npts) return;   // whole wave (no barrier below)
     float *X = tx[wave], *Y = ty[wave];
     const int p = base + lane;
@@ -565,7 +570,7 @@ k_interp2d(const float2 *__restrict__ fine, float2 *__restrict__ C, const double
         Y[lane * YW + d] = es_kernel((float)((double)(d - NU_W / 2) + f.dy) * ihw, g.beta);
     }
     tpos[wave][lane] = make_int2(f.lx, f.ly);
-    const bool wrap = __ballot(f.lx + NU_W > g.nf) != 0;   // a footprint row crosses the edge
+    const bool wrap = __ballot(lane < PW && f.lx + NU_W > g.nf) != 0;   // a footprint row crosses the edge
     wave_lds_fence();
     const float2 *fs = fine + (int64_t)blockIdx.y * g.nf * g.nf;
     const int half = lane >> 5, r = (lane >> 2) & 7, c2 = 2 * (lane & 3);
@@ -590,13 +595,13 @@ k_interp2d(const float2 *__restrict__ fine, float2 *__restrict__ C, const double
         if ((lane & 31) == 31) res[wave][q] = make_float2(re, im);
     };
     if (wrap) {
-        for (int i = 0; i < 32; ++i) point(2 * i + half, std::true_type{});
+        for (int i = 0; i < PW / 2; ++i) point(2 * i + half, std::true_type{});
     } else {
 #pragma unroll 4
-        for (int i = 0; i < 32; ++i) point(2 * i + half, std::false_type{});
+        for (int i = 0; i < PW / 2; ++i) point(2 * i + half, std::false_type{});
     }
     wave_lds_fence();
-    if (p < npts) C[(int64_t)blockIdx.y * npts + p] = res[wave][lane];
+    if (lane < PW && p < npts) C[(int64_t)blockIdx.y * npts + p] = res[wave][lane];
 }
 
 // ---------------------------------------------------------------------------
@@ -1111,8 +1116,14 @@ void type2(Ctx &c, const Geom2D &g, const NuWork &w, const float *vol, int ns) {
         hipLaunchKernelGGL((k_fine_rows_t2<NU_NT, NU_ME, 0>), dim3(ceil_div(nf, nl), ns), dim3(NU_NT), shr,
                            c.stream(), w.V, w.F, nf, N, nl, u.plan_nf, tw);
     LC_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_interp2d, dim3(ceil_div(npts, 64 * IW), ns), dim3(64 * IW), 0, c.stream(), w.F, w.C,
-                       g.nu.cs.as<double2>(), grid2(g), (int)npts);
+    auto interp = [&](auto pw) {
+        constexpr int PW = decltype(pw)::value;
+        hipLaunchKernelGGL(k_interp2d<PW>, dim3(ceil_div(npts, PW * IW), ns), dim3(64 * IW), 0, c.stream(), w.F, w.C,
+                           g.nu.cs.as<double2>(), grid2(g), (int)npts);
+    };
+    // below four waves per SIMD the time is that of a wave's loop over its points
+    if ((int64_t)ceil_div(npts, 64) * ns < 4096) interp(std::integral_constant<int, 16>{});
+    else interp(std::integral_constant<int, 64>{});
     LC_HIP(hipGetLastError());
 }
 

@@ -169,6 +169,22 @@ def test_projectors_tile_edges_match_oracle(lc, orc64, N, nang, nrad, ns):
         ctx.close()
 
 
+# the interpolation's two numbers of points per wave, on either side of the line
+# between them (4096 waves of 64 points: 63 and 64 stacked slices of 65 waves, the
+# last one partial); a point's sum is the same with both
+def test_forward2d_small_and_large_stacks_agree(lc, orc64):
+    announce("forward2d waves")
+    N, nang, nrad = 16, 134, 31
+    th = uniform_theta(nang)
+    g = lc.PolarGrid2D(th, nrad)
+    vol = np.random.default_rng(3).random((64, N, N))
+    y = lc.forward2d(vol, g)
+    # the projectors' own FP32 error is about 5e-7
+    assert rel_l2(y, orc64.forward2d(vol, th, nrad, tol=1e-12)) < 5e-6
+    assert np.array_equal(lc.forward2d(vol[1:], g), y[1:])
+    assert np.array_equal(lc.forward2d(vol[5:6], g), y[5:6])
+
+
 # points on the lattice of the fine grid (2 N cells, nrad = N, rows along the
 # axes): one per row at cell 3, whose footprint starts at the periodic edge and
 # is lost if the sort and the spread take its corner on different sides of it
