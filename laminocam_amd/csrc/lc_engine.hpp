@@ -57,7 +57,8 @@ void bluestein_tables(int n, int L, std::vector<std::complex<double>> &chirp,
 
 // NUFFT projectors on device buffers (src/projection.cpp:146-182):
 // forward2d: vol (ns x N x N) -> sino (ns x nang x nrad); backproj2d: reverse
-void nufft2d_init(Ctx &c, Geom2D &g);
+// own_work: on working space of its own, freed on return, in place of c's scratch
+void nufft2d_init(Ctx &c, Geom2D &g, bool own_work = false);
 void forward2d_dev(Ctx &c, Geom2D &g, const float *vol, float *sino, int ns);
 void backproj2d_dev(Ctx &c, Geom2D &g, const float *sino, float *vol, int ns);
 // sysmat2d(x, grid) = Re(T1(T2 x)) / nrad (src/gradient.cpp:59-69)
@@ -262,6 +263,7 @@ int nufft3d_num_shapes();
 int nufft3d_autotune(Ctx &c, Geom3D &g, double *best_ms);
 // the same for the 2-D spread, per fine-grid size, timed on nslices slices
 int nufft2d_num_shapes();
+size_t nufft2d_order_bytes(int64_t nang, int64_t nrad, int nf);
 int nufft2d_autotune(Ctx &c, Geom2D &g, int nslices, double *best_ms);
 // An odd image size N needs column blocks of at least two columns (the block
 // copies move pairs of complex values).  A column shape too small for 2 M

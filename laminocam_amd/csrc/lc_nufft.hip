@@ -812,9 +812,8 @@ void bluestein_tables(int n, int L, std::vector<std::complex<double>> &chirp, st
     for (auto &v : bhat) v /= (double)L;
 }
 
-// (cos, sin) of every projection angle, FP64, once per geometry: the spread
-// tests every angle against every tile and the interpolation reads one per
-// point
+// (cos, sin) of every projection angle, FP64, once per geometry: the sort, the
+// spread and the interpolation read the point's angle's
 __global__ void k_angle_table(const double *__restrict__ theta, double2 *__restrict__ cs, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {
@@ -864,9 +863,17 @@ Grid2 grid2(const Geom2D &g) {
     return s;
 }
 
+int tiles_of(int nf, int shape) {
+    int n = 0;
+    with_shape2(shape, [&](auto sh) { n = ceil_div(nf, decltype(sh)::T) * ceil_div(nf, TX); });
+    return n;
+}
+
 // the points sorted by corner bin, the bins' starts, and per tile shape the
-// tiles, fullest first
-void sort_points(Ctx &c, Geom2D &g) {
+// tiles, fullest first.  The sort's working space, about 20 bytes per point, is
+// the projections' scratch, which the caller's own call is about to use, or
+// (own_work) freed again: a server's main context never projects
+void sort_points(Ctx &c, Geom2D &g, bool own_work) {
     Nufft2D &u = g.nu;
     const Grid2 s = grid2(g);
     LC_REQUIRE(g.nang * g.nrad < (int64_t)1 << 31, "2-D projector: 2^31 or more points per slice");
@@ -874,20 +881,21 @@ void sort_points(Ctx &c, Geom2D &g) {
     int bits = 1;
     while ((1 << bits) < nbins) ++bits;
     int tiles = 0;
-    for (int i = 0; i < N_SHAPES2; ++i)
-        with_shape2(i, [&](auto sh) {
-            u.tiles_off[i] = tiles;
-            u.ntiles[i] = ceil_div(s.nf, decltype(sh)::T) * ceil_div(s.nf, TX);
-            tiles += u.ntiles[i];
-        });
+    for (int i = 0; i < N_SHAPES2; ++i) {
+        u.tiles_off[i] = tiles;
+        u.ntiles[i] = tiles_of(s.nf, i);
+        tiles += u.ntiles[i];
+    }
     const size_t bK = al256(sizeof(unsigned) * (size_t)std::max(npts, tiles));
     size_t tb = 0, tt = 0;
     LC_HIP(rocprim::radix_sort_pairs(nullptr, tb, (unsigned *)nullptr, (unsigned *)nullptr, (unsigned *)nullptr,
                                      (unsigned *)nullptr, (size_t)npts, 0, bits, c.stream()));
     LC_HIP(rocprim::radix_sort_pairs(nullptr, tt, (unsigned *)nullptr, (unsigned *)nullptr, (int *)nullptr,
                                      (int *)nullptr, (size_t)tiles, 0, 31, c.stream()));
-    // working space: what the first projection allocates anyway
-    char *ws = reinterpret_cast<char *>(c.scratch(3, 3 * bK + al256(std::max(tb, tt)) + sizeof(int) * N_SHAPES2));
+    const size_t need = 3 * bK + al256(std::max(tb, tt)) + sizeof(int) * N_SHAPES2;
+    DBuf own;
+    if (own_work) own.alloc(need);
+    char *ws = own_work ? own.as<char>() : reinterpret_cast<char *>(c.scratch(3, need));
     unsigned *ka = reinterpret_cast<unsigned *>(ws), *kb = reinterpret_cast<unsigned *>(ws + bK),
              *va = reinterpret_cast<unsigned *>(ws + 2 * bK);
     void *tmp = ws + 3 * bK;
@@ -919,7 +927,15 @@ void sort_points(Ctx &c, Geom2D &g) {
 }
 } // namespace
 
-void nufft2d_init(Ctx &c, Geom2D &g) {
+// device bytes of the points' order and the tiles that a geometry keeps
+size_t nufft2d_order_bytes(int64_t nang, int64_t nrad, int nf) {
+    const size_t nb = ceil_div(nf, CB);
+    size_t b = al256(sizeof(unsigned) * (size_t)(nang * nrad)) + sizeof(int) * (nb * nb + 1);
+    for (int i = 0; i < N_SHAPES2; ++i) b += sizeof(int) * (size_t)tiles_of(nf, i);
+    return b;
+}
+
+void nufft2d_init(Ctx &c, Geom2D &g, bool own_work) {
     Nufft2D &u = g.nu;
     u.cs.alloc(sizeof(double2) * g.nang);
     hipLaunchKernelGGL(k_angle_table, dim3(ceil_div(g.nang, 256)), dim3(256), 0, c.stream(),
@@ -941,7 +957,7 @@ void nufft2d_init(Ctx &c, Geom2D &g) {
     u.det_fast = g.nrad <= DET_FFT_MAX && fft_make_plan((int)g.nrad, u.plan_det);
     u.det_blue = !u.det_fast && 2 * g.nrad - 1 <= DET_FFT_MAX;
     if (u.det_blue) det_blue_init(c, u, (int)g.nrad);
-    sort_points(c, g);
+    sort_points(c, g, own_work);
     u.ready = true;
 }
 

@@ -35,7 +35,8 @@ double now_s() {
 } // namespace
 
 // device bytes one request holds while it runs (batch vectors, Toeplitz
-// intermediates, Split-Bregman fields, back-projection scratch)
+// intermediates, Split-Bregman fields, back-projection scratch, the order of
+// its geometry's points)
 size_t request_bytes(const ServerRequest &r) {
     int64_t N, ns, M, H, extra = 0, bp = 0;
     if (r.g3) {
@@ -65,7 +66,9 @@ size_t request_bytes(const ServerRequest &r) {
         H = g.H;
         if (r.has_sino) {
             const int64_t nf = g.nu.ready ? g.nu.nf : nufft2d_fine_n(g.N);
-            bp = 4 * ns * g.nang * g.nrad + 8 * ns * (g.nang * g.nrad + nf * nf + nf * N);
+            // (the order is the geometry's: charged to every request on it)
+            bp = 4 * ns * g.nang * g.nrad + 8 * ns * (g.nang * g.nrad + nf * nf + nf * N) +
+                 (int64_t)nufft2d_order_bytes(g.nang, g.nrad, (int)nf);
         }
     }
     const int64_t n = ns * N * N;
@@ -131,7 +134,7 @@ uint64_t Server::submit(std::unique_ptr<ServerRequest> r) {
                 if (r->has_sino && !r->g3->nu.ready) nufft3d_init(main_, *r->g3);
             } else {
                 if (!r->g2->psf_ready) geom2d_build_psf(main_, *r->g2);
-                if (r->has_sino && !r->g2->nu.ready) nufft2d_init(main_, *r->g2);
+                if (r->has_sino && !r->g2->nu.ready) nufft2d_init(main_, *r->g2, true);
             }
             main_.sync();
         }

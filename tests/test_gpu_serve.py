@@ -1,6 +1,7 @@
 """Reconstruction server (lc_server_*): continuous batching with HBM-budget
 admission.  Every result must be bitwise the result of solving that request
 alone through the single-problem entry points, whatever else ran with it."""
+import ctypes as C
 import threading
 import time
 
@@ -300,3 +301,33 @@ def test_request_bytes_is_what_admission_charges(lc, problems):
     small = ReconParams(regularizer=Regularizer.SPLIT_BREGMAN, recon_dims=(21, 511, 511))
     huge = ReconParams(regularizer=Regularizer.SPLIT_BREGMAN, recon_dims=(4096, 4096, 4096))
     assert lc.volume_fits_one_gpu(small) and not lc.volume_fits_one_gpu(huge)
+
+
+def test_server_accounts_for_a_geometrys_points(lc):
+    # the order of a 2-D geometry's points (4 bytes each) belongs to a request's
+    # charge, and what submit needs to make it is given back: after the request
+    # the device holds no more than the order and small tables
+    announce("server geometry tables")
+    hip = C.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    N, nang, nrad = 32, 2048, 4096
+    npts, nf = nang * nrad, 2 * N
+    y = np.random.default_rng(1).standard_normal((1, nang, nrad)).astype(np.float32)
+    small = lc.PointSpreadFunction2D(lc.PolarGrid2D(np.arange(60) * np.pi / 60, N), N)
+    with lc.Server(hbm_budget=8 << 30, lanes=1) as srv:
+        srv.result(srv.submit(small, sino=y[:, :60, :N].copy(), max_iter=1), timeout=60.0)
+    psf = lc.PointSpreadFunction2D(lc.PolarGrid2D(np.arange(nang) * np.pi / nang, nrad), N)
+    free0 = free_bytes()
+    with lc.Server(hbm_budget=8 << 30, lanes=1) as srv:
+        # sinogram, spectra, fine grid and line passes, and the order
+        more = srv.request_bytes(psf, sino=y) - srv.request_bytes(psf, rhs=np.zeros((1, N, N), np.float32))
+        assert more >= 4 * npts + 8 * (npts + nf * nf + nf * N) + 4 * npts
+        srv.result(srv.submit(psf, sino=y, max_iter=1), timeout=60.0)
+    held = free0 - free_bytes()
+    print(f"held {held / 2**20:.1f} MiB, order {4 * npts / 2**20:.1f} MiB")
+    assert held <= 4 * npts + (24 << 20)
