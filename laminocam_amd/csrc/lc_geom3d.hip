@@ -271,8 +271,12 @@ __device__ __forceinline__ void dirichlet_run(double (&s)[RUN], double tc, doubl
 // tables' uniform addresses make them scalar loads.  The PSF of the
 // laminography shape (64 x 1536^2, 360 projections of 89 x 721) takes 7.5 ms
 // against 12.0 ms with the sines by recurrence in runs of 16 and 47.8 ms with
-// both factors per projection.
-template <int RUN>
+// both factors per projection.  MANY: several groups, whose sums meet in
+// registers (added up in P, every group but the first reads and writes all of
+// it): the PSF of 21 x 359^2 from 60 projections takes 1.3 ms with 30 tilts
+// (14.4 through P) and 1.9 ms with 60, against 2.3 ms by k_psf3d_gen, which
+// only at 12 projections of 12 tilts is no slower (0.33 against 0.35 ms).
+template <int RUN, bool MANY>
 __global__ void __launch_bounds__(256, RUN == 32 ? 3 : 4)
 k_psf3d_gen_grouped(double2 *__restrict__ P, const double4 *__restrict__ v, const int *__restrict__ goff,
                     const double *__restrict__ gu, const double4 *__restrict__ tab, int ngroups, int nrows, int ncols,
@@ -289,7 +293,17 @@ k_psf3d_gen_grouped(double2 *__restrict__ P, const double4 *__restrict__ v, cons
     const double my = (double)(iy < (M + 1) / 2 ? iy : iy - M);
     const double mc = (double)(x0 - M / 2) + 0.5 * (RUN - 1);   // the run's middle
     const int nv = goff[ngroups];
-    for (int q = 0; q < ngroups; ++q) {
+    double t[MANY ? RUN : 1];   // the groups so far
+#pragma unroll
+    for (int j = 0; j < RUN; ++j)
+        if constexpr (MANY) t[j] = 0.0;
+    const bool mirror = iz >= 1 && 2 * iz < M1;
+    auto put = [&](int j, double val) {
+        const int m = x0 + j - M / 2, ix = m < 0 ? m + M : m;
+        P[((size_t)iz * M + iy) * M + ix] = make_double2(val, 0.0);
+        if (mirror) P[((size_t)(M1 - iz) * M + (M - iy) % M) * M + (M - ix) % M] = make_double2(val, 0.0);
+    };
+    for (int q = 0; q < (MANY ? ngroups : 1); ++q) {
         double s[RUN];
 #pragma unroll
         for (int j = 0; j < RUN; ++j) s[j] = 0.0;
@@ -301,16 +315,16 @@ k_psf3d_gen_grouped(double2 *__restrict__ P, const double4 *__restrict__ v, cons
         const double ux = gu[3 * q];
         dirichlet_run<RUN, true>(s, mc * ux + my * gu[3 * q + 1] + mz * gu[3 * q + 2], ux, ncols, inv_c,
                                  tab + (size_t)(nv + q) * (RUN / 2), 1.0, thr);
-        const bool mirror = iz >= 1 && 2 * iz < M1;
 #pragma unroll
         for (int j = 0; j < RUN; ++j) {
-            if (x0 + j >= M) break;
-            const int m = x0 + j - M / 2, ix = m < 0 ? m + M : m;
-            double2 *p = P + ((size_t)iz * M + iy) * M + ix;
-            const double t = s[j] + (q ? p->x : 0.0);
-            *p = make_double2(t, 0.0);
-            if (mirror) P[((size_t)(M1 - iz) * M + (M - iy) % M) * M + (M - ix) % M] = make_double2(t, 0.0);
+            if constexpr (MANY) t[j] += s[j];
+            else if (x0 + j < M) put(j, s[j]);
         }
+    }
+    if constexpr (MANY) {
+#pragma unroll
+        for (int j = 0; j < RUN; ++j)
+            if (x0 + j < M) put(j, t[j]);
     }
 }
 
@@ -480,11 +494,12 @@ void geom3d_build_psf(Ctx &c, Geom3D &g, bool f64) {
     const int64_t threads = (int64_t)(M1 / 2 + 1) * M * ceil_div(M, P3_RUN);
     const PsfGroups gr = psf_groups(g, !f64);
     DBuf dgr;   // the runs' tables, v, u, off
-    if (gr.off.size() > 1 && 2 * (gr.off.size() - 1) <= (size_t)g.nproj) {
+    if (gr.off.size() > 1) {
         const int ng = (int)gr.off.size() - 1, nv = (int)gr.v.size();
         // runs of 32 share the middle's sines among more terms; runs of 16 where
-        // those would leave the chip below three waves per SIMD
-        const int run = (int64_t)(M1 / 2 + 1) * M * ceil_div(M, 32) >= 3 * 1024 * 64 ? 32 : 16;
+        // those would leave the chip below three waves per SIMD, and for several
+        // groups, whose sums would not fit the registers beside 32 terms
+        const int run = ng == 1 && (int64_t)(M1 / 2 + 1) * M * ceil_div(M, 32) >= 3 * 1024 * 64 ? 32 : 16;
         const size_t bv = sizeof(double4) * gr.v.size(), bt = sizeof(double4) * (size_t)(nv + ng) * (run / 2),
                      bu = sizeof(double) * gr.u.size(), bo = sizeof(int) * gr.off.size();
         std::vector<char> host(bv + bu + bo);
@@ -499,17 +514,19 @@ void geom3d_build_psf(Ctx &c, Geom3D &g, bool f64) {
         const double4 *dv = reinterpret_cast<const double4 *>(d + bt);
         const double *du = reinterpret_cast<const double *>(d + bt + bv);
         const int *doff = reinterpret_cast<const int *>(d + bt + bv + bu);
-        auto gen = [&](auto run_c) {
+        auto gen = [&](auto run_c, auto many) {
             constexpr int RUN = decltype(run_c)::value;
             hipLaunchKernelGGL(k_psf3d_steps<RUN>, dim3(ceil_div((int64_t)(nv + ng) * (RUN / 2), 256)), dim3(256), 0,
                                c.stream(), dt, dv, nv, du, ng, (int)g.nrows, (int)g.ncols);
             LC_HIP(hipGetLastError());
             const int64_t n = (int64_t)(M1 / 2 + 1) * M * ceil_div(M, RUN);
-            hipLaunchKernelGGL(k_psf3d_gen_grouped<RUN>, dim3(ceil_div(n, 256)), dim3(256), 0, c.stream(), P, dv, doff,
-                               du, dt, ng, (int)g.nrows, (int)g.ncols, M1, M, f64 ? 1e-3 : 1e-4);
+            constexpr bool MANY = decltype(many)::value;
+            hipLaunchKernelGGL((k_psf3d_gen_grouped<RUN, MANY>), dim3(ceil_div(n, 256)), dim3(256), 0, c.stream(), P, dv, doff, du, dt, ng,
+                               (int)g.nrows, (int)g.ncols, M1, M, f64 ? 1e-3 : 1e-4);
         };
-        if (run == 32) gen(std::integral_constant<int, 32>{});
-        else gen(std::integral_constant<int, 16>{});
+        if (ng > 1) gen(std::integral_constant<int, 16>{}, std::true_type{});
+        else if (run == 32) gen(std::integral_constant<int, 32>{}, std::false_type{});
+        else gen(std::integral_constant<int, 16>{}, std::false_type{});
     } else {
         hipLaunchKernelGGL(k_psf3d_gen, dim3(ceil_div(threads, 256)), dim3(256), 0, c.stream(), P,
                            g.d_rot.as<double>(), (int)g.nproj, (int)g.nrows, (int)g.ncols, M1, M, 0);

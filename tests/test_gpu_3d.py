@@ -229,9 +229,9 @@ def test_backproj3d_mid_size_matches_oracle(lc, orc64, dims, nproj, nrows, ncols
 
 # tilts per projection and the span of theta: one tilt over a full turn (opposite
 # projections coincide: even and odd counts), two tilts, a tilt per projection
-# (no two share a column direction), and repeated angles
-@pytest.mark.parametrize("kind,nproj", [("turn", 24), ("turn", 25), ("two", 24), ("each", 11), ("repeat", 12),
-                                        ("beta", 18)])
+# (no two share a column direction) and for every two, and repeated angles
+@pytest.mark.parametrize("kind,nproj", [("turn", 24), ("turn", 25), ("two", 24), ("each", 11), ("pairs", 26),
+                                        ("repeat", 12), ("beta", 18)])
 def test_psf3d_projection_groups_match_oracle(lc, orc64, kind, nproj):
     announce(f"psf3d groups {kind} nproj={nproj}")
     dims, nrows, ncols = (5, 22, 22), 9, 21
@@ -241,6 +241,8 @@ def test_psf3d_projection_groups_match_oracle(lc, orc64, kind, nproj):
         ga[nproj // 2:] = 0.3
     elif kind == "each":
         ga = np.linspace(-0.6, 0.2, nproj)
+    elif kind == "pairs":
+        ga = np.linspace(-0.6, 0.2, nproj // 2)[np.arange(nproj) % (nproj // 2)]
     elif kind == "repeat":
         th = np.repeat(th[::3], 3)
     elif kind == "beta":
@@ -288,15 +290,16 @@ def test_forward3d_ranges_match_a_small_grid(lc):
     assert rel_l2(all_of, few) < 1e-6   # the same FP32 operations per point
 
 
-# a PSF large enough for runs of 32 values (the sizes above take 16), the last
-# run of a row partly empty; detectors of fewer rows than a run crosses have
-# several removable zeros in one run
+# a PSF large enough for runs of 32 values (the sizes above and several tilts take
+# 16), the last run of a row partly empty; detectors of fewer rows than a run
+# crosses have several removable zeros in one run
+@pytest.mark.parametrize("tilts", [1, 2])
 @pytest.mark.parametrize("nrows", [5, 40])
-def test_psf3d_long_runs_match_oracle(lc, orc64, nrows):
-    announce(f"psf3d long runs nrows={nrows}")
+def test_psf3d_long_runs_match_oracle(lc, orc64, nrows, tilts):
+    announce(f"psf3d long runs nrows={nrows} tilts={tilts}")
     dims, nproj = (9, 401, 401), 6
     th = np.arange(nproj) * (2 * np.pi / nproj)
-    ga = np.repeat([-np.pi / 6, 0.3], nproj // 2)
+    ga = np.repeat([-np.pi / 6, 0.3 if tilts == 2 else -np.pi / 6], nproj // 2)
     psf = lc.PointSpreadFunction(lc.PolarGrid(th, ga, np.zeros(nproj), nrows, 401), dims)
     x = np.random.default_rng(6).random(dims)
     ref = orc64.psf3d(th, ga, np.zeros(nproj), nrows, 401, dims, method=0).convolve(x)
