@@ -95,7 +95,7 @@ k_det_fft(const float *__restrict__ real_in, const float2 *__restrict__ cplx_in,
     }
 }
 
-// The same for widths that are not 2^p 3^q (up to 2048): Bluestein's algorithm
+// The same for widths that are not 2^p 3^q (65 to 2048): Bluestein's algorithm
 // with a power-of-two length L >= 2 n - 1, in FP64 (as the direct sum below
 // accumulates; the FP64 rate equals that of unpacked FP32 and the rows are few):
 //   X_m = a_m sum_k (x_k a_k) b_{m-k},  a_k = e^{SIGN i pi k^2 / n},  b_k = conj(a_k)
@@ -153,7 +153,8 @@ k_det_blue(const float *__restrict__ real_in, const float2 *__restrict__ cplx_in
     }
 }
 
-// direct DFT for widths above 2048 that are not 2^p 3^q, or above 4096
+// direct DFT for widths that are not 2^p 3^q, up to 64 or above 2048, and for
+// all above 4096
 template <int SIGN>
 __global__ void k_det_dft(const float *__restrict__ real_in, const float2 *__restrict__ cplx_in,
                           float2 *__restrict__ cplx_out, float *__restrict__ real_out, int nrows,
@@ -955,7 +956,9 @@ void nufft2d_init(Ctx &c, Geom2D &g, bool own_work) {
     c.sync();
     LC_REQUIRE(fft_make_plan(u.nf, u.plan_nf), "nufft: fine grid size not 2^p 3^q");
     u.det_fast = g.nrad <= DET_FFT_MAX && fft_make_plan((int)g.nrad, u.plan_det);
-    u.det_blue = !u.det_fast && 2 * g.nrad - 1 <= DET_FFT_MAX;
+    // (back-projection of 360 rows, us, directly / by Bluestein: 37 columns 80 / 96,
+    // 53 105 / 118, 67 126 / 124, 127 212 / 198, 511 1084 / 677)
+    u.det_blue = !u.det_fast && g.nrad > 64 && 2 * g.nrad - 1 <= DET_FFT_MAX;
     if (u.det_blue) det_blue_init(c, u, (int)g.nrad);
     sort_points(c, g, own_work);
     u.ready = true;

@@ -74,11 +74,12 @@ def test_backproj2d_matches_oracle(lc, orc64, N, nang, nrad, ns, span):
     assert err < PROJ_TOL
 
 
-# detector widths that are not 2^p 3^q: the smallest, ones whose transform
-# length is compiled (256 .. 2048: several rows per block, a partial last
-# block, one row per two blocks) and ones around 1024 / 2048, where it changes
-@pytest.mark.parametrize("nrad,nang", [(5, 7), (95, 33), (130, 17), (511, 9), (1021, 5), (1025, 4), (2047, 3),
-                                       (2051, 2)])
+# detector widths that are not 2^p 3^q: the smallest and the last that are summed
+# directly, the first by Bluestein's algorithm, ones whose transform length is
+# compiled (256 .. 2048: several rows per block, a partial last block, one row
+# per two blocks) and ones around 1024 / 2048, where it changes
+@pytest.mark.parametrize("nrad,nang", [(5, 7), (63, 9), (65, 9), (95, 33), (130, 17), (511, 9), (1021, 5), (1025, 4),
+                                       (2047, 3), (2051, 2)])
 def test_detector_widths_match_oracle(lc, orc64, nrad, nang):
     # both directions against the FP64 oracle; the projectors' own FP32 error is
     # about 5e-7, so a wrong detector bin or phase (1 / nrad of the energy or
