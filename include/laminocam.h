@@ -425,22 +425,21 @@ int lc_autotune2d(lc_ctx ctx, lc_geom2d g, int32_t nslices, int32_t *variant, do
 int lc_set_tuning2d(lc_ctx ctx, int64_t image_n, const int32_t *variant);
 int lc_get_tuning2d(lc_ctx ctx, int64_t image_n, int32_t *variant);
 
-/* ---- 3-D NUFFT spread bin shapes per grid (no reference counterpart) ----
- * The type-1 spread of lc_backproj3d sorts the points into bins of footprint
- * corners; the library is compiled for several bin shapes (shape 0, at most
- * 9 x 9 x 9 corner cells along z, y, x, is the default; 1 is 9 x 25 x 9; 2 is
- * the default's with dense bins shared out among more waves from 512 points
- * instead of 2048).
- * lc_autotune3d times a back-projection of g's grid with each shape,
+/* ---- 3-D NUFFT spread choices per grid (no reference counterpart) ----
+ * The type-1 spread of lc_backproj3d sorts the points into bins of at most
+ * 9 x 9 x 9 footprint corners and shares the points of a dense bin out among
+ * more waves: from 2048 points with choice 0, the default, and from 512 with
+ * choice 2.  (Choice 1, once another bin shape, is the same as 0.)
+ * lc_autotune3d times a back-projection of g's grid with each choice,
  * installs the fastest in the context for g's fine-grid shape (the volume's
  * dims, oversampled) and returns it, with the time of one back-projection in
  * ms.  lc_set_tuning3d installs a known choice; lc_get_tuning3d reads the
  * current one.  Every choice gives the same result up to the order of the
  * spread's sums (it is deterministic for a given choice). */
 int lc_autotune3d(lc_ctx ctx, lc_geom3d g, int32_t *shape, double *ms);
-/* The 2-D spread of lc_backproj2d likewise (no reference counterpart): output
- * tiles of 16 (shape 0, the default) or 32 (shape 1) rows of 16 cells per fine-
- * grid size, timed on nslices slices of g. */
+/* The 2-D spread of lc_backproj2d likewise (no reference counterpart), per
+ * fine-grid size and timed on nslices slices of g.  Choices 0 and 1 are both
+ * accepted and the same: the other tile shape was never the faster one. */
 int lc_autotune2d_nufft(lc_ctx ctx, lc_geom2d g, int32_t nslices, int32_t *shape, double *ms);
 int lc_set_tuning2d_nufft(lc_ctx ctx, lc_geom2d g, int32_t shape);
 int lc_get_tuning2d_nufft(lc_ctx ctx, lc_geom2d g, int32_t *shape);

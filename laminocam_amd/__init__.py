@@ -90,11 +90,11 @@ class Context:
         _lib.check(self.lib.lc_get_tuning2d(self.handle, int(image_n), v))
         return tuple(v)
 
-    # ---- 2-D NUFFT spread bin shape per fine-grid size ----
+    # ---- 2-D NUFFT spread choice per fine-grid size ----
     def autotune2d_nufft(self, psf: "PointSpreadFunction2D", nslices: int = 8):
-        """Time the 2-D spread's compiled bin shapes on nslices slices of
-        psf's grid, install the fastest for its fine-grid size; returns
-        (shape index, ms per back-projection)."""
+        """Time the 2-D spread on nslices slices of psf's grid and install
+        its choice (one is compiled) for that fine-grid size; returns
+        (choice, ms per back-projection)."""
         sh = C.c_int32()
         ms = C.c_double()
         _lib.check(self.lib.lc_autotune2d_nufft(self.handle, psf.handle, int(nslices), C.byref(sh),
@@ -109,11 +109,11 @@ class Context:
         _lib.check(self.lib.lc_get_tuning2d_nufft(self.handle, psf.handle, C.byref(sh)))
         return sh.value
 
-    # ---- 3-D NUFFT spread bin shape per grid ----
+    # ---- 3-D NUFFT spread choice per grid ----
     def autotune3d(self, psf: "PointSpreadFunction"):
-        """Time the 3-D spread's compiled bin shapes on psf's grid (its
+        """Time the 3-D spread's compiled choices on psf's grid (its
         back-projection), install the fastest for that grid's fine-grid
-        shape; returns (shape index, ms per back-projection)."""
+        shape; returns (choice, ms per back-projection)."""
         sh = C.c_int32()
         ms = C.c_double()
         _lib.check(self.lib.lc_autotune3d(self.handle, psf.handle, C.byref(sh), C.byref(ms)))

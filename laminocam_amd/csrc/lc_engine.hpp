@@ -23,10 +23,10 @@ struct Nufft2D {
     FftPlan plan_det{};   // detector FFT (det_fast: of the width; det_blue: Bluestein length)
     bool det_fast = false, det_blue = false;
     // the points of a slice sorted by corner bin (unsigned[nang * nrad], then
-    // int[bins + 1] starts) and the spread's tiles, fullest first, per tile
-    // shape: ntiles of them from tiles_off, the first nheavy heavy
+    // int[bins + 1] starts) and the spread's tiles, fullest first, the first
+    // nheavy heavy
     DBuf points, tiles;
-    int tiles_off[2] = {0, 0}, ntiles[2] = {0, 0}, nheavy[2] = {0, 0};
+    int ntiles = 0, nheavy = 0;
     DBuf chirp;           // det_blue: double2 chirp[nrad], then its spectrum [plan_det.L]
     bool ready = false;
 };
@@ -257,8 +257,8 @@ int toep3d_block_width(int N, int M, bool f64);
 int nufft2d_fine_n(int64_t N);
 int nufft3d_fine_n(int64_t n);
 size_t nufft3d_spread_bytes(int64_t npts, const int nf[3]);
-// the 3-D spread's compiled bin shapes, and the autotuner that picks one per
-// fine-grid shape (returns its index; installs it in c.nu3_tuning)
+// the numbers of the 3-D spread's choices, and the autotuner that picks one per
+// fine-grid shape (returns it; installs it in c.nu3_tuning)
 int nufft3d_num_shapes();
 int nufft3d_autotune(Ctx &c, Geom3D &g, double *best_ms);
 // the same for the 2-D spread, per fine-grid size, timed on nslices slices

@@ -187,7 +187,7 @@ __global__ void k_det_dft(const float *__restrict__ real_in, const float2 *__res
 // Type-1 spreading by output tiles.  A point's corner is its first footprint
 // cell, ceil(g - 4) per axis, taken modulo nf.  The geometry holds the points
 // sorted by 8 x 8 bins of corners (row major; the points do not depend on the
-// data, so nufft2d_init sorts them once), so a tile of T rows x 16 columns of
+// data, so nufft2d_init sorts them once), so a tile of 16 x 16 cells of
 // the fine grid finds the points that reach it (corners from 7 cells before it
 // to its end) in one or two runs per row of bins.  It takes them in that order
 // and writes its cells once: no clearing, no adding into the grid, no order
@@ -195,7 +195,7 @@ __global__ void k_det_dft(const float *__restrict__ real_in, const float2 *__res
 // rest of the stack.
 //
 // A tile is a matrix product: with wy, wx a point's 8 weights per axis placed
-// in T (16) slots, zero elsewhere,
+// in 16 slots, zero elsewhere,
 //   tile[y][x] = sum_p wy_p[y] (c_p wx_p[x])
 // which runs on FP32 MFMA tiles (v_mfma_f32_16x16x4_f32: lane l holds
 // A[l & 15][l >> 4], B[l >> 4][l & 15] and, in register q,
@@ -212,22 +212,13 @@ __global__ void k_det_dft(const float *__restrict__ real_in, const float2 *__res
 // loop the sums moved between register files and the spread took 423 us.
 // ---------------------------------------------------------------------------
 constexpr int CB = 8;                       // corner bin edge
-constexpr int TX = 16;                      // tile columns
+constexpr int TE = 16;                      // tile edge, that of an MFMA tile (tiles of 32 rows took 1.1 to
+                                            // 1.5 times as long at each of 14 sizes)
 constexpr int TAB = 64;                     // points per table
 constexpr int TS = 17;                      // row stride of a 16-slot table
 constexpr int SW = 4;                       // waves per block
-// a compiled tile: rows, and the heavy tiles' threshold (1024 points: 253 us in
-// place of 231 for 16 slices of 256^2 from 360 angles, 2048: 310 us)
-template <int T_> struct Tile2 {
-    static constexpr int T = T_, M = T / 16;
-    static constexpr int HEAVY = 512;
-    static_assert(T % 16 == 0, "tiles are rows of MFMA tiles");
-};
-constexpr int N_SHAPES2 = 2;
-template <typename F> void with_shape2(int i, F &&f) {
-    if (i == 1) f(Tile2<32>{});
-    else f(Tile2<16>{});
-}
+constexpr int HEAVY = 512;                  // points of the fullest light tile (1024: 253 us in place of 231
+                                            // for 16 slices of 256^2 from 360 angles, 2048: 310 us)
 
 struct Grid2 {
     int nang, nrad, nf;
@@ -303,10 +294,10 @@ __global__ void k_bin2_starts(const unsigned *__restrict__ skey, int npts, int *
     start[b] = lo;
 }
 
-// The corner bins that reach cells [c0, c0 + n) of an axis (n <= 32, 7 corners
+// The corner bins that reach cells [c0, c0 + n) of an axis (n <= 16, 7 corners
 // before them): the bins lo .. hi of the grid itself (image 0, corners as they
 // are) and, for the first tile, the last bins (image 1, corners less nf).
-__host__ __device__ inline void tile_bins(int c0, int n, int nf, int image, int &lo, int &hi) {
+__device__ __forceinline__ void tile_bins(int c0, int n, int nf, int image, int &lo, int &hi) {
     if (image == 0) {
         lo = (c0 >= NU_W - 1 ? c0 - (NU_W - 1) : 0) / CB;
         hi = (c0 + n - 1) / CB;
@@ -317,55 +308,53 @@ __host__ __device__ inline void tile_bins(int c0, int n, int nf, int image, int 
 }
 
 // the runs of sorted points of a tile, walked in a fixed order
-template <typename F> __host__ __device__ __forceinline__ void tile_runs(int y0, int x0, int t, int nf, int nb, F &&run) {
+template <typename F> __device__ __forceinline__ void tile_runs(int y0, int x0, int nf, int nb, F &&run) {
     for (int iy = 1; iy >= 0; --iy) {
         int yl, yh;
-        tile_bins(y0, nf - y0 < t ? nf - y0 : t, nf, iy, yl, yh);
+        tile_bins(y0, min(nf - y0, TE), nf, iy, yl, yh);
         for (int by = yl; by <= yh; ++by)
             for (int ix = 1; ix >= 0; --ix) {
                 int xl, xh;
-                tile_bins(x0, nf - x0 < TX ? nf - x0 : TX, nf, ix, xl, xh);
+                tile_bins(x0, min(nf - x0, TE), nf, ix, xl, xh);
                 if (xl <= xh) run(by * nb + xl, by * nb + xh + 1, iy ? nf : 0, ix ? nf : 0);
             }
     }
 }
-// key[t] = 2^31 - 1 - points of tile t, val[t] = t; heavy counts the tiles of more than S::HEAVY
-template <typename S>
+// key[t] = 2^31 - 1 - points of tile t, val[t] = t; heavy counts the tiles of more than HEAVY
 __global__ void k_tile_keys(const int *__restrict__ start, unsigned *__restrict__ key, int *__restrict__ val,
                             int *__restrict__ heavy, int ntiles, int ntx, int nf, int nb) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ntiles) return;
     int n = 0;
-    tile_runs(t / ntx * S::T, t % ntx * TX, S::T, nf, nb, [&](int b0, int b1, int, int) { n += start[b1] - start[b0]; });
+    tile_runs(t / ntx * TE, t % ntx * TE, nf, nb, [&](int b0, int b1, int, int) { n += start[b1] - start[b0]; });
     key[t] = 0x7fffffffu - (unsigned)n;
     val[t] = t;
-    if (n > S::HEAVY) atomicAdd(heavy, 1);
+    if (n > HEAVY) atomicAdd(heavy, 1);
 }
 // most runs of a tile: its own rows of bins and the wrapped ones, in two pieces
-template <typename S> constexpr int max_runs() { return 2 * ((S::T + NU_W - 2) / CB + 2 + 2); }
+constexpr int MAX_RUNS = 2 * ((TE + NU_W - 2) / CB + 2 + 2);
 
 // (a multiple of 16 bytes: every wave's tables start where 16-byte accesses may)
-template <typename S, int SC> struct alignas(16) SpreadLds2 {
-    float x[TAB * TS], y[S::M][TAB * TS];
+template <int SC> struct alignas(16) SpreadLds2 {
+    float x[TAB * TS], y[TAB * TS];
     float2 c[SC][TAB];
-    int rbeg[max_runs<S>()], rpos[max_runs<S>() + 1], roff[max_runs<S>()];
+    int rbeg[MAX_RUNS], rpos[MAX_RUNS + 1], roff[MAX_RUNS];
 };
 
 // spreads tile `tile` of slices s0 .. s0 + SC - 1 with one wave, or with the
 // block's SW waves (TEAM)
-template <typename S, int SC, bool TEAM>
+template <int SC, bool TEAM>
 __device__ __forceinline__ void spread2_tile(const float2 *__restrict__ C, float2 *__restrict__ fine,
                                              const double2 *__restrict__ cs, const unsigned *__restrict__ sval,
                                              const int *__restrict__ start, int tile, int s0, int ntx,
-                                             const Grid2 &g, SpreadLds2<S, SC> *lds) {
-    constexpr int T = S::T, MT = S::M;
+                                             const Grid2 &g, SpreadLds2<SC> *lds) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int ty = tile / ntx, y0 = ty * T, x0 = (tile - ty * ntx) * TX;
+    const int ty = tile / ntx, y0 = ty * TE, x0 = (tile - ty * ntx) * TE;
     const int npts = g.nang * g.nrad;
-    SpreadLds2<S, SC> &L = lds[wave];
+    SpreadLds2<SC> &L = lds[wave];
     // the runs: first sorted point, position of it in the tile's sequence, image
     int nr = 0, total = 0;
-    tile_runs(y0, x0, T, g.nf, g.nb, [&](int b0, int b1, int oy, int ox) {
+    tile_runs(y0, x0, g.nf, g.nb, [&](int b0, int b1, int oy, int ox) {
         const int a = start[b0], n = start[b1] - a;
         if (lane == 0) {
             L.rbeg[nr] = a;
@@ -376,11 +365,9 @@ __device__ __forceinline__ void spread2_tile(const float2 *__restrict__ C, float
         ++nr;
     });
     wave_lds_fence();
-    f32x4 tr[SC][MT], ti[SC][MT];
+    f32x4 tr[SC], ti[SC];
 #pragma unroll
-    for (int s = 0; s < SC; ++s)
-#pragma unroll
-        for (int m = 0; m < MT; ++m) tr[s][m] = ti[s][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < SC; ++s) tr[s] = ti[s] = f32x4{0.f, 0.f, 0.f, 0.f};
     // wave w of a team takes the w-th part of the sequence, in order
     constexpr int NW = TEAM ? SW : 1;
     const int per = ((total + NW - 1) / NW + TAB - 1) / TAB * TAB;
@@ -424,104 +411,86 @@ __device__ __forceinline__ void spread2_tile(const float2 *__restrict__ C, float
             const float wx = es_kernel(((float)(dx - NU_W / 2) + f.fx) * ihw, g.beta);
             const float wy = es_kernel(((float)(dy - NU_W / 2) + f.fy) * ihw, g.beta);
 #pragma unroll
-            for (int sl = q; sl < TX; sl += NU_W) L.x[lane * TS + sl] = (ok && sl == ox + dx) ? wx : 0.f;
-#pragma unroll
-            for (int sl = q; sl < T; sl += NU_W)
-                L.y[sl / 16][lane * TS + sl % 16] = sl == oy + dy ? wy : 0.f;
+            for (int sl = q; sl < TE; sl += NU_W) {
+                L.x[lane * TS + sl] = (ok && sl == ox + dx) ? wx : 0.f;
+                L.y[lane * TS + sl] = sl == oy + dy ? wy : 0.f;
+            }
         }
         wave_lds_fence();
         if (more) fetch(pn);
         im = imn;
-        f32x4 ar[SC][MT], ai[SC][MT];   // this table's sums (short rounding chains)
+        f32x4 ar[SC], ai[SC];   // this table's sums (short rounding chains)
 #pragma unroll
-        for (int s = 0; s < SC; ++s)
-#pragma unroll
-            for (int m = 0; m < MT; ++m) ar[s][m] = ai[s][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < SC; ++s) ar[s] = ai[s] = f32x4{0.f, 0.f, 0.f, 0.f};
         const int ng = (min(TAB, we - base) + 3) >> 2;
         for (int gr = 0; gr < ng; ++gr) {
             const int pt = 4 * gr + k4;
-            const float wx = L.x[pt * TS + n];
-            float wy[MT];
-#pragma unroll
-            for (int m = 0; m < MT; ++m) wy[m] = L.y[m][pt * TS + n];
+            const float wx = L.x[pt * TS + n], wy = L.y[pt * TS + n];
 #pragma unroll
             for (int s = 0; s < SC; ++s) {
                 const float2 c = L.c[s][pt];
-                const float br = wx * c.x, bi = wx * c.y;
-#pragma unroll
-                for (int m = 0; m < MT; ++m) {
-                    ar[s][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(wy[m], br, ar[s][m], 0, 0, 0);
-                    ai[s][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(wy[m], bi, ai[s][m], 0, 0, 0);
-                }
+                ar[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(wy, wx * c.x, ar[s], 0, 0, 0);
+                ai[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(wy, wx * c.y, ai[s], 0, 0, 0);
             }
         }
 #pragma unroll
-        for (int s = 0; s < SC; ++s)
-#pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                tr[s][m] += ar[s][m];
-                ti[s][m] += ai[s][m];
-            }
+        for (int s = 0; s < SC; ++s) {
+            tr[s] += ar[s];
+            ti[s] += ai[s];
+        }
     }
-    auto put = [&](int s, int m, const f32x4 &vr, const f32x4 &vi) {
+    auto put = [&](int s, const f32x4 &vr, const f32x4 &vi) {
         float2 *fs = fine + (int64_t)(s0 + s) * g.nf * g.nf;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int y = y0 + 16 * m + 4 * k4 + q, x = x0 + n;
+            const int y = y0 + 4 * k4 + q, x = x0 + n;
             if (y < g.nf && x < g.nf) fs[(int64_t)y * g.nf + x] = make_float2(vr[q], vi[q]);
         }
     };
     if constexpr (!TEAM) {
 #pragma unroll
-        for (int s = 0; s < SC; ++s)
-#pragma unroll
-            for (int m = 0; m < MT; ++m)
-                put(s, m, tr[s][m], ti[s][m]);
+        for (int s = 0; s < SC; ++s) put(s, tr[s], ti[s]);
     } else {
         // summed in wave order, through the tables' space
         static_assert(sizeof(L.x) >= sizeof(f32x4) * 2 * 64, "the exchange fits the tables");
-        static_assert(alignof(SpreadLds2<S, SC>) >= alignof(f32x4), "and starts where f32x4 may, in every wave");
+        static_assert(alignof(SpreadLds2<SC>) >= alignof(f32x4), "and starts where f32x4 may, in every wave");
 #pragma unroll
-        for (int s = 0; s < SC; ++s)
-#pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                __syncthreads();
-                f32x4 *ex = reinterpret_cast<f32x4 *>(L.x);   // [re, im][lane]
-                ex[lane] = tr[s][m];
-                ex[64 + lane] = ti[s][m];
-                __syncthreads();
-                if (wave == (s * MT + m) % SW) {
-                    const f32x4 *e0 = reinterpret_cast<const f32x4 *>(lds[0].x);
-                    f32x4 vr = e0[lane], vi = e0[64 + lane];
-                    for (int v = 1; v < SW; ++v) {
-                        const f32x4 *ev = reinterpret_cast<const f32x4 *>(lds[v].x);
-                        vr += ev[lane];
-                        vi += ev[64 + lane];
-                    }
-                    put(s, m, vr, vi);
+        for (int s = 0; s < SC; ++s) {
+            __syncthreads();
+            f32x4 *ex = reinterpret_cast<f32x4 *>(L.x);   // [re, im][lane]
+            ex[lane] = tr[s];
+            ex[64 + lane] = ti[s];
+            __syncthreads();
+            if (wave == s % SW) {
+                const f32x4 *e0 = reinterpret_cast<const f32x4 *>(lds[0].x);
+                f32x4 vr = e0[lane], vi = e0[64 + lane];
+                for (int v = 1; v < SW; ++v) {
+                    const f32x4 *ev = reinterpret_cast<const f32x4 *>(lds[v].x);
+                    vr += ev[lane];
+                    vi += ev[64 + lane];
                 }
+                put(s, vr, vi);
             }
+        }
     }
 }
 
 // order: the tiles, fullest first; the first nheavy take a block each, the
 // others a wave each.  grid.y: SC slices each, from slice `first`
-template <typename S, int SC>
+template <int SC>
 __global__ void __launch_bounds__(64 * SW)
 k_spread2d(const float2 *__restrict__ C, float2 *__restrict__ fine, const double2 *__restrict__ cs,
            const unsigned *__restrict__ sval, const int *__restrict__ start, const int *__restrict__ order,
            int ntiles, int nheavy, int first, int ntx, Grid2 g) {
-    __shared__ __align__(16) SpreadLds2<S, SC> lds[SW];
+    __shared__ SpreadLds2<SC> lds[SW];
     const int s0 = first + blockIdx.y * SC, b = blockIdx.x;
     if (b < nheavy) {
-        spread2_tile<S, SC, true>(C, fine, cs, sval, start, __builtin_amdgcn_readfirstlane(order[b]), s0, ntx, g,
-                                  lds);
+        spread2_tile<SC, true>(C, fine, cs, sval, start, __builtin_amdgcn_readfirstlane(order[b]), s0, ntx, g, lds);
         return;
     }
     const int t = nheavy + (b - nheavy) * SW + (int)(threadIdx.x >> 6);
     if (t >= ntiles) return;   // whole wave (no barrier below)
-    spread2_tile<S, SC, false>(C, fine, cs, sval, start, __builtin_amdgcn_readfirstlane(order[t]), s0, ntx, g,
-                               lds);
+    spread2_tile<SC, false>(C, fine, cs, sval, start, __builtin_amdgcn_readfirstlane(order[t]), s0, ntx, g, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -864,14 +833,10 @@ Grid2 grid2(const Geom2D &g) {
     return s;
 }
 
-int tiles_of(int nf, int shape) {
-    int n = 0;
-    with_shape2(shape, [&](auto sh) { n = ceil_div(nf, decltype(sh)::T) * ceil_div(nf, TX); });
-    return n;
-}
+int tiles_of(int nf) { return ceil_div(nf, TE) * ceil_div(nf, TE); }
 
-// the points sorted by corner bin, the bins' starts, and per tile shape the
-// tiles, fullest first.  The sort's working space, about 20 bytes per point, is
+// the points sorted by corner bin, the bins' starts, and the tiles, fullest
+// first.  The sort's working space, about 20 bytes per point, is
 // the projections' scratch, which the caller's own call is about to use, or
 // (own_work) freed again: a server's main context never projects
 void sort_points(Ctx &c, Geom2D &g, bool own_work) {
@@ -881,19 +846,14 @@ void sort_points(Ctx &c, Geom2D &g, bool own_work) {
     const int npts = (int)(g.nang * g.nrad), nbins = s.nb * s.nb;
     int bits = 1;
     while ((1 << bits) < nbins) ++bits;
-    int tiles = 0;
-    for (int i = 0; i < N_SHAPES2; ++i) {
-        u.tiles_off[i] = tiles;
-        u.ntiles[i] = tiles_of(s.nf, i);
-        tiles += u.ntiles[i];
-    }
+    const int tiles = u.ntiles = tiles_of(s.nf);
     const size_t bK = al256(sizeof(unsigned) * (size_t)std::max(npts, tiles));
     size_t tb = 0, tt = 0;
     LC_HIP(rocprim::radix_sort_pairs(nullptr, tb, (unsigned *)nullptr, (unsigned *)nullptr, (unsigned *)nullptr,
                                      (unsigned *)nullptr, (size_t)npts, 0, bits, c.stream()));
     LC_HIP(rocprim::radix_sort_pairs(nullptr, tt, (unsigned *)nullptr, (unsigned *)nullptr, (int *)nullptr,
                                      (int *)nullptr, (size_t)tiles, 0, 31, c.stream()));
-    const size_t need = 3 * bK + al256(std::max(tb, tt)) + sizeof(int) * N_SHAPES2;
+    const size_t need = 3 * bK + al256(std::max(tb, tt)) + sizeof(int);
     DBuf own;
     if (own_work) own.alloc(need);
     char *ws = own_work ? own.as<char>() : reinterpret_cast<char *>(c.scratch(3, need));
@@ -912,18 +872,12 @@ void sort_points(Ctx &c, Geom2D &g, bool own_work) {
     hipLaunchKernelGGL(k_bin2_starts, dim3(ceil_div(nbins + 1, 256)), dim3(256), 0, c.stream(), kb, npts, st, nbins);
     LC_HIP(hipGetLastError());
     u.tiles.alloc(sizeof(int) * tiles);
-    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(N_SHAPES2), 0, c.stream(), heavy);
-    for (int i = 0; i < N_SHAPES2; ++i)
-        with_shape2(i, [&](auto sh) {
-            using S = decltype(sh);
-            const int nt = u.ntiles[i];
-            hipLaunchKernelGGL(k_tile_keys<S>, dim3(ceil_div(nt, 256)), dim3(256), 0, c.stream(), st, ka, (int *)va,
-                               heavy + i, nt, ceil_div(s.nf, TX), s.nf, s.nb);
-            LC_HIP(hipGetLastError());
-            LC_HIP(rocprim::radix_sort_pairs(tmp, tt, ka, kb, (int *)va, u.tiles.as<int>() + u.tiles_off[i],
-                                             (size_t)nt, 0, 31, c.stream()));
-        });
-    LC_HIP(hipMemcpyAsync(u.nheavy, heavy, sizeof(int) * N_SHAPES2, hipMemcpyDeviceToHost, c.stream()));
+    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, c.stream(), heavy);
+    hipLaunchKernelGGL(k_tile_keys, dim3(ceil_div(tiles, 256)), dim3(256), 0, c.stream(), st, ka, (int *)va, heavy,
+                       tiles, ceil_div(s.nf, TE), s.nf, s.nb);
+    LC_HIP(hipGetLastError());
+    LC_HIP(rocprim::radix_sort_pairs(tmp, tt, ka, kb, (int *)va, u.tiles.as<int>(), (size_t)tiles, 0, 31, c.stream()));
+    LC_HIP(hipMemcpyAsync(&u.nheavy, heavy, sizeof(int), hipMemcpyDeviceToHost, c.stream()));
     c.sync();
 }
 } // namespace
@@ -931,9 +885,7 @@ void sort_points(Ctx &c, Geom2D &g, bool own_work) {
 // device bytes of the points' order and the tiles that a geometry keeps
 size_t nufft2d_order_bytes(int64_t nang, int64_t nrad, int nf) {
     const size_t nb = ceil_div(nf, CB);
-    size_t b = al256(sizeof(unsigned) * (size_t)(nang * nrad)) + sizeof(int) * (nb * nb + 1);
-    for (int i = 0; i < N_SHAPES2; ++i) b += sizeof(int) * (size_t)tiles_of(nf, i);
-    return b;
+    return al256(sizeof(unsigned) * (size_t)(nang * nrad)) + sizeof(int) * (nb * nb + 1 + (size_t)tiles_of(nf));
 }
 
 void nufft2d_init(Ctx &c, Geom2D &g, bool own_work) {
@@ -1057,18 +1009,17 @@ NuWork nu_work(Ctx &c, const Geom2D &g, int ns) {
     return w;
 }
 
-// type-1 spread of nch runs of SC slices from slice `first` by tiles of shape S: C -> F
-template <typename S, int SC> void spread2(Ctx &c, const Geom2D &g, const NuWork &w, int first, int nch, int shape) {
+// type-1 spread of nch runs of SC slices from slice `first`: C -> F
+template <int SC> void spread2(Ctx &c, const Geom2D &g, const NuWork &w, int first, int nch) {
     if (nch == 0) return;
     const Nufft2D &u = g.nu;
     const Grid2 s = grid2(g);
-    const int ntx = ceil_div(s.nf, TX), nt = u.ntiles[shape], nh = u.nheavy[shape];
     const unsigned *sval = u.points.as<unsigned>();
     const int *start = reinterpret_cast<const int *>(u.points.as<char>() +
                                                      al256(sizeof(unsigned) * (size_t)(g.nang * g.nrad)));
-    hipLaunchKernelGGL((k_spread2d<S, SC>), dim3(nh + ceil_div(nt - nh, SW), nch), dim3(64 * SW), 0,
-                       c.stream(), w.C, w.F, u.cs.as<double2>(), sval, start,
-                       u.tiles.as<int>() + u.tiles_off[shape], nt, nh, first, ntx, s);
+    hipLaunchKernelGGL(k_spread2d<SC>, dim3(u.nheavy + ceil_div(u.ntiles - u.nheavy, SW), nch), dim3(64 * SW), 0,
+                       c.stream(), w.C, w.F, u.cs.as<double2>(), sval, start, u.tiles.as<int>(), u.ntiles, u.nheavy,
+                       first, ceil_div(s.nf, TE), s);
     LC_HIP(hipGetLastError());
 }
 
@@ -1076,14 +1027,10 @@ template <typename S, int SC> void spread2(Ctx &c, const Geom2D &g, const NuWork
 void type1(Ctx &c, const Geom2D &g, const NuWork &w, float *vol, int ns) {
     const Nufft2D &u = g.nu;
     const int N = (int)g.N, nf = u.nf;
-    const int shape = c.nu2_shape(nf);
-    with_shape2(shape, [&](auto sh) {
-        using S = decltype(sh);
-        // slices share a wave's weights by fours, the last ones by two and one
-        spread2<S, 4>(c, g, w, 0, ns / 4, shape);
-        spread2<S, 2>(c, g, w, ns & ~3, (ns & 2) >> 1, shape);
-        spread2<S, 1>(c, g, w, ns & ~1, ns & 1, shape);
-    });
+    // slices share a wave's weights by fours, the last ones by two and one
+    spread2<4>(c, g, w, 0, ns / 4);
+    spread2<2>(c, g, w, ns & ~3, (ns & 2) >> 1);
+    spread2<1>(c, g, w, ns & ~1, ns & 1);
     const float2 *tw = c.twiddles<float>(nf);
     const int nl = std::min(NU_NT * NU_ME / nf, nf);
     const size_t shr = sizeof(float2) * lds_round(nl * nf);
@@ -1177,50 +1124,36 @@ void sysmat2d_nufft_dev(Ctx &c, Geom2D &g, const float *x, float *y, int ns) {
     type1(c, g, w, y, ns);
 }
 
-// Times the back-projection of nslices zero sinograms on g's grid with every
-// compiled tile shape of the spread, installs the fastest in c.nu2_tuning for
-// that fine-grid size and returns its index (best_ms: one back-projection).
+// Times the back-projection of nslices zero sinograms on g's grid (best_ms) and
+// installs choice 0: both numbers name the one compiled spread.
 int nufft2d_autotune(Ctx &c, Geom2D &g, int nslices, double *best_ms) {
     nu_check(c, g, nslices);
-    const int nf = g.nu.nf;
     const int64_t npts = g.nang * g.nrad;
     DBuf sino(sizeof(float) * (size_t)(nslices * npts)), vol(sizeof(float) * (size_t)nslices * g.N * g.N);
     LC_HIP(hipMemsetAsync(sino.as(), 0, sizeof(float) * (size_t)(nslices * npts), c.stream()));
-    const auto saved = c.nu2_tuning;
     hipEvent_t e0, e1;
     LC_HIP(hipEventCreate(&e0));
     LC_HIP(hipEventCreate(&e1));
-    int best = 0;
-    float tbest = 1e30f;
+    float ms = 0.f;
     try {
-        for (int i = 0; i < N_SHAPES2; ++i) {
-            c.nu2_tuning[nf] = i;
-            backproj2d_dev(c, g, sino.as<float>(), vol.as<float>(), nslices);   // warm-up
-            LC_HIP(hipEventRecord(e0, c.stream()));
-            for (int r = 0; r < 3; ++r) backproj2d_dev(c, g, sino.as<float>(), vol.as<float>(), nslices);
-            LC_HIP(hipEventRecord(e1, c.stream()));
-            LC_HIP(hipEventSynchronize(e1));
-            float ms = 0.f;
-            LC_HIP(hipEventElapsedTime(&ms, e0, e1));
-            if (ms / 3 < tbest) {
-                tbest = ms / 3;
-                best = i;
-            }
-        }
+        backproj2d_dev(c, g, sino.as<float>(), vol.as<float>(), nslices);   // warm-up
+        LC_HIP(hipEventRecord(e0, c.stream()));
+        for (int r = 0; r < 3; ++r) backproj2d_dev(c, g, sino.as<float>(), vol.as<float>(), nslices);
+        LC_HIP(hipEventRecord(e1, c.stream()));
+        LC_HIP(hipEventSynchronize(e1));
+        LC_HIP(hipEventElapsedTime(&ms, e0, e1));
     } catch (...) {
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
-        c.nu2_tuning = saved;
         throw;
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    c.nu2_tuning = saved;
-    c.nu2_tuning[nf] = best;
-    if (best_ms) *best_ms = tbest;
-    return best;
+    c.nu2_tuning[g.nu.nf] = 0;
+    if (best_ms) *best_ms = ms / 3;
+    return 0;
 }
 
-int nufft2d_num_shapes() { return N_SHAPES2; }
+int nufft2d_num_shapes() { return 2; }
 
 } // namespace lc

@@ -97,40 +97,35 @@ __device__ __forceinline__ bool inside_pi(double x, double y, double z) {
 // into nb bins of corners, bin i starting at floor(i nf / nb): an even number
 // of bins of 7 to BE cells (three bins where no even number gives such widths:
 // nf = 24 and 27), so that the footprints of one bin lie in a region of 16
-// cells along z and x (ROWS along y), and the regions of two bins an even
-// distance apart are disjoint, around the periodic wrap too.  k_bin_keys
+// cells along each axis, and the regions of two bins an even distance apart
+// are disjoint, around the periodic wrap too.  k_bin_keys
 // gives every point its bin and, below it, its corner's row in the bin; a
 // stable radix sort (rocPRIM) orders the points, keeping point order where
 // the keys agree; k_bin_ranges marks each bin's run.
 // ---------------------------------------------------------------------------
-constexpr int RGN = 16;                     // region cells along z and x: the edge of an MFMA tile
-constexpr int BE = RGN - W3 + 1;            // most corner cells of a bin along z and x
+constexpr int RGN = 16;                     // region cells along an axis: the edge of an MFMA tile
+constexpr int BE = RGN - W3 + 1;            // most corner cells of a bin along an axis
+constexpr int YB = 4;                       // key bits of a corner's row in its bin
+constexpr int TEAMS = 4;                    // teams of a heavy bin (their tables fill the LDS)
+static_assert(RGN % 8 == 0 && BE < 1 << YB, "rows go to four waves in turn; a row index fits its key bits");
 
-// A compiled region shape: ROWS region rows along y (bins of ROWS - W3 + 1
-// corner rows).  More rows mean fewer bins, whose regions overlap less.
-// A bin of more than HEAVY points is spread by several teams of waves.
-template <int ROWS_, unsigned HEAVY_ = 2048> struct Shape3 {
-    static constexpr int ROWS = ROWS_;
-    static constexpr unsigned HEAVY = HEAVY_;
-    static constexpr int EY = ROWS - W3 + 1;
-    static constexpr int YB = EY <= 16 ? 4 : EY <= 32 ? 5 : 6;   // key bits of the corner row
-    static constexpr int TEAMS = ROWS <= 16 ? 4 : 3;             // teams of a heavy bin (their tables fill the LDS)
-    static_assert(ROWS % 8 == 0 && EY <= 64, "rows go to four waves in turn; a row index has six bits");
-};
-// the shapes the autotuner (nufft3d_autotune) chooses from for the spread, per
-// fine-grid shape; shape 0 is the default.  Interpolation uses shape 0.
+// The spread's choices, per fine-grid shape (nufft3d_autotune): a bin of more
+// than HEAVY points is spread by several teams of waves.  2048 is the default;
+// 512 wins where the fullest bins of a phase are its time, and loses where the
+// phases are long (back-projection, us, 2048 / 512: 8 x 256^2 from 180 x 64 rows
+// 1417 / 1182, 16 x 128^2 from 360 x 48 1903 / 1568, 128^3 from 360 x 128 3093 /
+// 2744; 32 x 256^2 from 720 x 96 4687 / 5281, 32 x 511^2 from 720 x 128 9832 /
+// 11404).  Choice 1, once bins of 25 rows (2.0 to 3.4 times the default's time
+// over twelve scans), is the default too.
 constexpr int N_SHAPES3 = 3;
-template <typename F> void with_shape3(int i, F &&f) {
-    switch (i) {
-    case 1: f(Shape3<32>{}); break;
-    case 2: f(Shape3<16, 512>{}); break;
-    default: f(Shape3<16>{}); break;
-    }
+template <typename F> void with_heavy3(int i, F &&f) {
+    if (i == 2) f(std::integral_constant<unsigned, 512>{});
+    else f(std::integral_constant<unsigned, 2048>{});
 }
 
-// bins along an axis of nf >= 16 cells, for bins of at most `edge` corners
-__host__ __device__ constexpr int bins_along(int nf, int edge) {
-    int nb = 2 * ((nf + 2 * edge - 1) / (2 * edge));
+// bins along an axis of nf >= 16 cells
+__host__ __device__ constexpr int bins_along(int nf) {
+    int nb = 2 * ((nf + 2 * BE - 1) / (2 * BE));
     return nf / nb >= W3 - 1 ? nb : 3;
 }
 
@@ -173,18 +168,17 @@ __device__ __forceinline__ Corner3 corner3(const double *rot, unsigned pt, const
 // key[i]: bin << YB | corner row in the bin of point i, or nbins << YB (sorted
 // last) for a point the mask drops, whose value in `drop` (if given) becomes
 // 0; val[i] = i
-template <typename S>
 __global__ void k_bin_keys(const double *__restrict__ rot, Grid3 g, Bins3 bn, unsigned *__restrict__ key,
                            unsigned *__restrict__ val, int64_t npts, unsigned nbins, float2 *__restrict__ drop) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= npts) return;
     const Corner3 c = corner3(rot, (unsigned)i, g);
-    unsigned b = nbins << S::YB;
+    unsigned b = nbins << YB;
     if (c.ok) {
         const int lz = wrapi(c.lz, g.nf[0]), ly = wrapi(c.ly, g.nf[1]), lx = wrapi(c.lx, g.nf[2]);
         const int bz = bin_of(lz, g.nf[0], bn.nb[0]), by = bin_of(ly, g.nf[1], bn.nb[1]),
                   bx = bin_of(lx, g.nf[2], bn.nb[2]);
-        b = (unsigned)(((int64_t)bz * bn.nb[1] + by) * bn.nb[2] + bx) << S::YB |
+        b = (unsigned)(((int64_t)bz * bn.nb[1] + by) * bn.nb[2] + bx) << YB |
             (unsigned)(ly - bin_first(by, g.nf[1], bn.nb[1]));
     } else if (drop) {
         drop[i] = make_float2(0.f, 0.f);
@@ -196,13 +190,13 @@ __global__ void k_bin_keys(const double *__restrict__ rot, Grid3 g, Bins3 bn, un
 // [start[b], end[b]) is bin b's run in the sorted keys (start = end = 0 when
 // empty: both arrays cleared first)
 __global__ void k_bin_ranges(const unsigned *__restrict__ skey, int64_t n, unsigned *__restrict__ start,
-                             unsigned *__restrict__ end, unsigned nbins, int yb) {
+                             unsigned *__restrict__ end, unsigned nbins) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const unsigned b = skey[i] >> yb;
+    const unsigned b = skey[i] >> YB;
     if (b >= nbins) return;
-    if (i == 0 || (skey[i - 1] >> yb) != b) start[b] = (unsigned)i;
-    if (i == n - 1 || (skey[i + 1] >> yb) != b) end[b] = (unsigned)(i + 1);
+    if (i == 0 || (skey[i - 1] >> YB) != b) start[b] = (unsigned)i;
+    if (i == n - 1 || (skey[i + 1] >> YB) != b) end[b] = (unsigned)(i + 1);
 }
 
 // launch phases along an axis: two (even and odd bins), or one per bin of three
@@ -246,7 +240,7 @@ __global__ void k_phase_shift3d(float2 *__restrict__ C, const double *__restrict
 
 // ---------------------------------------------------------------------------
 // Both directions run on the matrix cores.  With wz, wy, wx a point's 8 weights
-// per axis, placed at its corner in 16 (ROWS) slots that are zero elsewhere,
+// per axis, placed at its corner in 16 slots that are zero elsewhere,
 //   spread:  R[z][y][x]  = sum_p (wz_p[z] wy_p[y]) (c_p wx_p[x])   K = points
 //   interp:  G[p][x]     = sum_{y,z} (wz_p[z] wy_p[y]) F[z][y][x]  K = (z, y)
 //            c_p         = sum_x wx_p[x] G[p][x]
@@ -393,7 +387,6 @@ __global__ void __launch_bounds__(256, 4)
 k_interp3d(const float2 *__restrict__ F, float2 *__restrict__ C, const double *__restrict__ rot,
            const unsigned *__restrict__ skey, const unsigned *__restrict__ sval,
            const unsigned *__restrict__ bend, unsigned npts, unsigned nbins, unsigned chunk, Grid3 g, Bins3 bn) {
-    using S = Shape3<16>;
     __shared__ float Zt[BATCH * RGN], Yt[BATCH * RGN], Xt[BATCH * XS];   // [group][slot][16 points], x: [point][slot]
     __shared__ float2 part[4][BATCH];
     __shared__ int meta[BATCH / 16];
@@ -403,7 +396,7 @@ k_interp3d(const float2 *__restrict__ F, float2 *__restrict__ C, const double *_
     unsigned a = blockIdx.x * chunk;
     const unsigned stop = min(npts, a + chunk);
     while (a < stop) {
-        const unsigned bin = __builtin_amdgcn_readfirstlane(skey[a] >> S::YB);
+        const unsigned bin = __builtin_amdgcn_readfirstlane(skey[a] >> YB);
         if (bin >= nbins) return;   // the masked points: all of the rest (the whole block agrees)
         const unsigned e = min(stop, bend[bin]);
         const int b[3] = {(int)(bin / (unsigned)(bn.nb[1] * bn.nb[2])), (int)(bin / (unsigned)bn.nb[2]) % bn.nb[1],
@@ -493,7 +486,7 @@ k_interp3d(const float2 *__restrict__ F, float2 *__restrict__ C, const double *_
     }
 }
 
-// Bins of more than S::HEAVY points are spread by S::TEAMS teams of four
+// Bins of more than HEAVY points are spread by TEAMS teams of four
 // waves, each taking a consecutive part of the bin's points; their sums are
 // added in team order.  Whether a bin is heavy depends only on its own count.
 
@@ -501,19 +494,19 @@ k_interp3d(const float2 *__restrict__ F, float2 *__restrict__ C, const double *_
 // reordered to [wave][row / 4]), the row strides padded against bank conflicts,
 // and the point groups' rows
 constexpr int ZS = RGN + 1;
-template <typename S> struct alignas(16) SpreadLds {
+struct alignas(16) SpreadLds {
     float z[BATCH * ZS], xr[BATCH * ZS], xi[BATCH * ZS];
-    alignas(16) float y[BATCH * (S::ROWS + 4)];   // read four rows at a time
+    alignas(16) float y[BATCH * (RGN + 4)];   // read four rows at a time
     int meta[BATCH / 4];
 };
 
-// type 1: adds bin `bin`'s points to the fine grid F with TEAMS teams of four waves
-template <typename S, int TEAMS>
+// type 1: adds bin `bin`'s points to the fine grid F with NT teams of four waves
+template <int NT>
 __device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2 *__restrict__ F,
                                             const double *__restrict__ rot, const unsigned *__restrict__ sval,
                                             int bin, unsigned s0, unsigned s1, const Grid3 &g, const Bins3 &bn,
-                                            SpreadLds<S> *lds) {
-    constexpr int NQ = S::ROWS / 4, YS = S::ROWS + 4;
+                                            SpreadLds *lds) {
+    constexpr int NQ = RGN / 4, YS = RGN + 4;
     const int b[3] = {bin / (bn.nb[1] * bn.nb[2]), (bin / bn.nb[2]) % bn.nb[1], bin % bn.nb[2]};
     int s[3], ext[3];   // the region's first cell and extent (the bin's corners + W3 - 1)
 #pragma unroll
@@ -522,10 +515,10 @@ __device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2
         ext[i] = bin_first(b[i] + 1, g.nf[i], bn.nb[i]) - s[i] + W3 - 1;
     }
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
-    const int team = TEAMS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const int team = NT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
     const int p = threadIdx.x & (BATCH - 1), h = (threadIdx.x >> 7) & 1;
     const int n = lane & 15, k4 = lane >> 4;
-    SpreadLds<S> &L = lds[team];
+    SpreadLds &L = lds[team];
     // sums over the batches so far (tr, ti) and within one: two levels keep the
     // chains of rounded additions short where a bin holds thousands of points
     f32x4 tr[NQ], ti[NQ];
@@ -533,7 +526,7 @@ __device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2
     for (int q = 0; q < NQ; ++q) tr[q] = ti[q] = f32x4{0.f, 0.f, 0.f, 0.f};
     // team t takes the t-th part of the bin's points, in order; every team
     // runs the same number of batches
-    const unsigned per = ((s1 - s0 + TEAMS - 1) / TEAMS + BATCH - 1) / BATCH * BATCH;
+    const unsigned per = ((s1 - s0 + NT - 1) / NT + BATCH - 1) / BATCH * BATCH;
     const unsigned ws = min(s1, s0 + team * per), we = min(s1, ws + per);
     const int nit = (int)(per / BATCH);
     // the next batch's points are fetched during this one
@@ -553,7 +546,7 @@ __device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2
             const float cr = ok ? cv.x : 0.f, ci = ok ? cv.y : 0.f;
             // past the last point every product is 0 x a stored weight
             axis_weights<RGN>(ft.t[0], ft.f[0], h, g.beta, [&](int sl, float v) { zt[sl] = ok ? v : 0.f; });
-            axis_weights<S::ROWS>(ft.t[1], ft.f[1], h, g.beta,
+            axis_weights<RGN>(ft.t[1], ft.f[1], h, g.beta,
                                   [&](int sl, float v) { yt[(sl & 3) * NQ + (sl >> 2)] = v; });
             axis_weights<RGN>(ft.t[2], ft.f[2], h, g.beta, [&](int sl, float v) {
                 xr[sl] = v * cr;
@@ -618,7 +611,7 @@ __device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2
         zz -= zz >= g.nf[0] ? g.nf[0] : 0;
         return F + ((int64_t)zz * g.nf[1] + yy) * g.nf[2] + xx;
     };
-    if constexpr (TEAMS == 1) {
+    if constexpr (NT == 1) {
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
             float2 v[4];
@@ -637,16 +630,16 @@ __device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2
         }
     } else {
         // row slot by row slot through LDS (the tables' space): team q mod
-        // TEAMS adds the teams' sums in team order
+        // NT adds the teams' sums in team order
         f32x4 *ex = reinterpret_cast<f32x4 *>(lds);   // [team][wave][re, im][lane]
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
             ex[((team * 4 + w) * 2) * 64 + lane] = tr[q];
             ex[((team * 4 + w) * 2 + 1) * 64 + lane] = ti[q];
             __syncthreads();
-            if (q % TEAMS == team) {
+            if (q % NT == team) {
                 f32x4 sr = ex[(w * 2) * 64 + lane], si = ex[(w * 2 + 1) * 64 + lane];
-                for (int t = 1; t < TEAMS; ++t) {
+                for (int t = 1; t < NT; ++t) {
                     sr += ex[((t * 4 + w) * 2) * 64 + lane];
                     si += ex[((t * 4 + w) * 2 + 1) * 64 + lane];
                 }
@@ -666,21 +659,21 @@ __device__ __forceinline__ void spread3_bin(const float2 *__restrict__ C, float2
 }
 
 // one block per light bin of this phase (order: the phase's bins, fullest first)
-template <typename S>
-__global__ void __launch_bounds__(256, S::ROWS <= 16 ? 4 : 1)
+template <unsigned HEAVY>
+__global__ void __launch_bounds__(256, 4)
 k_spread3d_bin(const float2 *__restrict__ C, float2 *__restrict__ F, const double *__restrict__ rot,
                const unsigned *__restrict__ sval, const unsigned *__restrict__ bstart,
                const unsigned *__restrict__ bend, const unsigned *__restrict__ order, Grid3 g, Bins3 bn) {
     const int bin = __builtin_amdgcn_readfirstlane(order[blockIdx.x]);
     const unsigned s0 = bstart[bin], s1 = bend[bin];
-    if (s0 >= s1 || s1 - s0 > S::HEAVY) return;   // empty, or a heavy bin
-    spread3_bin<S, 1>(C, F, rot, sval, bin, s0, s1, g, bn, reinterpret_cast<SpreadLds<S> *>(lc_smem));
+    if (s0 >= s1 || s1 - s0 > HEAVY) return;   // empty, or a heavy bin
+    spread3_bin<1>(C, F, rot, sval, bin, s0, s1, g, bn, reinterpret_cast<SpreadLds *>(lc_smem));
 }
 
 // the phase's heavy bins (a prefix of its order): each block takes bins
 // j, j + gridDim.x, ... until the first light one
-template <typename S>
-__global__ void __launch_bounds__(256 * S::TEAMS)
+template <unsigned HEAVY>
+__global__ void __launch_bounds__(256 * TEAMS)
 k_spread3d_bin_heavy(const float2 *__restrict__ C, float2 *__restrict__ F, const double *__restrict__ rot,
                      const unsigned *__restrict__ sval, const unsigned *__restrict__ bstart,
                      const unsigned *__restrict__ bend, const unsigned *__restrict__ order, unsigned nphase,
@@ -688,8 +681,8 @@ k_spread3d_bin_heavy(const float2 *__restrict__ C, float2 *__restrict__ F, const
     for (unsigned j = blockIdx.x; j < nphase; j += gridDim.x) {
         const int bin = __builtin_amdgcn_readfirstlane(order[j]);
         const unsigned s0 = bstart[bin], s1 = bend[bin];
-        if (s1 - s0 <= S::HEAVY) break;   // the order is fullest first: the rest are light
-        spread3_bin<S, S::TEAMS>(C, F, rot, sval, bin, s0, s1, g, bn, reinterpret_cast<SpreadLds<S> *>(lc_smem));
+        if (s1 - s0 <= HEAVY) break;   // the order is fullest first: the rest are light
+        spread3_bin<TEAMS>(C, F, rot, sval, bin, s0, s1, g, bn, reinterpret_cast<SpreadLds *>(lc_smem));
     }
 }
 
@@ -994,30 +987,21 @@ struct Work3 {
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-template <typename S> Bins3 bins_of(const int nf[3]) {
-    const Bins3 bn{{bins_along(nf[0], BE), bins_along(nf[1], S::EY), bins_along(nf[2], BE)}};
-    const int edge[3] = {BE, S::EY, BE};
+Bins3 bins_of(const int nf[3]) {
+    const Bins3 bn{{bins_along(nf[0]), bins_along(nf[1]), bins_along(nf[2])}};
     for (int a = 0; a < 3; ++a)
-        LC_REQUIRE(nf[a] >= RGN && ceil_div(nf[a], bn.nb[a]) <= edge[a], "3-D NUFFT: no bins for this fine grid");
+        LC_REQUIRE(nf[a] >= RGN && ceil_div(nf[a], bn.nb[a]) <= BE, "3-D NUFFT: no bins for this fine grid");
     return bn;
 }
 unsigned count_of(const Bins3 &bn) { return (unsigned)bn.nb[0] * bn.nb[1] * bn.nb[2]; }
-// the most bins any compiled shape makes of this grid, and the most values
-// their sort keys take (work buffers fit every shape)
-unsigned nbins_max(const int nf[3]) {
-    unsigned m = 0;
-    for (int i = 0; i < N_SHAPES3; ++i)
-        with_shape3(i, [&](auto sh) { m = std::max(m, count_of(bins_of<decltype(sh)>(nf))); });
-    return m;
-}
 
 // bits of the sort key: bins 0 .. nbins - 1 and nbins for dropped points, above
-// the yb bits of the corner row
-int key_bits(unsigned nbins, int yb) {
+// the bits of the corner row
+int key_bits(unsigned nbins) {
     int b = 1;
     while (b < 32 && (1ull << b) <= nbins) ++b;
-    LC_REQUIRE(b + yb <= 32, "3-D NUFFT: too many bins");
-    return b + yb;
+    LC_REQUIRE(b + YB <= 32, "3-D NUFFT: too many bins");
+    return b + YB;
 }
 
 size_t sort_tmp_bytes(int64_t npts, unsigned nbins) {
@@ -1031,7 +1015,7 @@ size_t sort_tmp_bytes(int64_t npts, unsigned nbins) {
 
 // bytes of the sorted points' buffers
 size_t spread_bytes(int64_t npts, const int nf[3]) {
-    const unsigned nbins = nbins_max(nf);
+    const unsigned nbins = count_of(bins_of(nf));
     return 4 * align256(sizeof(unsigned) * (size_t)npts) + 6 * align256(sizeof(unsigned) * (size_t)nbins) +
            align256(sort_tmp_bytes(npts, nbins));
 }
@@ -1053,7 +1037,7 @@ Work3 work3(Ctx &c, const Geom3D &g, int64_t nsort) {
     const size_t bV1 = align256(sizeof(float2) * (size_t)u.nf[0] * u.nf[1] * g.n3);
     const size_t bV2 = align256(sizeof(float2) * (size_t)u.nf[0] * g.n2 * g.n3);
     const size_t base = bC + bF + bV1 + bV2;
-    const unsigned nbins = nbins_max(u.nf);
+    const unsigned nbins = count_of(bins_of(u.nf));
     const size_t bK = align256(sizeof(unsigned) * (size_t)npts);
     const size_t bB = align256(sizeof(unsigned) * (size_t)nbins);
     Work3 w{};
@@ -1164,16 +1148,15 @@ void det_axis(Ctx &c, const DetLine &d, const void *in, void *out, int64_t outer
     LC_HIP(hipGetLastError());
 }
 
-// orders the points of np projections from p0 on by the bins of shape S
+// orders the points of np projections from p0 on by their bins
 // (w.key_b, w.val_b, w.bstart, w.bend); drop: the values of masked points among
 // them are cleared there
-template <typename S>
 Bins3 sort_points(Ctx &c, const Geom3D &g, const Work3 &w, const Grid3 &gg, float2 *drop, int64_t p0, int64_t np) {
-    const Bins3 bn = bins_of<S>(g.nu.nf);
+    const Bins3 bn = bins_of(g.nu.nf);
     const unsigned nbins = count_of(bn);
     const int64_t npts = np * g.nrows * g.ncols;
-    const int bits = key_bits(nbins, S::YB);
-    hipLaunchKernelGGL(k_bin_keys<S>, dim3((unsigned)ceil_div(npts, 256)), dim3(256), 0, c.stream(),
+    const int bits = key_bits(nbins);
+    hipLaunchKernelGGL(k_bin_keys, dim3((unsigned)ceil_div(npts, 256)), dim3(256), 0, c.stream(),
                        g.d_rot.as<double>() + 6 * p0, gg, bn, w.key_a, w.val_a, npts, nbins, drop);
     LC_HIP(hipGetLastError());
     size_t tb = w.sort_bytes;
@@ -1182,7 +1165,7 @@ Bins3 sort_points(Ctx &c, const Geom3D &g, const Work3 &w, const Grid3 &gg, floa
     hipLaunchKernelGGL(k_zero_u32, dim3(1024), dim3(256), 0, c.stream(), w.bstart,
                        (int64_t)(w.bend - w.bstart) + nbins);
     hipLaunchKernelGGL(k_bin_ranges, dim3((unsigned)ceil_div(npts, 256)), dim3(256), 0, c.stream(), w.key_b,
-                       npts, w.bstart, w.bend, nbins, S::YB);
+                       npts, w.bstart, w.bend, nbins);
     LC_HIP(hipGetLastError());
     return bn;
 }
@@ -1194,11 +1177,11 @@ Bins3 sort_points(Ctx &c, const Geom3D &g, const Work3 &w, const Grid3 &gg, floa
 // 256^2 0.3 M 319 / 354, 0.6 M 509 / 434; 32 x 511^2 0.5 M 1090 / 1165, 0.8 M 1396 /
 // 1294; 29 x 721^2 0.6 M 2241 / 2365, 1.0 M 2675 / 2650.
 bool interp_direct(int64_t npts, const int nf[3]) {
-    return npts <= 450000 + 2 * (int64_t)count_of(bins_of<Shape3<16>>(nf));
+    return npts <= 450000 + 2 * (int64_t)count_of(bins_of(nf));
 }
 
 // vol -> w.C, nsort projections at a time; sort: leaves the last ones' points
-// sorted by the bins of Shape3<16>, for a type 1 to follow
+// sorted, for a type 1 to follow
 void type2_3d(Ctx &c, const Geom3D &g, const Work3 &w, const float *vol, bool mask, int64_t nsort, bool sort) {
     const Nufft3D &u = g.nu;
     const int n1 = (int)g.n1, n2 = (int)g.n2, n3 = (int)g.n3;
@@ -1221,7 +1204,7 @@ void type2_3d(Ctx &c, const Geom3D &g, const Work3 &w, const float *vol, bool ma
     for (int64_t p0 = 0; p0 < g.nproj; p0 += nsort) {
         const int64_t np = std::min<int64_t>(nsort, g.nproj - p0), npts = np * g.nrows * g.ncols;
         float2 *C = w.C + p0 * g.nrows * g.ncols;
-        const Bins3 bn = sort_points<Shape3<16>>(c, g, w, gg, C, p0, np);
+        const Bins3 bn = sort_points(c, g, w, gg, C, p0, np);
         // long runs read a bin's region once; short ones keep a small grid's blocks many
         const unsigned chunk =
             (unsigned)std::min<int64_t>(1024, std::max<int64_t>(1, npts / (4096 * BATCH)) * BATCH);
@@ -1232,11 +1215,11 @@ void type2_3d(Ctx &c, const Geom3D &g, const Work3 &w, const float *vol, bool ma
     }
 }
 
-// the sorted-bin spread with region shape S: w.C -> w.F (sorted: the points
-// are already in the order of S's bins)
-template <typename S> void spread3d(Ctx &c, const Geom3D &g, const Work3 &w, const Grid3 &gg, bool sorted) {
+// the sorted-bin spread: w.C -> w.F (sorted: the points are already
+// in the order of the bins)
+template <unsigned HEAVY> void spread3d(Ctx &c, const Geom3D &g, const Work3 &w, const Grid3 &gg, bool sorted) {
     const Nufft3D &u = g.nu;
-    const Bins3 bn = sorted ? bins_of<S>(u.nf) : sort_points<S>(c, g, w, gg, nullptr, 0, g.nproj);
+    const Bins3 bn = sorted ? bins_of(u.nf) : sort_points(c, g, w, gg, nullptr, 0, g.nproj);
     const unsigned nbins = count_of(bn);
     hipLaunchKernelGGL(k_bin_order_keys, dim3(ceil_div(nbins, 256)), dim3(256), 0, c.stream(), w.bstart,
                        w.bend, bn, w.okey_a, w.oval_a, nbins);
@@ -1255,10 +1238,10 @@ template <typename S> void spread3d(Ctx &c, const Geom3D &g, const Work3 &w, con
         const int r[3] = {ph / (per[1] * per[2]), (ph / per[2]) % per[1], ph % per[2]};
         int nblk = 1;
         for (int a = 0; a < 3; ++a) nblk *= (bn.nb[a] - r[a] + per[a] - 1) / per[a];
-        hipLaunchKernelGGL(k_spread3d_bin_heavy<S>, dim3(std::min(nblk, 256)), dim3(256 * S::TEAMS),
-                           sizeof(SpreadLds<S>) * S::TEAMS, c.stream(), w.C, w.F, g.d_rot.as<double>(), w.val_b,
+        hipLaunchKernelGGL(k_spread3d_bin_heavy<HEAVY>, dim3(std::min(nblk, 256)), dim3(256 * TEAMS),
+                           sizeof(SpreadLds) * TEAMS, c.stream(), w.C, w.F, g.d_rot.as<double>(), w.val_b,
                            w.bstart, w.bend, w.order + first, (unsigned)nblk, gg, bn);
-        hipLaunchKernelGGL(k_spread3d_bin<S>, dim3(nblk), dim3(256), sizeof(SpreadLds<S>), c.stream(), w.C, w.F,
+        hipLaunchKernelGGL(k_spread3d_bin<HEAVY>, dim3(nblk), dim3(256), sizeof(SpreadLds), c.stream(), w.C, w.F,
                            g.d_rot.as<double>(), w.val_b, w.bstart, w.bend, w.order + first, gg, bn);
         LC_HIP(hipGetLastError());
         first += nblk;
@@ -1277,10 +1260,7 @@ void type1_3d(Ctx &c, const Geom3D &g, const Work3 &w, float *vol, bool mask, co
                            shifts, gg, np);
         LC_HIP(hipGetLastError());
     }
-    with_shape3(c.nu3_shape(u.nf), [&](auto sh) {
-        using S = decltype(sh);
-        spread3d<S>(c, g, w, gg, sorted && S::ROWS == 16);
-    });
+    with_heavy3(c.nu3_shape(u.nf), [&](auto heavy) { spread3d<decltype(heavy)::value>(c, g, w, gg, sorted); });
     const float *corr = g.nu.corr.as<float>();
     // x: rows (nf0*nf1, nf2) -> (nf0*nf1, n3)
     nu_axis<1, false, false>(c, w.F, w.V1, (int64_t)u.nf[0] * u.nf[1], 1, u.nf[2], n3,
@@ -1337,7 +1317,7 @@ size_t nufft3d_spread_bytes(int64_t npts, const int nf[3]) { return spread_bytes
 
 int nufft3d_num_shapes() { return N_SHAPES3; }
 
-// Times the back-projection of g's grid with every compiled bin shape of the
+// Times the back-projection of g's grid with every compiled choice of the
 // spread (zero projections: the spread's work depends on where the points
 // fall, not on their values), installs the fastest in c.nu3_tuning for g's
 // fine-grid shape and returns its index (best_ms: one back-projection).
@@ -1354,7 +1334,7 @@ int nufft3d_autotune(Ctx &c, Geom3D &g, double *best_ms) {
     int best = 0;
     float tbest = 1e30f;
     try {
-        for (int i = 0; i < N_SHAPES3; ++i) {
+        for (int i : {0, 2}) {
             c.nu3_tuning[key] = i;
             backproj3d_dev(c, g, proj.as<float>(), vol.as<float>(), nullptr);   // warm-up
             LC_HIP(hipEventRecord(e0, c.stream()));

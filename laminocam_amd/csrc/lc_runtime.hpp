@@ -215,14 +215,14 @@ class Ctx {
   public:
     // per image size N: kernel shapes chosen by the autotuner (or installed)
     std::map<int, ToepVariant> toep_tuning;
-    // per 3-D fine-grid shape (nf0, nf1, nf2): the type-1 spread's bin shape
-    // (an index into the compiled shapes; 0 when none was chosen)
+    // per 3-D fine-grid shape (nf0, nf1, nf2): the choice of the type-1 spread
+    // (0 when none was made)
     std::map<std::array<int, 3>, int> nu3_tuning;
     int nu3_shape(const int nf[3]) const {
         auto it = nu3_tuning.find({nf[0], nf[1], nf[2]});
         return it == nu3_tuning.end() ? 0 : it->second;
     }
-    // per 2-D fine-grid size nf: the type-1 spread's bin shape
+    // the same per 2-D fine-grid size nf
     std::map<int, int> nu2_tuning;
     int nu2_shape(int nf) const {
         auto it = nu2_tuning.find(nf);

@@ -394,9 +394,10 @@ def test_projectors3d_lattice_points_match_oracle(lc, orc64, dims, nproj, nrows,
 
 
 def test_backproj3d_bin_shapes_and_autotune(lc, orc64):
-    # every compiled bin shape of the spread (0: 4x4x8, 1: 8x4x4, 2: 8x8x8
-    # corner cells) gives the oracle's back-projection, deterministically;
-    # the autotuner installs one of them for the grid's fine-grid shape
+    # every choice of the spread (bins of more than 2048 points shared out among
+    # teams of waves, or of more than 512 with choice 2) gives the oracle's
+    # back-projection, deterministically; the autotuner installs one of them for
+    # the grid's fine-grid shape
     dims, nproj, nrows, ncols = (16, 96, 96), 90, 32, 96
     announce(f"backproj3d bin shapes dims={dims}")
     rng = np.random.default_rng(77)

@@ -202,9 +202,9 @@ def test_projectors_lattice_points_match_oracle(lc, orc64, N):
 
 
 def test_backproj2d_bin_shapes_and_autotune(lc, orc64):
-    # both compiled bin sizes of the sorted-bin spread (16 and 32 corner
-    # cells) give the oracle's back-projection; a slice is the same alone and
-    # in a stack for each; the autotuner installs one of them
+    # both accepted choices of the spread (they name the same tiles) give the
+    # oracle's back-projection; a slice is the same alone and in a stack; the
+    # autotuner installs one of them
     N, nang, ns = 128, 180, 3
     announce(f"backproj2d bin shapes N={N}")
     rng = np.random.default_rng(19)
