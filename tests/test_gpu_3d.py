@@ -324,7 +324,8 @@ def test_projectors3d_bin_edges_match_oracle(lc, orc64, dims, nproj, nrows, ncol
     vol, proj = rng.random(dims), rng.standard_normal((nproj, nrows, ncols))
     yr = orc64.forward3d(vol, th, ga, be, nrows, ncols, tol=1e-12)
     xr = orc64.backproj3d(proj, th, ga, be, dims, tol=1e-12)
-    assert rel_l2(lc.forward(vol, g), yr) < PROJ_TOL
+    # the projectors' FP32 error: at most 9e-7 at these sizes
+    assert rel_l2(lc.forward(vol, g), yr) < 3e-6
     ctx = lc.Context(0)
     try:
         psf = lc.PointSpreadFunction(g, dims, ctx=ctx, lazy=True)
@@ -333,7 +334,7 @@ def test_projectors3d_bin_edges_match_oracle(lc, orc64, dims, nproj, nrows, ncol
             x = lc.backproj(proj, g, dims, ctx=ctx)
             err = rel_l2(x, xr)
             print(f"shape {shape}: rel_l2 = {err:.3e}")
-            assert err < PROJ_TOL
+            assert err < 3e-6
             assert np.array_equal(lc.backproj(proj, g, dims, ctx=ctx), x)
     finally:
         ctx.close()

@@ -79,7 +79,24 @@ def test_split_bregman_sizes_match_oracle(lc, orc64, ns, N, outer, inner, zero_p
             assert rel_l2(x, xr) < 1e-9
         x32, _ = lc.split_bregman(psf, rhs.astype(np.float32), start.astype(np.float32), 0.3, 8.0, outer, inner,
                                   0.0, 0.0, zero_pad=zero_pad)
-        assert rel_l2(x32, xr) < 1e-3
+        # (the FP32 rounding of these steps: at most 1.5e-6)
+        assert rel_l2(x32, xr) < 5e-6
+
+
+# Every second outer iteration carries the residual over instead of forming it
+# anew.  Over 200 of them the FP32 solve ends 3.8e-6 from the FP64 oracle, as it
+# does with every residual formed anew, and 7.6e-6 if none ever is.
+def test_split_bregman_long_solve_keeps_its_residual(lc, orc64):
+    announce("sb long solve")
+    th, P, rhs = _problem(orc64, 32, 45, 5, 21)
+    xr, rr = orc64.split_bregman(P, rhs, np.zeros_like(rhs), 0.1, 10.0, 200, 1, 0.0, 0.0)
+    psf = lc.PointSpreadFunction2D(lc.PolarGrid2D(th, 32), 32)
+    for graph in (False, True):
+        x, rep = lc.split_bregman(psf, rhs, np.zeros_like(rhs), 0.1, 10.0, 200, 1, 0.0, 0.0, graph=graph)
+        assert rep["outer"] == rr["outer"] == 200
+        err = rel_l2(x, xr)
+        print(f"graph={graph} rel_l2={err:.3e}", flush=True)
+        assert err < 5.5e-6
 
 
 def test_mbir2d_sanity_split_bregman_gpu(lc, orc64):
