@@ -28,7 +28,7 @@ struct Nufft2D {
     DBuf points, tiles;
     int ntiles = 0, nheavy = 0;
     DBuf chirp;           // det_blue: double2 chirp[nrad], then its spectrum [plan_det.L]
-    bool ready = false;
+    bool ready = false, ordered = false;
 };
 
 // ---------------------------------------------------------------------------
@@ -57,8 +57,10 @@ void bluestein_tables(int n, int L, std::vector<std::complex<double>> &chirp,
 
 // NUFFT projectors on device buffers (src/projection.cpp:146-182):
 // forward2d: vol (ns x N x N) -> sino (ns x nang x nrad); backproj2d: reverse
+void nufft2d_init(Ctx &c, Geom2D &g);
+// the points' order, for type 1 (backproj2d and the NUFFT sysmat2d), after nufft2d_init;
 // own_work: on working space of its own, freed on return, in place of c's scratch
-void nufft2d_init(Ctx &c, Geom2D &g, bool own_work = false);
+void nufft2d_order(Ctx &c, Geom2D &g, bool own_work = false);
 void forward2d_dev(Ctx &c, Geom2D &g, const float *vol, float *sino, int ns);
 void backproj2d_dev(Ctx &c, Geom2D &g, const float *sino, float *vol, int ns);
 // sysmat2d(x, grid) = Re(T1(T2 x)) / nrad (src/gradient.cpp:59-69)

@@ -187,7 +187,7 @@ __global__ void k_det_dft(const float *__restrict__ real_in, const float2 *__res
 // Type-1 spreading by output tiles.  A point's corner is its first footprint
 // cell, ceil(g - 4) per axis, taken modulo nf.  The geometry holds the points
 // sorted by 8 x 8 bins of corners (row major; the points do not depend on the
-// data, so nufft2d_init sorts them once), so a tile of 16 x 16 cells of
+// data, so nufft2d_order sorts them once), so a tile of 16 x 16 cells of
 // the fine grid finds the points that reach it (corners from 7 cells before it
 // to its end) in one or two runs per row of bins.  It takes them in that order
 // and writes its cells once: no clearing, no adding into the grid, no order
@@ -834,12 +834,13 @@ Grid2 grid2(const Geom2D &g) {
 }
 
 int tiles_of(int nf) { return ceil_div(nf, TE) * ceil_div(nf, TE); }
+} // namespace
 
 // the points sorted by corner bin, the bins' starts, and the tiles, fullest
-// first.  The sort's working space, about 20 bytes per point, is
+// first: what type 1 needs beside nufft2d_init's tables.  The sort's working space, about 20 bytes per point, is
 // the projections' scratch, which the caller's own call is about to use, or
 // (own_work) freed again: a server's main context never projects
-void sort_points(Ctx &c, Geom2D &g, bool own_work) {
+void nufft2d_order(Ctx &c, Geom2D &g, bool own_work) {
     Nufft2D &u = g.nu;
     const Grid2 s = grid2(g);
     LC_REQUIRE(g.nang * g.nrad < (int64_t)1 << 31, "2-D projector: 2^31 or more points per slice");
@@ -879,8 +880,8 @@ void sort_points(Ctx &c, Geom2D &g, bool own_work) {
     LC_HIP(rocprim::radix_sort_pairs(tmp, tt, ka, kb, (int *)va, u.tiles.as<int>(), (size_t)tiles, 0, 31, c.stream()));
     LC_HIP(hipMemcpyAsync(&u.nheavy, heavy, sizeof(int), hipMemcpyDeviceToHost, c.stream()));
     c.sync();
+    u.ordered = true;
 }
-} // namespace
 
 // device bytes of the points' order and the tiles that a geometry keeps
 size_t nufft2d_order_bytes(int64_t nang, int64_t nrad, int nf) {
@@ -888,7 +889,7 @@ size_t nufft2d_order_bytes(int64_t nang, int64_t nrad, int nf) {
     return al256(sizeof(unsigned) * (size_t)(nang * nrad)) + sizeof(int) * (nb * nb + 1 + (size_t)tiles_of(nf));
 }
 
-void nufft2d_init(Ctx &c, Geom2D &g, bool own_work) {
+void nufft2d_init(Ctx &c, Geom2D &g) {
     Nufft2D &u = g.nu;
     u.cs.alloc(sizeof(double2) * g.nang);
     hipLaunchKernelGGL(k_angle_table, dim3(ceil_div(g.nang, 256)), dim3(256), 0, c.stream(),
@@ -912,7 +913,6 @@ void nufft2d_init(Ctx &c, Geom2D &g, bool own_work) {
     // 53 105 / 118, 67 126 / 124, 127 212 / 198, 511 1084 / 677)
     u.det_blue = !u.det_fast && g.nrad > 64 && 2 * g.nrad - 1 <= DET_FFT_MAX;
     if (u.det_blue) det_blue_init(c, u, (int)g.nrad);
-    sort_points(c, g, own_work);
     u.ready = true;
 }
 
@@ -1093,16 +1093,17 @@ void type2(Ctx &c, const Geom2D &g, const NuWork &w, const float *vol, int ns) {
     LC_HIP(hipGetLastError());
 }
 
-void nu_check(Ctx &c, Geom2D &g, int ns) {
+void nu_check(Ctx &c, Geom2D &g, int ns, bool type1) {
     if (!g.nu.ready) nufft2d_init(c, g);
     LC_REQUIRE(g.nu.nf <= NU_NT * NU_ME, "nufft: fine grid too large (image size above 2048)");
     LC_REQUIRE(ns >= 1 && ns <= 65535, "nufft: 1 to 65535 slices per call");
+    if (type1 && !g.nu.ordered) nufft2d_order(c, g);
 }
 } // namespace
 
 // backproj2d: sino (ns x nang x nrad real, device) -> vol (ns x N x N real, device)
 void backproj2d_dev(Ctx &c, Geom2D &g, const float *sino, float *vol, int ns) {
-    nu_check(c, g, ns);
+    nu_check(c, g, ns, true);
     const NuWork w = nu_work(c, g, ns);
     det_transform(c, g, -1, sino, nullptr, w.C, nullptr, ns);
     type1(c, g, w, vol, ns);
@@ -1110,7 +1111,7 @@ void backproj2d_dev(Ctx &c, Geom2D &g, const float *sino, float *vol, int ns) {
 
 // forward2d: vol (ns x N x N real, device) -> sino (ns x nang x nrad real, device)
 void forward2d_dev(Ctx &c, Geom2D &g, const float *vol, float *sino, int ns) {
-    nu_check(c, g, ns);
+    nu_check(c, g, ns, false);
     const NuWork w = nu_work(c, g, ns);
     type2(c, g, w, vol, ns);
     det_transform(c, g, 1, nullptr, w.C, nullptr, sino, ns);
@@ -1118,7 +1119,7 @@ void forward2d_dev(Ctx &c, Geom2D &g, const float *vol, float *sino, int ns) {
 
 // sysmat2d(x, grid) = Re(T1(T2 x)) / nrad (src/gradient.cpp:59-69)
 void sysmat2d_nufft_dev(Ctx &c, Geom2D &g, const float *x, float *y, int ns) {
-    nu_check(c, g, ns);
+    nu_check(c, g, ns, true);
     const NuWork w = nu_work(c, g, ns);
     type2(c, g, w, x, ns);
     type1(c, g, w, y, ns);
@@ -1127,7 +1128,7 @@ void sysmat2d_nufft_dev(Ctx &c, Geom2D &g, const float *x, float *y, int ns) {
 // Times the back-projection of nslices zero sinograms on g's grid (best_ms) and
 // installs choice 0: both numbers name the one compiled spread.
 int nufft2d_autotune(Ctx &c, Geom2D &g, int nslices, double *best_ms) {
-    nu_check(c, g, nslices);
+    nu_check(c, g, nslices, true);
     const int64_t npts = g.nang * g.nrad;
     DBuf sino(sizeof(float) * (size_t)(nslices * npts)), vol(sizeof(float) * (size_t)nslices * g.N * g.N);
     LC_HIP(hipMemsetAsync(sino.as(), 0, sizeof(float) * (size_t)(nslices * npts), c.stream()));

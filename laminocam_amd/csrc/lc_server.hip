@@ -124,7 +124,7 @@ uint64_t Server::submit(std::unique_ptr<ServerRequest> r) {
     {
         std::lock_guard<std::mutex> lk(main_.mu);
         const bool build = r->g3 ? !r->g3->psf_ready || (r->has_sino && !r->g3->nu.ready)
-                                 : !r->g2->psf_ready || (r->has_sino && !r->g2->nu.ready);
+                                 : !r->g2->psf_ready || (r->has_sino && !r->g2->nu.ordered);
         if (build) {   // (a request on a ready geometry launches nothing here)
             // no lane captures while this thread allocates and synchronises
             std::lock_guard<std::recursive_mutex> cl(capture_mutex());
@@ -134,7 +134,8 @@ uint64_t Server::submit(std::unique_ptr<ServerRequest> r) {
                 if (r->has_sino && !r->g3->nu.ready) nufft3d_init(main_, *r->g3);
             } else {
                 if (!r->g2->psf_ready) geom2d_build_psf(main_, *r->g2);
-                if (r->has_sino && !r->g2->nu.ready) nufft2d_init(main_, *r->g2, true);
+                if (r->has_sino && !r->g2->nu.ready) nufft2d_init(main_, *r->g2);
+                if (r->has_sino && !r->g2->nu.ordered) nufft2d_order(main_, *r->g2, true);
             }
             main_.sync();
         }

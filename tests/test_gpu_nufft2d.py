@@ -1,6 +1,7 @@
 """GPU parity of the 2-D NUFFT projectors forward2d / backproj2d
 (src/projection.cpp:146-182) against the FP64 oracle and the committed golden
 vectors, through the C ABI.  Bar: 1e-4 relative L2 on projections."""
+import ctypes as C
 import os
 
 import numpy as np
@@ -231,5 +232,32 @@ def test_backproj2d_bin_shapes_and_autotune(lc, orc64):
         print(f"autotune2d_nufft: shape {best}, {ms:.3f} ms")
         assert best in (0, 1) and ms > 0.0
         assert ctx.get_tuning2d_nufft(psf) == best
+    finally:
+        ctx.close()
+
+
+def test_forward2d_alone_sorts_no_points(lc):
+    # the points' order is for the spread: a forward projection on a new geometry
+    # neither makes it nor takes the sort's working space (28 bytes per point)
+    announce("forward2d alone")
+    hip = C.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    N, nang, nrad = 32, 2048, 4096
+    npts = nang * nrad
+    x = np.random.default_rng(2).random((1, N, N)).astype(np.float32)
+    ctx = lc.Context(0)
+    try:
+        lc.forward2d(x, lc.PolarGrid2D(uniform_theta(60), N), ctx=ctx)
+        free0 = free_bytes()
+        lc.forward2d(x, lc.PolarGrid2D(uniform_theta(nang), nrad), ctx=ctx)
+        held = free0 - free_bytes()
+        print(f"held {held / 2**20:.1f} MiB")
+        # the staged sinogram (4 bytes per point) and the detector spectrum (8)
+        assert held <= 12 * npts + (24 << 20)
     finally:
         ctx.close()
