@@ -70,11 +70,11 @@ struct Grid3 {
     int mask;           // 1: drop points with any |coordinate| > pi
 };
 
-// The operations of a point's position are written out, with every fused
-// multiply-add explicit: positions that are whole numbers up to rounding are
-// common (an untilted scan with ncols = n has no others along x), and kernels
-// that let the compiler contract these products each in its own way took
-// different corners for them, on the two sides of the periodic edge at worst.
+// A point's position is rounded alike in every kernel: its fused multiply-adds are
+// explicit.  Positions that are whole numbers up to rounding are common (an
+// untilted scan with ncols = n has no others along x), and kernels that let the
+// compiler fuse these products each in its own way took different corners for
+// them, on the two sides of the periodic edge at worst.
 __device__ __forceinline__ double lattice_coord(int k, double step) {   // (k + 1/2) step - pi
     return __builtin_fma((double)k + 0.5, step, -M_PI);
 }
@@ -87,7 +87,13 @@ __device__ __forceinline__ void point3(const double *rot, int p, int j, int k, c
     z = __builtin_fma(qy, r[5], qx * r[2]);
 }
 
-__device__ __forceinline__ bool inside_pi(double x, double y, double z) {
+// the reference's mask (include/polar_grid.h:80-86): some coordinates equal pi up
+// to rounding, so by its own operations, of which none is fused
+__device__ __forceinline__ bool inside_pi(const double *rot, int p, int j, int k, const Grid3 &g) {
+#pragma clang fp contract(off)
+    const double *r = rot + 6 * (int64_t)p;
+    const double qx = ((double)k + 0.5) * g.dX - M_PI, qy = ((double)j + 0.5) * g.dY - M_PI;
+    const double x = qx * r[0] + qy * r[3], y = qx * r[1] + qy * r[4], z = qx * r[2] + qy * r[5];
     return fabs(x) <= M_PI && fabs(y) <= M_PI && fabs(z) <= M_PI;
 }
 
@@ -148,7 +154,7 @@ __device__ __forceinline__ Corner3 corner3(const double *rot, int p, int j, int 
     Corner3 c;
     double x, y, z;
     point3(rot, p, j, k, g, x, y, z);
-    c.ok = !g.mask || inside_pi(x, y, z);
+    c.ok = !g.mask || inside_pi(rot, p, j, k, g);
     const double hw = 0.5 * W3;
     c.gz = __builtin_fma(z, g.nf[0] / (2.0 * M_PI), 0.5 * g.nf[0]);
     c.gy = __builtin_fma(y, g.nf[1] / (2.0 * M_PI), 0.5 * g.nf[1]);
@@ -302,6 +308,9 @@ __device__ __forceinline__ void axis_weights(int t, T f, int h, float beta, F &&
 }
 // smallest and largest corner row of the groups of G consecutive lanes
 template <int G> __device__ __forceinline__ void group_rows(int ty, bool ok, int &lo, int &hi) {
+    // (a corner's row lies in its bin: the bounds change no value, but the spread of
+    // 8 x 256^2 from 180 x 64 rows takes 1400 us with them and 1413 without)
+    ty = min(max(ty, 0), 63);
     lo = ok ? ty : 127;
     hi = ok ? ty : 0;
 #pragma unroll
@@ -1170,14 +1179,18 @@ Bins3 sort_points(Ctx &c, const Geom3D &g, const Work3 &w, const Grid3 &gg, floa
     return bn;
 }
 
-// Whether the forward projector interpolates npts points unsorted.  Sorting them
-// takes about 100 us whatever their number, and few points in many bins read a
-// bin's region for each, so the line rises with the bins.  Forward projection
-// (us, unsorted / sorted): 8 x 64^2 0.4 M points 239 / 269, 0.8 M 376 / 349; 16 x
-// 256^2 0.3 M 319 / 354, 0.6 M 509 / 434; 32 x 511^2 0.5 M 1090 / 1165, 0.8 M 1396 /
-// 1294; 29 x 721^2 0.6 M 2241 / 2365, 1.0 M 2675 / 2650.
+// Whether the forward projector interpolates npts points unsorted: what that
+// takes, by the plane of the fine grid that a point's neighbours in a row walk
+// over, against the sort's launches and a region read for every bin, both fitted
+// to 14 volumes from 8 x 64^2 to 29 x 721^2 of 3e4 to 2e6 points (the measured
+// crossings lie within a tenth of the time).  Forward projection (us, unsorted /
+// sorted): 8 x 64^2 0.5 M points 266 / 285, 0.8 M 376 / 349; 16 x 256^2 0.3 M 319 /
+// 354, 0.5 M 448 / 422; 5 x 200^2 0.2 M 252 / 301, 0.4 M 405 / 361; 32 x 511^2 0.5 M
+// 1090 / 1165, 0.8 M 1396 / 1294; 29 x 721^2 0.6 M 2241 / 2365, 1.5 M 3168 / 2808.
 bool interp_direct(int64_t npts, const int nf[3]) {
-    return npts <= 450000 + 2 * (int64_t)count_of(bins_of(nf));
+    const double plane = (double)nf[1] * nf[2];
+    const double ns = std::min(0.8, std::max(0.26, 0.42 + 0.13 * std::log2(plane / 65536.0)));   // per point
+    return (double)npts * ns * 1e-3 < 175.0 + 0.003 * count_of(bins_of(nf));                     // us
 }
 
 // vol -> w.C, nsort projections at a time; sort: leaves the last ones' points
