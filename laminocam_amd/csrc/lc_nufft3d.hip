@@ -14,7 +14,8 @@
 // shift; the (-1)^m phase and 1/psi_hat sit in per-axis correction factors.
 //   type 1: deterministic sorted-bin spreading -> fine grid, then one pruned
 //           FFT pass per axis (x, y, z), deconvolution in each pass;
-//   type 2: the reverse passes, then 8x8x8 interpolation of the sorted points.
+//   type 2: the reverse passes, then 8x8x8 interpolation of the points, sorted
+//           where there are enough of them.
 // Detector transforms are line FFTs along x then y with the reference's shift
 // index maps; widths that are not 2^p 3^q use Bluestein's algorithm with an
 // FP64-built chirp and chirp spectrum.
